@@ -72,15 +72,6 @@ k_sdot_part(const double2 *__restrict__ x, const double2 *__restrict__ y, int n,
     if (threadIdx.x == 0) part[(long)a * gridDim.x + blockIdx.x] = s;
 }
 
-__global__ void k_rows(const double *__restrict__ part, int n, int nchunk, double scale, double *__restrict__ out)
-{
-    const int a = blockIdx.x * blockDim.x + threadIdx.x;
-    if (a >= n) return;
-    double s = 0.0;
-    for (int k = 0; k < nchunk; k++) s += part[(long)a * nchunk + k];
-    out[a] = s * scale;
-}
-
 // ---------------------------------------------------------------------------
 // out = acc + (hterm - em_a mu) - 2 s_a (g1 + e_a g2)  (elementwise), and the potential
 // gradient of H: with nu = mu - s_a psi,
@@ -539,7 +530,7 @@ static int sdot(tdw_ctx *c, int n, const double2 *x, const double2 *y, double sc
     const long chunk = dot_chunk(c, &nchunk);
     TDW_TRY(ensure_part(c, (size_t)n * nchunk));
     hipLaunchKernelGGL(k_sdot_part, dim3(nchunk, n), dim3(AT), 0, c->stream, x, y, n, (long)c->N, chunk, c->d_part);
-    hipLaunchKernelGGL(k_rows, dim3((n + 255) / 256), dim3(256), 0, c->stream, c->d_part, n, nchunk, scale, out);
+    TDW_TRY(row_sums(c, c->d_part, n, nchunk, scale, out));
     return (int)hipGetLastError();
 }
 
@@ -595,8 +586,7 @@ static int dens_t(tdw_ctx *c, int n, const double2 *psi, double2 *out, const dou
     else
         hipLaunchKernelGGL(k_dens_t<3>, g, dim3(AT), 0, c->stream, psi, out, lD, c->d_fbeta, c->d_kt, c->d_cnt, n, N,
                            chunk, tr, cubic, piz, c->d_part);
-    hipLaunchKernelGGL(k_rows, dim3((n + 255) / 256), dim3(256), 0, c->stream, c->d_part, n, nchunk, dvol_norm(c),
-                       tvec);
+    TDW_TRY(row_sums(c, c->d_part, n, nchunk, dvol_norm(c), tvec));
     return (int)hipGetLastError();
 }
 
@@ -843,7 +833,7 @@ extern "C" int tdw_adj_backward_step(tdw_ctx *c, tdw_adj_state *A, int it, const
         auto kr = h == 3 ? k_recon<3> : h == 4 ? k_recon<4> : k_recon<5>;
         hipLaunchKernelGGL(kr, dim3(nchunk, n), dim3(AT), 0, c->stream, LY, CD2(y1), CD2(y0), F[0], F[1], F[2], F[3],
                            F[4], W0, W3, W4, t1, t->scal, cf, c->p.dt, n, N, chunk, c->d_part);
-        hipLaunchKernelGGL(k_rows, dim3((n + 255) / 256), dim3(256), 0, c->stream, c->d_part, n, nchunk, dv, svp);
+        TDW_TRY(row_sums(c, c->d_part, n, nchunk, dv, svp));
         TDW_HIP(hipGetLastError());
     }
     // F_p = H(U_p) yh_p - e_p yh_p

@@ -497,43 +497,6 @@ dg_yz(const ac_t<SP> *__restrict__ y, const double *__restrict__ fbeta, const do
     }
 }
 
-// dens (the 12*N block) from the chunk partials of dg_x and dg_yz: one
-// thread per (output field, point), each summing its field over the chunks
-// in chunk order
-__global__ void __launch_bounds__(AT)
-dg_final(const double *__restrict__ px, const double *__restrict__ pyz, int nchunk, long N, double tr,
-         double *__restrict__ dens)
-{
-    const long t = (long)blockIdx.x * AT + threadIdx.x;
-    if (t >= 12 * N) return;
-    const int f = (int)(t / N);
-    const long i = t - (long)f * N;
-    // source field in the x partials (8 per chunk) and the yz partials (6 per chunk), -1: none
-    // output f: 0 Re nu, 1 Im nu, 2 rho_a, 3 tau_a, 4 j_a,x, 5 j_a,y, 6 j_a,z, 7 rho_b, 8 tau_b, 9 j_b,x,
-    //           10 j_b,y, 11 j_b,z
-    constexpr int sx[12] = {2, 3, 0, 4, 6, -1, -1, 1, 5, 7, -1, -1};
-    constexpr int sy[12] = {-1, -1, -1, 0, -1, 2, 3, -1, 1, -1, 4, 5};
-    const int fx = sx[f], fy = sy[f];
-    double a = 0.0, b = 0.0;
-    if (fx >= 0)
-        for (int k = 0; k < nchunk; k++) a += px[((long)k * 8 + fx) * N + i];
-    if (fy >= 0)
-        for (int k = 0; k < nchunk; k++) b += pyz[((long)k * 6 + fy) * N + i];
-    const double v = (a + b) / 10000. / tr;
-    if (f < 2) dens[2 * i + f] = v;
-    else dens[(long)f * N + i] = v;
-}
-
-// qpe[a] = dv * sum of the state's NX plane partials
-__global__ void ah_qpe(const double *__restrict__ part, int n, int NX, double dv, double *__restrict__ qpe)
-{
-    const int a = blockIdx.x * blockDim.x + threadIdx.x;
-    if (a >= n) return;
-    double s = 0.0;
-    for (int k = 0; k < NX; k++) s += part[(long)a * NX + k];
-    qpe[a] = dv * s;
-}
-
 template <bool SP> struct AFns {
     typedef ac_t<SP> C;
     typedef void (*ahx_fn)(const C *, C *, const double *, int, long, int, const C *, double, double, const double *);
@@ -658,10 +621,10 @@ static int dens_grad_t(tdw_ctx *c, int n, const ac_t<SP> *wf, const double *fbet
     const double k1z = 2.0 * M_PI / c->Lphys[2] / c->nz, k2z = pow(2.0 * M_PI / c->Lphys[2], 2) / c->nz;
     hipLaunchKernelGGL(fy, dim3((unsigned)((long)nchunk * c->nx)), dim3(nt), lds, c->stream, wf, fbeta, wgt, n, N,
                        c->nx, G, F::tw(c, 1), F::tw(c, 2), k1y, k2y, k1z, k2z, pyz_part);
-    hipLaunchKernelGGL(dg_final, dim3((unsigned)((12 * N + AT - 1) / AT)), dim3(AT), 0, c->stream, px_part, pyz_part,
-                       nchunk, N, dens_transverse(c), dens);
     TDW_TRY((int)hipGetLastError());
-    return spin_fold(c, dens);
+    const ChunkSrc fx_src{px_part, 8, {2, 3, 0, 4, 6, -1, -1, 1, 5, 7, -1, -1}};
+    const ChunkSrc fy_src{pyz_part, 6, {-1, -1, -1, 0, -1, 2, 3, -1, 1, -1, 4, 5}};
+    return chunk_final(c, fx_src, fy_src, nchunk, dens);
 }
 
 int dens_grad_fused(tdw_ctx *c, int n, const double2 *wf, const double *fbeta, const double *wgt, double *dens)
@@ -707,7 +670,7 @@ static int aslda_h_t(tdw_ctx *c, int n, const ac_t<SP> *in, ac_t<SP> *out, ac_t<
         const double k1z = 2.0 * M_PI / c->Lphys[2] / c->nz, k2z = pow(2.0 * M_PI / c->Lphys[2], 2) / c->nz;
         hipLaunchKernelGGL(fy, dim3((unsigned)((long)n * c->nx)), dim3(nt), lds, c->stream, in, T, out, pots, hx, n, N,
                            c->nx, F::tw(c, 1), F::tw(c, 2), k1y, k2y, k1z, k2z, c->p.mu_a, c->p.mu_b, part, sc);
-        hipLaunchKernelGGL(ah_qpe, dim3((n + 255) / 256), dim3(256), 0, c->stream, part, n, c->nx, dvol_norm(c), d_qpe);
+        TDW_TRY(row_sums(c, part, n, c->nx, dvol_norm(c), d_qpe));
     }
     return (int)hipGetLastError();
 }

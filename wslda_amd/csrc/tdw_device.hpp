@@ -85,6 +85,15 @@ __device__ __forceinline__ double wave_sum(double v)
     return v;
 }
 
+// Sum of a row of m doubles by one wavefront (lanes take consecutive values);
+// every lane gets the result.
+__device__ __forceinline__ double wave_row_sum(const double *__restrict__ row, int m)
+{
+    double s = 0.0;
+    for (int k = threadIdx.x & 63; k < m; k += 64) s += row[k];
+    return wave_sum(s);
+}
+
 // Block-wide sum; every thread gets the result.  red must hold
 // blockDim.x/64 doubles.  Deterministic for a fixed launch shape.
 __device__ __forceinline__ double block_sum(double v, double *red)

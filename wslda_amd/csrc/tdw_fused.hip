@@ -251,17 +251,21 @@ f_corr(double2 *__restrict__ y, const hc_t<SP> *hin, const hc_t<SP> *__restrict_
     put_norm_part(xk, wave != 0, P, Ptot, xpart);
 }
 
+// Per-state sums take a wave per state: with a thread per state the loads of
+// a wave lay a row apart and each thread chained its whole row (at 12^3, 144
+// pencil partials per component: 45-49 us per launch, 5.1-5.8 us with a wave).
+static constexpr int SPB = FT / 64;   // states per workgroup
+
 // s = 1/sqrt(norm * dV), s2 = s^2 per state (and norm * dV itself into nrm
 // when given); part holds `per` entries per component
-__global__ void f_norm_final(const double *__restrict__ part, int n, int per, double dv, double *__restrict__ s,
-                             double *__restrict__ s2, double *__restrict__ nrm_out)
+__global__ void __launch_bounds__(FT)
+f_norm_final(const double *__restrict__ part, int n, int per, double dv, double *__restrict__ s,
+             double *__restrict__ s2, double *__restrict__ nrm_out)
 {
-    const int a = blockIdx.x * blockDim.x + threadIdx.x;
+    const int a = blockIdx.x * SPB + (threadIdx.x >> 6);
     if (a >= n) return;
-    double su = 0.0, sv = 0.0;
-    const double *pu = part + (long)a * per, *pv = part + ((long)n + a) * per;
-    for (int k = 0; k < per; k++) su += pu[k];
-    for (int k = 0; k < per; k++) sv += pv[k];
+    const double su = wave_row_sum(part + (long)a * per, per), sv = wave_row_sum(part + ((long)n + a) * per, per);
+    if (threadIdx.x & 63) return;
     const double nrm = (su + sv) * dv;
     const double sc = 1.0 / sqrt(nrm);
     s[a] = sc;
@@ -644,21 +648,16 @@ f_sub(const double2 *__restrict__ in, double2 *__restrict__ out, const double *_
 // <H> per state from the yz pass's partials (per per state); with xpart,
 // plus the x part of the kinetic term from the predictor (xper entries per
 // component, unscaled: times s2 = s^2 of the state)
-__global__ void f_e_final(const double *__restrict__ part, int n, int per, double dv, double *__restrict__ e,
-                          double *__restrict__ e2, const double *__restrict__ xpart, int xper,
-                          const double *__restrict__ s2)
+__global__ void __launch_bounds__(FT)
+f_e_final(const double *__restrict__ part, int n, int per, double dv, double *__restrict__ e,
+          double *__restrict__ e2, const double *__restrict__ xpart, int xper, const double *__restrict__ s2)
 {
-    const int a = blockIdx.x * blockDim.x + threadIdx.x;
+    const int a = blockIdx.x * SPB + (threadIdx.x >> 6);
     if (a >= n) return;
-    double s = 0.0;
-    for (int k = 0; k < per; k++) s += part[(long)a * per + k];
-    if (xpart) {
-        double x = 0.0;
-        const double *pu = xpart + (long)a * xper, *pv = xpart + ((long)n + a) * xper;
-        for (int k = 0; k < xper; k++) x += pu[k];
-        for (int k = 0; k < xper; k++) x += pv[k];
-        s += x * s2[a];
-    }
+    double s = wave_row_sum(part + (long)a * per, per);
+    if (xpart)
+        s += (wave_row_sum(xpart + (long)a * xper, xper) + wave_row_sum(xpart + ((long)n + a) * xper, xper)) * s2[a];
+    if (threadIdx.x & 63) return;
     e[a] = s * dv;
     if (e2) e2[a] = s * dv;
 }
@@ -899,7 +898,7 @@ static int xpass_norm(tdw_ctx *c, int n, double *s_out, double *s2_out, int wave
 {
     const int per = wave ? c->S / 64 : c->S;
     TDW_TIMED(c, "f_norm");
-    hipLaunchKernelGGL(f_norm_final, dim3((n + 255) / 256), dim3(256), 0, c->stream, c->d_fpart, n, per,
+    hipLaunchKernelGGL(f_norm_final, dim3((n + SPB - 1) / SPB), dim3(FT), 0, c->stream, c->d_fpart, n, per,
                        dvol_norm(c), s_out, s2_out, nrm_out);
     return (int)hipGetLastError();
 }
@@ -930,7 +929,7 @@ static int hyz(tdw_ctx *c, int n, const hc_t<SP> *y, const hc_t<SP> *T, hc_t<SP>
         TDW_HIP(hipGetLastError());
     }
     TDW_TIMED(c, "f_e");
-    hipLaunchKernelGGL(f_e_final, dim3((n + 255) / 256), dim3(256), 0, c->stream, c->d_fpart, n, c->nx,
+    hipLaunchKernelGGL(f_e_final, dim3((n + SPB - 1) / SPB), dim3(FT), 0, c->stream, c->d_fpart, n, c->nx,
                        dvol_norm(c), e_out, e_out2, xpart, xper, s2);
     return (int)hipGetLastError();
 }

@@ -128,14 +128,34 @@ k_norm_part(const double2 *__restrict__ wf, int n, long N, long chunk, double *_
     if (threadIdx.x == 0) part[(long)a * gridDim.x + blockIdx.x] = s;
 }
 
-__global__ void k_rowsum(const double *__restrict__ part, int n, int nchunk, double scale,
-                         double *__restrict__ out)
+// row sums, W = 64 lanes or one thread per row (see row_sums)
+template <int W>
+__global__ void __launch_bounds__(NT)
+k_rowsum(const double *__restrict__ part, int n, int nchunk, double scale, double *__restrict__ out)
 {
-    int a = blockIdx.x * blockDim.x + threadIdx.x;
+    const int a = blockIdx.x * (NT / W) + threadIdx.x / W;
     if (a >= n) return;
+    const double *row = part + (long)a * nchunk;
     double s = 0.0;
-    for (int k = 0; k < nchunk; k++) s += part[(long)a * nchunk + k];
-    out[a] = s * scale;
+    if constexpr (W == 64) s = wave_row_sum(row, nchunk);
+    else
+        for (int k = 0; k < nchunk; k++) s += row[k];
+    if (threadIdx.x % W == 0) out[a] = s * scale;
+}
+
+// out[a] = scale * sum of the nchunk values of row a.  With a thread per row
+// the loads of a wave lie nchunk doubles apart and each thread chains nchunk
+// additions: fine up to four values (2.65 us for 128 rows of one value, 3.4
+// with a wave each);
+// longer rows take a wave each, consecutive loads and a shuffle tree.
+int row_sums(tdw_ctx *c, const double *part, int n, int nchunk, double scale, double *out)
+{
+    if (nchunk <= 4)
+        hipLaunchKernelGGL(k_rowsum<1>, dim3((n + NT - 1) / NT), dim3(NT), 0, c->stream, part, n, nchunk, scale, out);
+    else
+        hipLaunchKernelGGL(k_rowsum<64>, dim3((n + NT / 64 - 1) / (NT / 64)), dim3(NT), 0, c->stream, part, n, nchunk,
+                           scale, out);
+    return (int)hipGetLastError();
 }
 
 __global__ void __launch_bounds__(NT)
@@ -172,8 +192,7 @@ int norms_with(tdw_ctx *c, int n, const double2 *wf, double *d_nrm, double *part
     int nchunk;
     long chunk = pick_chunk(c, &nchunk);
     hipLaunchKernelGGL(k_norm_part, dim3(nchunk, n), dim3(NT), 0, c->stream, wf, n, (long)c->N, chunk, part);
-    hipLaunchKernelGGL(k_rowsum, dim3((n + 255) / 256), dim3(256), 0, c->stream, part, n, nchunk, dvol_norm(c),
-                       d_nrm);
+    TDW_TRY(row_sums(c, part, n, nchunk, dvol_norm(c), d_nrm));
     return (int)hipGetLastError();
 }
 
@@ -268,34 +287,48 @@ k_dens_part(const W *__restrict__ wf, const double2 *__restrict__ ddx, const dou
     }
 }
 
-template <bool GRAD>
-__global__ void __launch_bounds__(NT)
-k_dens_final(const double *__restrict__ part, int nchunk, long N, double tr, double *__restrict__ dens)
+// dens (the 12*N block) from the chunk partials.  Output f: 0 Re nu, 1 Im nu,
+// 2 rho_a, 3 tau_a, 4-6 j_a, 7 rho_b, 8 tau_b, 9-11 j_b; field f of a chunk
+// is field A.f[f] of the partials A plus field B.f[f] of B (-1: none).
+// A workgroup takes FP points of one field with FL lanes over the chunks, so
+// that the sum over the chunks (up to some hundreds on small lattices) is
+// spread over lanes instead of one chain per point: at 12^3 and 223 chunks a
+// thread per point took 76 us, this takes 7.7 us.  The order of the sum is
+// fixed by the launch shape.
+static constexpr int FP = 16, FL = 16;
+
+__global__ void __launch_bounds__(FP *FL)
+k_chunk_final(ChunkSrc A, ChunkSrc B, int nchunk, long N, double tr, double *__restrict__ dens)
 {
-    const long i = (long)blockIdx.x * NT + threadIdx.x;
-    if (i >= N) return;
-    const int NV = GRAD ? 12 : 4;
-    double s[12];
-#pragma unroll
-    for (int v = 0; v < 12; v++) s[v] = 0.0;
-    for (int k = 0; k < nchunk; k++) {
-        const double *p = part + (long)k * NV * N + i;
-#pragma unroll
-        for (int v = 0; v < NV; v++) s[v] += p[v * N];
+    __shared__ double red[FL][FP + 1];
+    const int f = blockIdx.y, p = threadIdx.x % FP, l = threadIdx.x / FP;
+    const long i = (long)blockIdx.x * FP + p;
+    const int fa = A.f[f], fb = B.f[f];
+    double s = 0.0;
+    if (i < N) {
+        if (fa >= 0)
+            for (int k = l; k < nchunk; k += FL) s += A.part[((long)k * A.nf + fa) * N + i];
+        if (fb >= 0)
+            for (int k = l; k < nchunk; k += FL) s += B.part[((long)k * B.nf + fb) * N + i];
     }
-    const double sc = 10000.;
-    dens[2 * i] = s[2] / sc / tr;          // nu (complex, first 2N doubles)
-    dens[2 * i + 1] = s[3] / sc / tr;
-    dens[2 * N + i] = s[0] / sc / tr;      // rho_a
-    dens[7 * N + i] = s[1] / sc / tr;      // rho_b
-    dens[3 * N + i] = GRAD ? s[4] / sc / tr : 0.0;
-    dens[8 * N + i] = GRAD ? s[5] / sc / tr : 0.0;
-    dens[4 * N + i] = GRAD ? s[6] / sc / tr : 0.0;
-    dens[5 * N + i] = GRAD ? s[7] / sc / tr : 0.0;
-    dens[6 * N + i] = GRAD ? s[8] / sc / tr : 0.0;
-    dens[9 * N + i] = GRAD ? s[9] / sc / tr : 0.0;
-    dens[10 * N + i] = GRAD ? s[10] / sc / tr : 0.0;
-    dens[11 * N + i] = GRAD ? s[11] / sc / tr : 0.0;
+    red[l][p] = s;
+    __syncthreads();
+    if (l || i >= N) return;
+    s = 0.0;
+#pragma unroll
+    for (int k = 0; k < FL; k++) s += red[k][p];
+    const double v = s / 10000. / tr;
+    if (f < 2) dens[2 * i + f] = v;
+    else dens[(long)f * N + i] = v;
+}
+
+int chunk_final(tdw_ctx *c, const ChunkSrc &A, const ChunkSrc &B, int nchunk, double *dens)
+{
+    const long N = (long)c->N;
+    hipLaunchKernelGGL(k_chunk_final, dim3((unsigned)((N + FP - 1) / FP), 12), dim3(FP * FL), 0, c->stream, A, B,
+                       nchunk, N, dens_transverse(c), dens);
+    TDW_TRY((int)hipGetLastError());
+    return spin_fold(c, dens);
 }
 
 // spin-symmetric mode (SPINSYMMETRY_MODE, pca_dens.cu:55-58, 71-90, 112-118):
@@ -362,11 +395,10 @@ static int densities_t(tdw_ctx *c, int n, const W *wf, const double2 *ddx, const
     else if (c->dim == 2) { if (grad) TDW_DP(2, true); else TDW_DP(2, false); }
     else { if (grad) TDW_DP(3, true); else TDW_DP(3, false); }
 #undef TDW_DP
-    double tr = dens_transverse(c);
-    if (grad) hipLaunchKernelGGL(k_dens_final<true>, dim3(nblk), dim3(NT), 0, c->stream, c->d_part, nchunk, N, tr, dens);
-    else hipLaunchKernelGGL(k_dens_final<false>, dim3(nblk), dim3(NT), 0, c->stream, c->d_part, nchunk, N, tr, dens);
     TDW_TRY((int)hipGetLastError());
-    return spin_fold(c, dens);
+    const ChunkSrc plain{c->d_part, 4, {2, 3, 0, -1, -1, -1, -1, 1, -1, -1, -1, -1}};
+    const ChunkSrc full{c->d_part, 12, {2, 3, 0, 4, 6, 7, 8, 1, 5, 9, 10, 11}};
+    return chunk_final(c, grad ? full : plain, CHUNK_NONE, nchunk, dens);
 }
 
 int densities(tdw_ctx *c, int n, const double2 *wf, const double2 *ddx, const double2 *ddy,
@@ -772,8 +804,7 @@ int apply_h(tdw_ctx *c, int it, int n, const double2 *in, double2 *out, const do
                        chunk, c->dim, c->p.functional == TDW_BDG, c->p.mu_a, c->p.mu_b, c->d_part);
     const double *q = useqpe;
     if (!q) {
-        hipLaunchKernelGGL(k_rowsum, dim3((n + 255) / 256), dim3(256), 0, c->stream, c->d_part, n, nchunk,
-                           dvol_norm(c), d_qpe);
+        TDW_TRY(row_sums(c, c->d_part, n, nchunk, dvol_norm(c), d_qpe));
         q = d_qpe;
     } else if (d_qpe && d_qpe != useqpe) {
         TDW_HIP(hipMemcpyAsync(d_qpe, useqpe, sizeof(double) * n, hipMemcpyDeviceToDevice, c->stream));
@@ -1014,8 +1045,7 @@ int apply_h_aslda(tdw_ctx *c, int n, const double2 *in, double2 *out, const doub
                        c->dim, c->p.mu_a, c->p.mu_b, c->d_part);
     const double *q = useqpe;
     if (!q) {
-        hipLaunchKernelGGL(k_rowsum, dim3((n + 255) / 256), dim3(256), 0, c->stream, c->d_part, n, nchunk,
-                           dvol_norm(c), d_qpe);
+        TDW_TRY(row_sums(c, c->d_part, n, nchunk, dvol_norm(c), d_qpe));
         q = d_qpe;
     } else if (d_qpe && d_qpe != useqpe) {
         TDW_HIP(hipMemcpyAsync(d_qpe, useqpe, sizeof(double) * n, hipMemcpyDeviceToDevice, c->stream));
@@ -1138,7 +1168,7 @@ int energy(tdw_ctx *c, int it, const double *dens, const double *pots, double *h
         TDW_TRY(c->proj->modify_energies(c->stream, it, (double *)dens, (double *)pots, pp));
         hipLaunchKernelGGL(k_pp_sum, dim3(nb), dim3(NT), 0, c->stream, N, pp, c->d_part);
     }
-    hipLaunchKernelGGL(k_rowsum, dim3(1), dim3(64), 0, c->stream, c->d_part, TDW_NITEMS, nb, 1.0, c->d_esum);
+    TDW_TRY(row_sums(c, c->d_part, TDW_NITEMS, nb, 1.0, c->d_esum));
     TDW_HIP(hipGetLastError());
     double e[TDW_NITEMS];
     TDW_HIP(hipMemcpyAsync(e, c->d_esum, sizeof(e), hipMemcpyDeviceToHost, c->stream));

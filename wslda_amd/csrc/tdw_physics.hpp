@@ -128,6 +128,19 @@ int density_tau(tdw_ctx *c, double *dens);
 // double nu, copy b to a (no-op when the mode is off)
 int spin_fold(tdw_ctx *c, double *dens);
 int copy_f64(tdw_ctx *c, const double *src, double *dst, long n);
+// out[a] = scale * sum of the m values of row a of part (n rows)
+int row_sums(tdw_ctx *c, const double *part, int n, int m, double scale, double *out);
+// partial densities of state chunks: nf fields of N points per chunk, f[o]
+// the field that contributes to output o of the density block (-1: none)
+struct ChunkSrc {
+    const double *part;
+    int nf;
+    int f[12];
+};
+static const ChunkSrc CHUNK_NONE{nullptr, 0, {-1, -1, -1, -1, -1, -1, -1, -1, -1, -1, -1, -1}};
+// the density block from the partials A + B of nchunk chunks (with the spin
+// fold where the mode is on)
+int chunk_final(tdw_ctx *c, const ChunkSrc &A, const ChunkSrc &B, int nchunk, double *dens);
 // grid-field helpers (tdw_grid.hip): spectral gradient, per-component
 // derivative and divergence of real fields (evolved axes only), the
 // Fermi-Dirac filter FD(k^2/2) of n real fields or one complex field, and the
