@@ -1,0 +1,90 @@
+"""The pointwise functional over the whole range of its inputs, through the C
+ABI against the CPU oracle: densities from far below the regularisation
+threshold to several times the uniform gas, mean fields on both sides of the
+band bottom (real and imaginary p0) and energies below the cutoff's reach
+(imaginary k_c), each functional, both regularisation schemes."""
+import ctypes as C
+
+import numpy as np
+import pytest
+
+from oracle import pyoracle as po
+from tests import tdgauss
+from tests.test_gpu_parity import cuda, say
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def torch():
+    import torch as t
+    if not t.cuda.is_available():
+        pytest.skip("no HIP device")
+    return t
+
+
+def inputs(N, seed):
+    r = np.random.default_rng(seed)
+    dens, pots = np.zeros(12 * N), np.zeros(12 * N)
+    na = 10.0 ** r.uniform(-8.5, -0.8, N)
+    nb = na * np.where(r.random(N) < 0.2, 1.0, r.uniform(0.0, 1.0, N))
+    nu = 0.5 * np.sqrt(na * nb) * np.exp(2j * np.pi * r.random(N))
+    dens[:2 * N] = nu.view(np.float64)
+    dens[2 * N:3 * N], dens[7 * N:8 * N] = na, nb
+    for k, n in ((3, na), (8, nb)):
+        dens[k * N:(k + 1) * N] = n ** (5 / 3) * r.uniform(0.5, 5.0, N)
+        for d in range(1, 4):
+            dens[(k + d) * N:(k + d + 1) * N] = n * r.uniform(-0.3, 0.3, N)
+    # V from well below to well above mu: the loop starts on either branch
+    pots[:2 * N] = r.uniform(-3.0, 3.0, 2 * N)
+    pots[2 * N:4 * N] = r.uniform(-0.5, 0.5, 2 * N)
+    pots[4 * N:6 * N] = r.uniform(0.9, 1.2, 2 * N)
+    return dens, pots
+
+
+@pytest.mark.parametrize("functional,a1", [(po.SLDA, 0), (po.BDG, 0), (po.ASLDA, 0), (po.SLDAE, 0), (po.SLDAE, 1)])
+@pytest.mark.parametrize("reg", [88, 89])
+@pytest.mark.parametrize("ec", [4.9, 0.3])
+def test_potentials_over_the_input_range(torch, functional, a1, reg, ec):
+    from wslda_amd import td
+    say("case: potentials functional=%d a1=%d regularization=%d ec=%.1f" % (functional, a1, reg, ec))
+    cfg = po.make_cfg(2, 24, 16, 4, dx=1.1, functional=functional, force_a1=a1,
+                      sclgth=-0.9 if functional in (po.BDG, po.SLDAE) else 0.0)
+    cfg.regularization, cfg.mf_correction = reg, 1
+    cfg.mu_a, cfg.mu_b, cfg.ec = 0.25, 0.2, ec
+    N = po.npts(cfg)
+    dens, pots = inputs(N, 7 + functional + reg)
+
+    def oracle(d, p):
+        p = p.copy()
+        po.lib().tdwo_potentials(C.byref(cfg), 1, po.ptr(np.ascontiguousarray(d)), po.ptr(p))
+        return p
+
+    ref = oracle(dens, pots)
+    # what a relative change of the inputs by 1e-13 does to the oracle's own
+    # result: the loop amplifies rounding near its resonance C~ = Re wz and
+    # near k_c = p0, where no two correct evaluations agree to round-off
+    r = np.random.default_rng(1)
+    amp = np.zeros_like(ref)
+    for _ in range(6):
+        amp = np.maximum(amp, np.abs(oracle(dens * (1 + 1e-13 * r.choice([-1, 1], dens.size)),
+                                            pots * (1 + 1e-13 * r.choice([-1, 1], pots.size))) - ref))
+    prm = tdgauss.to_params(cfg, td.FP64)
+    ctx = td.TDContext(prm, 4, 0)
+    dd, dp = cuda(torch, dens), cuda(torch, pots)
+    ctx.compute_potentials(1, dd, dp)
+    ctx.sync()
+    got = dp.cpu().numpy()
+    ctx.close()
+    assert np.array_equal(np.isnan(got), np.isnan(ref))
+    ok = ~np.isnan(ref)
+    # every point within ten times that amplification (the results of the
+    # point: V_a, V_b and Delta share one loop), plus round-off of the result
+    a = np.zeros(N)
+    for k in range(12):
+        f = amp[k * N:(k + 1) * N] if k not in (2, 3) else amp[2 * N:4 * N].reshape(N, 2).max(1)
+        a = np.maximum(a, np.where(np.isnan(f), 0.0, f))
+    lim = np.concatenate([np.repeat(a, 2) if k == 2 else a for k in range(12) if k != 3])
+    lim = 10.0 * lim + 1e-12 * np.maximum(np.abs(ref), 1.0)
+    d = np.abs(got - ref)
+    assert (d[ok] <= lim[ok]).all(), (d[ok] / lim[ok]).max()

@@ -67,6 +67,50 @@ __device__ __forceinline__ void abm_sums(double2 a, double2 b, double2 d, double
     }
 }
 
+// Reciprocal, square root and logarithm of positive normal numbers of
+// moderate size (about 1e-100 to 1e100), to two or three units in the last
+// place: the library functions handle every argument, with scaling,
+// exponent and special-case code that makes them two to four times as long
+// (the logarithm some 95 instructions against 35), which counts where a
+// chain of them is all that a kernel waits for.  Hardware estimates refined
+// by Newton steps (the estimates hold 23 bits or more, so two steps reach
+// double precision).
+__device__ __forceinline__ double rcp_pos(double x)
+{
+    double r = __builtin_amdgcn_rcp(x);
+    r = fma(fma(-x, r, 1.0), r, r);
+    return fma(fma(-x, r, 1.0), r, r);
+}
+__device__ __forceinline__ double sqrt_pos(double x)
+{
+    // g -> sqrt(x), h -> 1 / (2 sqrt(x)) together
+    const double y = __builtin_amdgcn_rsq(x);
+    double g = x * y, h = 0.5 * y;
+    double r = fma(-g, h, 0.5);
+    g = fma(g, r, g);
+    h = fma(h, r, h);
+    return fma(fma(-g, g, x), h, g);
+}
+// log x = e log 2 + 2 atanh(s), s = (m - 1) / (m + 1) for x = m 2^e with m in
+// [sqrt(1/2), sqrt(2)): |s| < 0.1716, so the series s + s^3/3 + ... ends
+// below 2^-56 of s after s^21
+__device__ __forceinline__ double log_pos(double x)
+{
+    int e = __builtin_amdgcn_frexp_exp(x);
+    double m = __builtin_amdgcn_frexp_mant(x);   // [1/2, 1)
+    const bool up = m < 0.70710678118654752440;
+    m = up ? m + m : m;
+    e -= up ? 1 : 0;
+    const double a = m - 1.0, b = m + 1.0, r = rcp_pos(b);
+    double s = a * r;
+    s = fma(fma(-b, s, a), r, s);
+    const double z = s * s, z2 = z * z, z4 = z2 * z2;
+    const double p01 = fma(z, 1. / 5., 1. / 3.), p23 = fma(z, 1. / 9., 1. / 7.), p45 = fma(z, 1. / 13., 1. / 11.),
+                 p67 = fma(z, 1. / 17., 1. / 15.), p89 = fma(z, 1. / 21., 1. / 19.);
+    const double p = fma(z4, fma(z4, p89, fma(z2, p67, p45)), fma(z2, p23, p01));
+    return fma((double)e, 0.69314718055994530942, 2.0 * fma(s * z, p, s));
+}
+
 // Lattice momentum of index i on an axis of n points and length L, standard
 // FFT order (hpc-engine/pca_derivative.cu:150-160).
 __device__ __forceinline__ double kval(int i, int n, double L)

@@ -121,7 +121,7 @@ __host__ __device__ __forceinline__ double ad_hypot(double x, double y) { return
 template <int K> __host__ __device__ __forceinline__ Dual<K> ad_pow(const Dual<K> &x, double e)
 {
     const double p = pow(x.v, e);
-    return dlin(p, e * pow(x.v, e - 1.0), x);
+    return dlin(p, e * (x.v != 0.0 ? p / x.v : pow(x.v, e - 1.0)), x);
 }
 template <int K> __host__ __device__ __forceinline__ Dual<K> ad_sqrt(const Dual<K> &x)
 {

@@ -66,27 +66,35 @@ __device__ __forceinline__ double funD(const FParams &f, double na, double nb)
            (funG(p) - alpha_f(p) * pow((1.0 + p) / 2.0, 5.0 / 3.0) -
             alpha_f(-1.0 * p) * pow((1.0 - p) / 2.0, 5.0 / 3.0));
 }
-// dD/dn_a (wrt_b=0) or dD/dn_b (wrt_b=1), pca_edf.h:232-296 with A1=A2=0.
-__device__ __forceinline__ double der_funD(const FParams &f, double na, double nb, int wrt_b)
+// x^(1/3), NaN for x < 0 as pow gives.  The functional's powers of 1/3, 2/3
+// and 5/3 are products of it: one cbrt instead of a pow each.
+__device__ __forceinline__ double c13(double x) { return x < 0.0 ? nan("") : cbrt(x); }
+
+// What the mixing loop holds fixed at a point: dD/dn_a, dD/dn_b, C~ and its
+// derivatives (ccoeff = 1), with alpha(p), alpha(-p), alpha_plus and their
+// p-derivatives given (pca_edf.h:232-352).
+struct EdfConst {
+    double dDa, dDb, C, dCa, dCb;
+};
+__device__ __forceinline__ EdfConst edf_const(const FParams &f, double n, double p, double dpa, double dpb,
+                                              double g0, double g1, double gamma0, double al_p, double al_m,
+                                              double dal_p, double dal_m, double alph_plus, double dalph_plus)
 {
-    double p = polar(f, na, nb);
-    double base = funG(p) - alpha_f(p) * pow((1.0 + p) / 2.0, 5.0 / 3.0) -
-                  alpha_f(-1.0 * p) * pow((1.0 - p) / 2.0, 5.0 / 3.0);
-    double dpol = der_pol(f, na, nb, wrt_b);
-    return (1.0 / 2.0) * pow(6.0 * M_PI * M_PI * (na + nb), 2.0 / 3.0) * base +
-           (1.0 / (20.0 * M_PI * M_PI)) * pow(6.0 * M_PI * M_PI * (na + nb), 5.0 / 3.0) *
-               (2.0 * TDW_G1 * p - (5.0 / 6.0) * alpha_f(p) * pow((1.0 + p) / 2.0, 2.0 / 3.0) +
-                (5.0 / 6.0) * alpha_f(-1.0 * p) * pow((1.0 - p) / 2.0, 2.0 / 3.0)) *
-               dpol;
-}
-__device__ __forceinline__ double tildeC(const FParams &f, double na, double nb)
-{
-    return TDW_A0 * pow(na + nb + f.denseps, 1.0 / 3.0) / (TDW_GAMMA0 * 1.0);
-}
-__device__ __forceinline__ double der_tildeC(const FParams &f, double na, double nb)
-{
-    // d(alpha_plus)/dn = 0 for A2 = 0
-    return ((1.0 / 3.0) * TDW_A0 * pow(na + nb + f.denseps, -2.0 / 3.0)) / (TDW_GAMMA0 * 1.0);
+    EdfConst r;
+    const double x = 6.0 * M_PI * M_PI * n, c = c13(x), x23 = c * c;
+    const double hp = (1.0 + p) / 2.0, hm = (1.0 - p) / 2.0;
+    const double cp = c13(hp), cm = c13(hm), hp23 = cp * cp, hm23 = cm * cm;
+    const double base = g0 + g1 * p * p - al_p * (hp * hp23) - al_m * (hm * hm23);
+    const double s = 2.0 * g1 * p - dal_p * (hp * hp23) - (5.0 / 6.0) * al_p * hp23 - dal_m * (hm * hm23) +
+                     (5.0 / 6.0) * al_m * hm23;
+    const double d0 = 0.5 * x23 * base, d1 = (1.0 / (20.0 * M_PI * M_PI)) * (x * x23) * s;
+    r.dDa = d0 + d1 * dpa;
+    r.dDb = d0 + d1 * dpb;
+    const double ce = c13(n + f.denseps), dce = (1.0 / 3.0) * alph_plus / (ce * ce);
+    r.C = alph_plus * ce / gamma0;
+    r.dCa = (dalph_plus * dpa * ce + dce) / gamma0;
+    r.dCb = (dalph_plus * dpb * ce + dce) / gamma0;
+    return r;
 }
 
 // complex helpers on double2 for the regularisation (principal branches, as
@@ -107,41 +115,105 @@ __device__ __forceinline__ double2 clog2(double2 z)
 }
 
 // One evaluation of the regularised coupling (tdwslda_functionals.h:251-265)
-// given mu_+ - V_+ = t7 and the alpha_plus scaling; returns wz before the
-// final inversion and p0 (for the mean-field correction).
-__device__ __forceinline__ void reg_wz(const FParams &f, double t7, double alph_plus, double kscale,
-                                       double2 &wz, double2 &p0)
+// given t7 = mu_+ - V_+ and kscale2 = 2 / alpha_plus for SLDA (p0 =
+// sqrt(2 t7 / alpha)), 2 for BdG: wz = R0 (k_c - R1 p0 log((k_c + p0)/(k_c -
+// p0))) before the final inversion, and p0 (for the mean-field correction).
+__device__ __forceinline__ void reg_wz(const FParams &f, double t7, double kscale2, double2 &wz, double2 &p0)
 {
-    // kscale = alph_plus for SLDA (p0 = sqrt(2 t7/alpha)), 1 for BdG
-    p0 = csqrt_real(2.0 * t7 / kscale);
-    if (p0.y < 0.) p0 = make_double2(-p0.x, -p0.y);
-    double2 kc;
-    if (f.cubic) kc = make_double2(M_PI / f.dx, 0.0);
-    else {
-        kc = csqrt_real(2.0 * (f.ec + t7) / kscale);
-        if (kc.y < 0.) kc = make_double2(-kc.x, -kc.y);
-    }
+    p0 = csqrt_real(t7 * kscale2);
+    const double2 kc = f.cubic ? make_double2(M_PI / f.dx, 0.0) : csqrt_real((f.ec + t7) * kscale2);
     double2 w = clog2(cdiv(kc + p0, kc - p0));
     if (w.y < 0.) w.y += 2. * M_PI;
-    // kc*R0*(1 - (p0/kc)*R1*w)
-    double2 q = cmul(cdiv(p0, kc), w) * f.R1;
-    double2 one_m = make_double2(1.0 - q.x, -q.y);
-    wz = cmul(kc, one_m) * f.R0;
+    wz = (kc - cmul(p0, w) * f.R1) * f.R0;
+}
+// Re(a / (c - wz)), a and c real
+__device__ __forceinline__ double re_inv(double a, double c, double2 wz)
+{
+    const double d = c - wz.x;
+    return wz.y == 0.0 ? a / d : a * d / (d * d + wz.y * wz.y);
 }
 
-// Mean-field correction of the regularisation scheme (:268-290); returns
-// dLam/dn or 0.
-__device__ __forceinline__ double mf_corr(const FParams &f, double2 p0, double wz_re, double lkF,
-                                          double n, double alph_plus)
+// Mean-field correction of the regularisation scheme (:268-290), dLam/dn or
+// 0.  With b = Re p0 / k_F and lx = b k_F dx / pi the reference's
+// (k_F / (3 n alpha)) (Lam0 + dLam0 b dx k_F / pi) is
+//   -(k_F / (3 n alpha)) R0 R1 b (log((1 + lx)/(1 - lx)) + 2 lx / (1 - lx^2))
+// (its two terms of opposite sign, b R0 / lx, cancel).
+struct MfConst {
+    double ikF, fx, pre;   // 1 / (k_F + 1e-12), k_F dx / pi, -k_F R0 R1 / (3 n alpha)
+};
+__device__ __forceinline__ MfConst mf_const(const FParams &f, double n, double alph_plus)
 {
-    double bcoeff = p0.x / (lkF + 1.0e-12);
-    double lx = bcoeff * lkF * f.dx / M_PI;
-    if (wz_re < -1.0e-10 && lx > 1.0e-10) {
-        double Lam0 = bcoeff * f.R0 / lx * (1.0 - f.R1 * lx * log((1.0 + lx) / (1.0 - lx)));
-        double dLam0 = (-2. * bcoeff * f.R0 * f.R1) / (1. - lx * lx) - bcoeff * f.R0 / lx / lx;
-        return (lkF / (3. * n * alph_plus)) * (Lam0 + dLam0 * bcoeff * f.dx * lkF / M_PI);
+    MfConst m;
+    const double kF = c13(3.0 * M_PI * M_PI * n);
+    m.ikF = 1.0 / (kF + 1.0e-12);
+    m.fx = kF * f.dx / M_PI;
+    m.pre = -(kF / (3. * n * alph_plus)) * f.R0 * f.R1;
+    return m;
+}
+__device__ __forceinline__ double mf_corr(const MfConst &m, double p0x, double g)
+{
+    const double b = p0x * m.ikF, lx = b * m.fx;
+    const double q = 1.0 / ((1.0 - lx) * (1.0 + lx));
+    const double v = m.pre * b * (log((1.0 + lx) * (1.0 + lx) * q) + 2.0 * lx * q);
+    return (g < -1.0e-10 && lx > 1.0e-10) ? v : 0.0;
+}
+
+// The same two above the band bottom: p0 = p and k_c real, p < k_c, lx < 1.
+// With k_c^2 - p^2 = d (2 ec / alpha, or (pi / dx)^2 - p^2) the logarithm's
+// argument is (k_c + p)^2 / d.  Arguments are positive and of order one, so
+// short square roots, reciprocals and logarithms do (see tdw_device.hpp).
+__device__ __forceinline__ bool reg_real(const FParams &f, const MfConst &m, double t7, double kscale2, double &wz,
+                                         double &mfv, double &lx)
+{
+    const double p2 = t7 * kscale2, kc2 = f.cubic ? (M_PI / f.dx) * (M_PI / f.dx) : (f.ec + t7) * kscale2;
+    const double d = f.cubic ? kc2 - p2 : f.ec * kscale2;
+    const double p = sqrt_pos(p2), k = f.cubic ? M_PI / f.dx : sqrt_pos(kc2);
+    const double b = p * m.ikF;
+    lx = b * m.fx;
+    const double q = rcp_pos((1.0 - lx) * (1.0 + lx));
+    const double l1 = log_pos((k + p) * (k + p) * rcp_pos(d)), l2 = log_pos((1.0 + lx) * (1.0 + lx) * q);
+    wz = (k - f.R1 * p * l1) * f.R0;
+    mfv = m.pre * b * (l2 + 2.0 * lx * q);
+    // small or large arguments, and every other branch, take the general form
+    return p2 >= 1.0e-30 && p2 < 1.0e30 && d > 1.0e-10 * kc2 && kc2 < 1.0e30 && lx < 0.999;
+}
+
+// The 15 mixing iterations of V_a, V_b and Delta = -nu Re(alpha_+ / (C - wz))
+// (tdwslda_functionals.h:236-300) from the previous V_a, V_b: each new V_s is
+// V_s,const - e_s Re(Delta* nu) - c_s |Delta|^2 + the mean-field correction.
+__device__ __forceinline__ void mix_loop(const FParams &f, double n, double2 nu, double alph_plus, double C,
+                                         double Va_const, double Vb_const, double ea, double eb, double ca, double cb,
+                                         double &Va, double &Vb, double2 &delta)
+{
+    // The loop is a chain of fifteen evaluations per point with too few points
+    // to hide it: with the general form alone (complex logarithm, five
+    // divisions and two logarithms one after the other) it was most of the 25
+    // us that k_potentials took on 64 points, and a third of that problem's
+    // step.  A wave whose points are all above the band bottom takes reg_real,
+    // one straight run in which the two logarithms overlap: 10.7 us.
+    const double kscale2 = 2.0 / alph_plus, nu2 = nu.x * nu.x + nu.y * nu.y;
+    MfConst m{0.0, 0.0, 0.0};
+    if (f.mf) m = mf_const(f, n, alph_plus);
+    double g = 0.0;
+    for (int k = 0; k < TDW_UD_SCITERS; k++) {
+        const double t7 = (f.mu_a - Va + f.mu_b - Vb) / 2.0;
+        double wr, mfv, lx, dl = 0.0;
+        if (__all(reg_real(f, m, t7, kscale2, wr, mfv, lx))) {
+            g = alph_plus / (C - wr);
+            dl = (f.mf && g < -1.0e-10 && lx > 1.0e-10) ? mfv : 0.0;
+        } else {
+            double2 wz, p0;
+            reg_wz(f, t7, kscale2, wz, p0);
+            g = re_inv(alph_plus, C, wz);
+            if (f.mf) dl = mf_corr(m, p0.x, g);
+        }
+        const double dn = -g * nu2, d2 = g * g * nu2;   // Re(Delta* nu), |Delta|^2
+        const double Vanew = Va_const - ea * dn - ca * d2 + dl * d2;
+        const double Vbnew = Vb_const - eb * dn - cb * d2 + dl * d2;
+        Va = TDW_UD_MIX * Vanew + (1.0 - TDW_UD_MIX) * Va;
+        Vb = TDW_UD_MIX * Vbnew + (1.0 - TDW_UD_MIX) * Vb;
     }
-    return 0.0;
+    delta = nu * (-1.0 * g);
 }
 
 // SLDA potentials at one point (tdwslda_functionals.h:47-306, FAST mode).
@@ -149,36 +221,10 @@ __device__ __forceinline__ void slda_point(const FParams &f, double na, double n
                                            double ua, double ub, double &Va, double &Vb,
                                            double2 &delta)
 {
-    const double alph_plus = TDW_A0;
-    double Va_const = ua + der_funD(f, na, nb, 0);
-    double Vb_const = ub + der_funD(f, na, nb, 1);
-    const double t3 = der_tildeC(f, na, nb) / alph_plus;
-    const double t4 = t3;
-    const double t5 = tildeC(f, na, nb);
-    double lkF = 0.0;
-    if (f.mf) lkF = pow(3.0 * M_PI * M_PI * (na + nb), 1.0 / 3.0);
-    double2 ld = make_double2(0.0, 0.0);
-    for (int k = 0; k < TDW_UD_SCITERS; k++) {
-        double t7 = (f.mu_a - Va + f.mu_b - Vb) / 2.0;
-        double2 wz, p0;
-        reg_wz(f, t7, alph_plus, alph_plus, wz, p0);
-        // alph_plus / (t5 - wz)
-        double2 g = cdiv(make_double2(alph_plus, 0.0), make_double2(t5 - wz.x, -wz.y));
-        ld = nu * (-1.0 * g.x);
-        double t6 = ld.x * nu.x + ld.y * nu.y;   // Re(conj(delta) * nu)
-        double t7b = ld.x * ld.x + ld.y * ld.y;
-        (void)t6;   // t1 = t2 = 0 in FAST mode
-        double Vanew = Va_const - t3 * t7b;
-        double Vbnew = Vb_const - t4 * t7b;
-        if (f.mf) {
-            double dl = mf_corr(f, p0, g.x, lkF, na + nb, alph_plus);
-            Vanew += dl * t7b;
-            Vbnew += dl * t7b;
-        }
-        Va = TDW_UD_MIX * Vanew + (1.0 - TDW_UD_MIX) * Va;
-        Vb = TDW_UD_MIX * Vbnew + (1.0 - TDW_UD_MIX) * Vb;
-    }
-    delta = ld;
+    const double n = na + nb, p = polar(f, na, nb);
+    const EdfConst e = edf_const(f, n, p, der_pol(f, na, nb, 0), der_pol(f, na, nb, 1), TDW_G0, TDW_G1, TDW_GAMMA0,
+                                 TDW_A0, TDW_A0, 0.0, 0.0, TDW_A0, 0.0);
+    mix_loop(f, n, nu, TDW_A0, e.C, ua + e.dDa, ub + e.dDb, 0.0, 0.0, e.dCa / TDW_A0, e.dCb / TDW_A0, Va, Vb, delta);
 }
 
 // ASLDA potentials at one point (tdwslda_functionals.h:47-306 without
@@ -216,8 +262,13 @@ __device__ __forceinline__ void aslda_point(const FParams &f, double na, double 
     Vb_const += dalphm_dnb * (taua - taub) / 2.0;
     Va_const += dalphp_dna * (taua + taub) / 2.0;
     Vb_const += dalphp_dnb * (taua + taub) / 2.0;
-    Va_const += aslda::der_funD(n, p, dpa);
-    Vb_const += aslda::der_funD(n, p, dpb);
+    // d alpha(p)/dp and d alpha(-p)/dp as pca_edf.h:245-314 takes them
+    const EdfConst e = edf_const(f, n, p, dpa, dpb, aslda::G0, aslda::G1, aslda::GAMMA0, aA, aB,
+                                 aslda::dalpha_plus_dp(p) + aslda::dalpha_minus_dp(p),
+                                 aslda::dalpha_plus_dp(p) - aslda::dalpha_minus_dp(p), alph_plus,
+                                 aslda::dalpha_plus_dp(p));
+    Va_const += e.dDa;
+    Vb_const += e.dDb;
     if (fa != 0.0) {
         const double t7 = fa * j2a / (2.0 * na);
         Va_const += ((alph_plus + alph_minus - 1.0) / na - (dalphp_dna + dalphm_dna)) * t7;
@@ -230,32 +281,8 @@ __device__ __forceinline__ void aslda_point(const FParams &f, double na, double 
         Vb_const += ((alph_plus - alph_minus - 1.0) / nb - (dalphp_dnb - dalphm_dnb)) * t7;
         Vb_const -= cc * der_p_reg(f, nb) * (alph_plus - alph_minus - 1.0) * j2b / (2.0 * nb);
     }
-    const double t1 = dalphp_dna / alph_plus, t2 = dalphp_dnb / alph_plus;
-    const double t3 = aslda::der_tildeC(n, p, dpa, f.denseps) / alph_plus;
-    const double t4 = aslda::der_tildeC(n, p, dpb, f.denseps) / alph_plus;
-    const double t5 = aslda::tildeC(n, p, f.denseps);
-    double lkF = 0.0;
-    if (f.mf) lkF = pow(3.0 * M_PI * M_PI * n, 1.0 / 3.0);
-    double2 ld = make_double2(0.0, 0.0);
-    for (int k = 0; k < TDW_UD_SCITERS; k++) {
-        double t7 = (f.mu_a - Va + f.mu_b - Vb) / 2.0;
-        double2 wz, p0;
-        reg_wz(f, t7, alph_plus, alph_plus, wz, p0);
-        double2 g = cdiv(make_double2(alph_plus, 0.0), make_double2(t5 - wz.x, -wz.y));
-        ld = nu * (-1.0 * g.x);
-        const double t6 = ld.x * nu.x + ld.y * nu.y;   // Re(conj(delta) * nu)
-        const double t7b = ld.x * ld.x + ld.y * ld.y;
-        double Vanew = Va_const - t1 * t6 - t3 * t7b;
-        double Vbnew = Vb_const - t2 * t6 - t4 * t7b;
-        if (f.mf) {
-            double dl = mf_corr(f, p0, g.x, lkF, n, alph_plus);
-            Vanew += dl * t7b;
-            Vbnew += dl * t7b;
-        }
-        Va = TDW_UD_MIX * Vanew + (1.0 - TDW_UD_MIX) * Va;
-        Vb = TDW_UD_MIX * Vbnew + (1.0 - TDW_UD_MIX) * Vb;
-    }
-    delta = ld;
+    mix_loop(f, n, nu, alph_plus, e.C, Va_const, Vb_const, dalphp_dna / alph_plus, dalphp_dnb / alph_plus,
+             e.dCa / alph_plus, e.dCb / alph_plus, Va, Vb, delta);
 }
 
 // SLDAE potentials at one point (tdwslda_functionals.h:530-812, with
@@ -300,28 +327,8 @@ __device__ __forceinline__ void sldae_point(const FParams &f, double na, double 
         Vb_const += ((af - 1.0) / nb - af_p) * t7;
         Vb_const -= cc * der_p_reg(f, nb) * (af - 1.0) * j2b / (2.0 * nb);
     }
-    double lkF = 0.0;
-    if (f.mf) lkF = pow(3.0 * M_PI * M_PI * n, 1.0 / 3.0);
-    double2 ld = make_double2(0.0, 0.0);
-    for (int k = 0; k < TDW_UD_SCITERS; k++) {
-        const double lmu = (f.mu_a - Va + f.mu_b - Vb) / 2.0;
-        double2 wz, p0;
-        reg_wz(f, lmu, af, af, wz, p0);
-        const double g_eff = af / (L.ctilde - wz.x);
-        ld = nu * (-1.0 * g_eff);
-        const double dn = ld.x * nu.x + ld.y * nu.y;   // Re(conj(delta) * nu)
-        const double d2 = ld.x * ld.x + ld.y * ld.y;
-        double Vanew = Va_const - (af_p / af) * dn - L.ctilde_p / af * d2;
-        double Vbnew = Vb_const - (af_p / af) * dn - L.ctilde_p / af * d2;
-        if (f.mf) {
-            const double dl = mf_corr(f, p0, g_eff, lkF, n, af);
-            Vanew += dl * d2;
-            Vbnew += dl * d2;
-        }
-        Va = TDW_UD_MIX * Vanew + (1.0 - TDW_UD_MIX) * Va;
-        Vb = TDW_UD_MIX * Vbnew + (1.0 - TDW_UD_MIX) * Vb;
-    }
-    delta = ld;
+    mix_loop(f, n, nu, af, L.ctilde, Va_const, Vb_const, af_p / af, af_p / af, L.ctilde_p / af, L.ctilde_p / af, Va, Vb,
+             delta);
 }
 
 // BdG potentials at one point (tdwslda_functionals.h:373-452).
@@ -331,17 +338,15 @@ __device__ __forceinline__ void bdg_point(const FParams &f, double na, double nb
 {
     const double alph_plus = 0.5 * (al_a + al_b);
     const double t5 = 1.0 / (4.0 * M_PI * f.sclgth * alph_plus);
-    double nab = na + nb;
-    double lkF = f.mf ? pow(3.0 * M_PI * M_PI * nab, 1.0 / 3.0) : 0.0;
     double t7 = (f.mu_a - Va + f.mu_b - Vb) / 2.0;
     double2 wz, p0;
-    reg_wz(f, t7, alph_plus, 1.0, wz, p0);
+    reg_wz(f, t7, 2.0, wz, p0);
     wz = wz * (1.0 / alph_plus);
-    double2 g = cdiv(make_double2(1.0, 0.0), make_double2(t5 - wz.x, -wz.y));
-    double2 ld = nu * (-1.0 * g.x);
+    const double g = re_inv(1.0, t5, wz);
+    double2 ld = nu * (-1.0 * g);
     double nVa = ua, nVb = ub;
     if (f.mf) {
-        double dl = mf_corr(f, p0, g.x, lkF, nab, alph_plus);
+        const double dl = mf_corr(mf_const(f, na + nb, alph_plus), p0.x, g);
         double t7b = ld.x * ld.x + ld.y * ld.y;
         nVa += dl * t7b;
         nVb += dl * t7b;

@@ -77,34 +77,39 @@ template <typename R> __host__ __device__ __forceinline__ Cx<R> csqrt_real(const
     return cx<R>(S<R>::c(0.0), ad_sqrt(-x));
 }
 
+// the real branch above the band bottom as in tdw_functional.hpp; real: wz
+// and p0 are real with zero tangents in their imaginary parts
 template <typename R>
-__host__ __device__ __forceinline__ void reg_wz(const FParams &f, const R &t7, double alph_plus, Cx<R> &wz, Cx<R> &p0)
+__host__ __device__ __forceinline__ bool reg_wz(const FParams &f, const R &t7, double alph_plus, Cx<R> &wz, Cx<R> &p0)
 {
-    p0 = csqrt_real(2.0 * t7 / alph_plus);
-    if (val(p0.y) < 0.) p0 = cx<R>(-p0.x, -p0.y);
-    Cx<R> kc;
-    if (f.cubic) kc = cx<R>(S<R>::c(M_PI / f.dx), S<R>::c(0.0));
-    else {
-        kc = csqrt_real(2.0 * (f.ec + t7) / alph_plus);
-        if (val(kc.y) < 0.) kc = cx<R>(-kc.x, -kc.y);
+    const R z = S<R>::c(0.0), kc2 = (2.0 / alph_plus) * (f.ec + t7), p02 = (2.0 / alph_plus) * t7;
+    if (val(t7) >= 0.0 && (f.cubic || val(kc2) >= 0.0)) {
+        const R p = ad_sqrt(p02), k = f.cubic ? S<R>::c(M_PI / f.dx) : ad_sqrt(kc2);
+        if (val(k) > val(p)) {
+            p0 = cx<R>(p, z);
+            wz = cx<R>((k - f.R1 * (p * ad_log((k + p) / (k - p)))) * f.R0, z);
+            return true;
+        }
     }
+    p0 = csqrt_real(p02);
+    Cx<R> kc = f.cubic ? cx<R>(S<R>::c(M_PI / f.dx), z) : csqrt_real(kc2);
     Cx<R> w = cxlog(cxdiv(kc + p0, kc - p0));
     if (val(w.y) < 0.) w.y = w.y + 2. * M_PI;
-    Cx<R> q = cxscale(cxmul(cxdiv(p0, kc), w), f.R1);
-    Cx<R> one_m = cx<R>(1.0 - q.x, -q.y);
-    wz = cxscale(cxmul(kc, one_m), f.R0);
+    wz = cxscale(kc - cxscale(cxmul(p0, w), f.R1), f.R0);
+    return false;
 }
 
+// (see mf_corr of tdw_functional.hpp for the form)
 template <typename R>
-__host__ __device__ __forceinline__ R mf_corr(const FParams &f, const Cx<R> &p0, const R &wz_re, const R &lkF,
-                                              const R &n, double alph_plus)
+__host__ __device__ __forceinline__ R mf_corr(const FParams &f, const R &p0x, const R &g, const R &lkF, const R &n,
+                                              double alph_plus)
 {
-    R bcoeff = p0.x / (lkF + 1.0e-12);
-    R lx = bcoeff * lkF * f.dx / M_PI;
-    if (val(wz_re) < -1.0e-10 && val(lx) > 1.0e-10) {
-        R Lam0 = bcoeff * f.R0 / lx * (1.0 - f.R1 * lx * ad_log((1.0 + lx) / (1.0 - lx)));
-        R dLam0 = (-2. * f.R0 * f.R1) * bcoeff / (1. - lx * lx) - bcoeff * f.R0 / lx / lx;
-        return (lkF / (3. * n * alph_plus)) * (Lam0 + dLam0 * bcoeff * f.dx * lkF / M_PI);
+    R b = p0x / (lkF + 1.0e-12);
+    R lx = b * lkF * (f.dx / M_PI);
+    if (val(g) < -1.0e-10 && val(lx) > 1.0e-10) {
+        R q = 1.0 / ((1.0 - lx) * (1.0 + lx));
+        return (-f.R0 * f.R1 / (3. * alph_plus)) * (lkF / n) * b *
+               (ad_log((1.0 + lx) * (1.0 + lx) * q) + 2.0 * (lx * q));
     }
     return S<R>::c(0.0);
 }
@@ -122,25 +127,26 @@ __host__ __device__ __forceinline__ void slda_point(const FParams &f, const R &n
     const R t5 = tildeC(f, na, nb);
     R lkF = S<R>::c(0.0);
     if (f.mf) lkF = ad_pow(3.0 * M_PI * M_PI * (na + nb), 1.0 / 3.0);
-    Cx<R> ld = cx<R>(S<R>::c(0.0), S<R>::c(0.0));
+    R g = S<R>::c(0.0);
+    const R nu2 = nu.x * nu.x + nu.y * nu.y;
     for (int k = 0; k < TDW_UD_SCITERS; k++) {
         R t7 = (f.mu_a - Va + f.mu_b - Vb) / 2.0;
         Cx<R> wz, p0;
-        reg_wz(f, t7, alph_plus, wz, p0);
-        Cx<R> g = cxdiv(cx<R>(S<R>::c(alph_plus), S<R>::c(0.0)), cx<R>(t5 - wz.x, -wz.y));
-        ld = cx<R>(nu.x * (-1.0 * g.x), nu.y * (-1.0 * g.x));
-        R t7b = ld.x * ld.x + ld.y * ld.y;
+        const bool real = reg_wz(f, t7, alph_plus, wz, p0);
+        const R d = t5 - wz.x;
+        g = real ? alph_plus / d : alph_plus * d / (d * d + wz.y * wz.y);
+        R t7b = (g * g) * nu2;
         R Vanew = Va_const - t3 * t7b;
         R Vbnew = Vb_const - t3 * t7b;
         if (f.mf) {
-            R dl = mf_corr(f, p0, g.x, lkF, na + nb, alph_plus);
+            R dl = mf_corr(f, p0.x, g, lkF, na + nb, alph_plus);
             Vanew = Vanew + dl * t7b;
             Vbnew = Vbnew + dl * t7b;
         }
         Va = TDW_UD_MIX * Vanew + (1.0 - TDW_UD_MIX) * Va;
         Vb = TDW_UD_MIX * Vbnew + (1.0 - TDW_UD_MIX) * Vb;
     }
-    delta = ld;
+    delta = cx<R>(-nu.x * g, -nu.y * g);
 }
 
 }  // namespace ad

@@ -686,11 +686,15 @@ FParams fparams(const tdw_ctx *c)
     return f;
 }
 
-__global__ void __launch_bounds__(NT)
+// one wave per workgroup: the points are few and each is a long chain, so
+// they are spread over as many CUs as there are waves
+static constexpr int PB = 64;
+
+__global__ void __launch_bounds__(PB)
 k_potentials(FParams f0, VextDev V, long N, int dim, double cc, const double *__restrict__ dens,
              double *__restrict__ pots)
 {
-    long i = (long)blockIdx.x * NT + threadIdx.x;
+    long i = (long)blockIdx.x * PB + threadIdx.x;
     if (i >= N) return;
     const double na = dens[2 * N + i], nb = dens[7 * N + i];
     const double2 nu = make_double2(dens[2 * i], dens[2 * i + 1]);
@@ -740,7 +744,7 @@ int potentials(tdw_ctx *c, int it, const double *dens, double *pots, double ccco
     long N = (long)c->N;
     FParams f = fparams(c);
     f.agrid = sclgth_grid(c, it);
-    hipLaunchKernelGGL(k_potentials, dim3((N + NT - 1) / NT), dim3(NT), 0, c->stream, f, make_vext(c, it), N,
+    hipLaunchKernelGGL(k_potentials, dim3((N + PB - 1) / PB), dim3(PB), 0, c->stream, f, make_vext(c, it), N,
                        c->dim, cccoeff, dens, pots);
     TDW_HIP(hipGetLastError());
     return project_modify_potentials(c, it, dens, pots);
