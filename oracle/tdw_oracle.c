@@ -103,7 +103,7 @@ typedef struct {
     int R[MAXSTAGES], Ns[MAXSTAGES];
     zc *tw[2][MAXSTAGES];   /* [sign][stage][k*R + t] */
 } fftplan;
-#define MAXPLANS 16
+#define MAXPLANS 64   /* axis lengths one process meets */
 static fftplan g_plans[MAXPLANS];
 static int g_nplans = 0;
 

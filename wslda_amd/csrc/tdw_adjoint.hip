@@ -17,6 +17,7 @@
 #include "tdw_fused.hpp"
 #include "tdw_internal.hpp"
 #include "tdw_physics.hpp"
+#include "tdw_resident.hpp"
 
 namespace tdw {
 
@@ -657,6 +658,7 @@ static int adj_forward(tdw_ctx *c, tdw_state *s, int it, tdw_complex *y_out, dou
                        tdw_tape_step *t)
 {
     TDW_TRY(fused_finalize(c, s));
+    if (resident_supported(c)) return resident_step(c, s, it, 0, t, y_out, cbuf, f_next);
     const int n = s->n;
     const AbmCoef cf = abm_coef(c->p.scheme);
     const int k = cf.h;
@@ -762,6 +764,7 @@ extern "C" int tdw_adj_history_entry(tdw_ctx *c, int it, const tdw_tape_step *t,
     if (!adj_supported(c)) return TDW_EINVAL;
     const int n = t->n;
     const double *e_c = t->scal + 3 * n;
+    if (resident_supported(c)) return resident_h(c, n, CD2(y1), D2(fnew), t->pots_c, nullptr, e_c);
     const bool plane = h2d_supported(c);
     const bool fused = !plane && fused_supported(c);
     if (plane) return apply_h_plane(c, it + 1, n, CD2(y1), D2(fnew), t->pots_c, c->d_kt, e_c, nullptr);

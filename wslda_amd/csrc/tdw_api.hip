@@ -7,6 +7,7 @@
 #include "tdw_internal.hpp"
 #include "tdw_physics.hpp"
 #include "tdw_fused.hpp"
+#include "tdw_resident.hpp"
 
 using namespace tdw;
 
@@ -202,6 +203,7 @@ extern "C" int tdw_create(const tdw_params *p, int nwf, int device, tdw_ctx **ou
         e = (int)hipMemcpy(c->d_cnt, ones, sizeof(int) * nwf, hipMemcpyHostToDevice);
         free(ones);
     }
+    if (!e) e = resident_setup(c);
     if (!e) e = project_attach(c);
     if (e) {
         tdw_destroy(c);
@@ -227,6 +229,7 @@ extern "C" int tdw_destroy(tdw_ctx *c)
         if (b) hipFree(b);
     project_release(c);
     fused_release(c);
+    resident_release(c);
     if (c->timers) {
         for (auto &r : *c->timers) { hipEventDestroy(r.a); hipEventDestroy(r.b); }
         delete c->timers;
@@ -504,6 +507,11 @@ extern "C" int tdw_step(tdw_ctx *c, tdw_state *s, int it, int grad_last)
         if (!s->ddx || (c->dim >= 2 && !s->ddy) || (c->dim >= 3 && !s->ddz)) return TDW_EINVAL;
         return step_aslda(c, s, it, k, qpe);
     }
+    // 1D and 2D lattices whose state fits in LDS run the resident step; lap is
+    // then written only by a gradient step.  In 3D this entry stays the kernel
+    // sequence that a caller of the separate entry points gets, to the bit;
+    // tdw_step_fused runs the resident step there.
+    if (c->dim < 3 && resident_supported(c)) return resident_step(c, s, it, grad_last);
     // 2D lattices with a one-pass plane kernel apply H with the Laplacian
     // formed in LDS on non-gradient half-steps (lap then holds H y_p, not the
     // Laplacian, after the step)

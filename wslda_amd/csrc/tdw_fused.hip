@@ -36,6 +36,7 @@
 #include "tdw_fused.hpp"
 #include "tdw_physics.hpp"
 #include "tdw_regfft.hpp"
+#include "tdw_resident.hpp"
 
 #include <algorithm>
 #include <type_traits>
@@ -1140,6 +1141,12 @@ int fused_adj_step(tdw_ctx *c, tdw_state *s, int it, tdw_complex *y_out, double2
 int fused_step(tdw_ctx *c, tdw_state *s, int it, int grad_last)
 {
     if (aslda_step_supported(c)) return aslda_fused_step(c, s, it, grad_last);
+    // FP64 states that fit in LDS: the resident step (15 S against 20 S, and
+    // half the launches), which leaves nothing pending
+    if (fused_supported(c) && resident_supported(c)) {
+        TDW_TRY(fused_finalize(c, s));
+        return resident_step(c, s, it, grad_last);
+    }
     if (!fused_supported(c)) {
         // the split form exists only as the fused step: its history arrays
         // hold FP32 values, which the FP64 step cannot continue from

@@ -10,6 +10,9 @@
 
 #define TDW_MAXST 8
 
+namespace tdw {
+struct RsPlan;
+}
 struct tdw_project;   // a project build's callback table (tdw_hooks.hpp)
 
 struct tdw_timer_rec {
@@ -58,6 +61,10 @@ struct tdw_ctx {
     double *d_sp, *d_s2, *d_ep;          // n: predictor scale, scale^2, predictor <H>
     double *d_fpart;  size_t fpart_cap;  // partial sums of the fused kernels
     int pending;                         // y and f[0] carry a pending scale / <H> fix-up
+    // resident-state step (tdw_resident.hip): plan and tables, null where a
+    // state does not fit in LDS
+    tdw::RsPlan *rplan;
+    void *d_rtab;
     // adjoint
     double *d_adjv;                      // 4n per-state scalars of the backward step
     // ASLDA (allocated on first use)

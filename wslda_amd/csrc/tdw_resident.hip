@@ -1,0 +1,510 @@
+// tdw_resident.hip -- the constant-mass PECE step of lattices whose whole
+// state (both components) fits in the LDS of one CU: one workgroup per state.
+//
+// With the state resident, everything between two density sums is one pass:
+//   rs_pred   predictor and partial corrector (tdwslda_ode_integrator.h:26-135)
+//             with the norm of y_p as a per-state factor: 8 S (AB5AM5);
+//   dens, potentials of the prediction (weights f s^2): 1 S;
+//   rs_h<1>   s y_p into LDS, its Laplacian in place (all axes), H psi and
+//             <H> (pca_kernels.cu:233-391, 806-832), the corrector
+//             (tdwslda_ode_integrator.h:138-220), its norm, the normalised y:
+//             3 S;
+//   dens, potentials of the corrected state: 1 S;
+//   rs_h<0>   H psi - <H> psi of it into the newest history slot: 2 S.
+// 15 S per state-step in nine launches.  The kernel-by-kernel step moves 31 S
+// (2D plane kernels) to 35 S in some twenty launches, the six-pass step of
+// tdw_fused.hip 20 S in sixteen.  Per step, before and after: 1D 64 points x
+// 128 states 87 -> 59 us, 36 x 18 x 300 190 -> 98 us, 64 x 64 x 1024 924 ->
+// 684 us, 12^3 x 1781 487 -> 400 us.
+//
+// Bounds: at 64 x 64 one 133 KB state fills a CU's LDS and its load, transform
+// and store phases follow one another (rs_h<1> 169 us for 3 S of 134 MB,
+// rs_h<0> 141 us for 2 S, against 292 and 169 us of the kernels they replace);
+// small lattices wait for launches, cold instruction fetches and the chain of
+// barriers of one state (15 us for up to 256 states of 36 x 18).
+#include "tdw_device.hpp"
+#include "tdw_fused.hpp"
+#include "tdw_internal.hpp"
+#include "tdw_physics.hpp"
+#include "tdw_regfft.hpp"
+#include "tdw_resident.hpp"
+
+#include <algorithm>
+#include <math.h>
+#include <vector>
+
+namespace tdw {
+
+// One radix-R stage of an axis: blocks of R * sub elements, tws = L / (R sub)
+// the step of its twiddles in the table of L.
+struct RsStage {
+    int R, sub, tws;
+    unsigned msub;   // division by sub
+};
+// An axis of the state in LDS.  Pencil q of P starts at q * qh (qd = 0) or at
+// (q / qd) * qh + q % qd; its elements lie `is` apart.
+struct RsAxis {
+    int L, nst, is, P, qd, qh, tw;
+    unsigned mP, mqd;
+    RsStage st[RS_MAXST];
+};
+struct RsPlan {
+    int dim, inner, npc, ll;      // points per x plane (padded), padded points per component, last axis length
+    unsigned mll;                 // division by the last axis length
+    RsAxis ax[3];
+};
+
+// x / d for the small operands here (x d < 2^32), m = floor(2^32 / d) + 1
+__device__ __forceinline__ unsigned rs_div(unsigned x, unsigned d, unsigned m) { return d == 1 ? x : __umulhi(x, m); }
+
+// Mixed-radix transforms in place.  Forward stages are decimation in
+// frequency: R elements sub apart, DFT, times W_{R sub}^{j t}; the inverse
+// stages undo them in reverse order, so the spectrum is used in the
+// digit-reversed order it is left in and nothing is reordered.
+// KIND 0: forward stage; 1: inverse stage; 2: the last forward stage of the
+// x axis, the factor -(k_x^2 + k_y^2 + k_z^2) / N and the first inverse stage
+// in registers.  Consecutive lanes take consecutive pencils.
+template <int R, int KIND>
+__device__ __forceinline__ void rs_stage(double2 *A, const double2 *tw, const RsAxis &ax, const RsStage &st,
+                                         const double *__restrict__ kx, const double *__restrict__ kin)
+{
+    const unsigned tot = ax.P * (ax.L / R);
+    for (unsigned b = threadIdx.x; b < tot; b += blockDim.x) {
+        const unsigned jj = rs_div(b, ax.P, ax.mP), q = b - jj * ax.P;
+        const unsigned blk = rs_div(jj, st.sub, st.msub), j = jj - blk * st.sub;
+        unsigned qi = q, base = q * ax.qh;
+        if (ax.qd) {
+            const unsigned hi = rs_div(q, ax.qd, ax.mqd);
+            qi = q - hi * ax.qd;
+            base = hi * ax.qh + qi;
+        }
+        const unsigned i0 = blk * (R * st.sub) + j, step = st.sub * ax.is;
+        double2 *p = A + base + i0 * ax.is;
+        double2 v[R];
+#pragma unroll
+        for (int t = 0; t < R; t++) v[t] = p[t * step];
+        if constexpr (KIND == 1) {
+            if (st.sub > 1) {
+#pragma unroll
+                for (int t = 1; t < R; t++) {
+                    const double2 w = tw[j * t * st.tws];
+                    v[t] = cmul(v[t], make_double2(w.x, -w.y));
+                }
+            }
+            rf::dft_inplace<R, +1, double2>(v);
+        } else {
+            rf::dft_inplace<R, -1, double2>(v);
+            if constexpr (KIND == 0) {
+                if (st.sub > 1) {
+#pragma unroll
+                    for (int t = 1; t < R; t++) v[t] = cmul(v[t], tw[j * t * st.tws]);
+                }
+            } else {
+                const double ki = kin[qi];
+#pragma unroll
+                for (int t = 0; t < R; t++) v[t] = v[t] * (kx[i0 + t] + ki);
+                rf::dft_inplace<R, +1, double2>(v);
+            }
+        }
+#pragma unroll
+        for (int t = 0; t < R; t++) p[t * step] = v[t];
+    }
+    __syncthreads();
+}
+
+template <int KIND>
+__device__ __forceinline__ void rs_run(double2 *A, const double2 *tw, const RsAxis &ax, int s,
+                                       const double *__restrict__ kx, const double *__restrict__ kin)
+{
+    const RsStage st = ax.st[s];
+    switch (st.R) {
+    case 2: rs_stage<2, KIND>(A, tw + ax.tw, ax, st, kx, kin); break;
+    case 3: rs_stage<3, KIND>(A, tw + ax.tw, ax, st, kx, kin); break;
+    case 4: rs_stage<4, KIND>(A, tw + ax.tw, ax, st, kx, kin); break;
+    case 6: rs_stage<6, KIND>(A, tw + ax.tw, ax, st, kx, kin); break;
+    case 8: rs_stage<8, KIND>(A, tw + ax.tw, ax, st, kx, kin); break;
+    case 9: rs_stage<9, KIND>(A, tw + ax.tw, ax, st, kx, kin); break;
+    default: rs_stage<12, KIND>(A, tw + ax.tw, ax, st, kx, kin); break;
+    }
+}
+
+// Laplacian of both components in LDS, in place
+__device__ __forceinline__ void rs_laplace(double2 *A, const double2 *tw, const RsPlan &pl,
+                                           const double *__restrict__ kx, const double *__restrict__ kin)
+{
+    for (int d = pl.dim - 1; d >= 0; d--) {
+        const int ns = d == 0 ? pl.ax[0].nst - 1 : pl.ax[d].nst;
+        for (int s = 0; s < ns; s++) rs_run<0>(A, tw, pl.ax[d], s, kx, kin);
+    }
+    rs_run<2>(A, tw, pl.ax[0], pl.ax[0].nst - 1, kx, kin);
+    for (int d = 0; d < pl.dim; d++) {
+        const int ns = d == 0 ? pl.ax[0].nst - 1 : pl.ax[d].nst;
+        for (int s = ns - 1; s >= 0; s--) rs_run<1>(A, tw, pl.ax[d], s, kx, kin);
+    }
+}
+
+// Predictor: y <- y_p (unnormalised), c <- the partial corrector, s = 1 /
+// sqrt(norm), s2 = s^2 per state; with nrm_out, the norm itself.  A state per
+// workgroup, so the norm needs no second launch.
+template <int SCH>
+__global__ void __launch_bounds__(RS_NT)
+rs_pred(const double2 *yin, double2 *y, double2 *c, const double2 *f1, const double2 *f2, const double2 *f3,
+        const double2 *f4, const double2 *f5, int n, int N, double dt, double dv, double *__restrict__ s_out,
+        double *__restrict__ s2_out, double *__restrict__ nrm_out)
+{
+    __shared__ double red[RS_NT / 64];
+    const int a = blockIdx.x;
+    double nrm = 0.0;
+    for (int i = threadIdx.x; i < N; i += blockDim.x) {
+        // both components' loads before the stores, which may alias them
+        const long idx[2] = {(long)a * N + i, ((long)n + a) * N + i};
+        double2 yk[2], F[2][5];
+#pragma unroll
+        for (int q = 0; q < 2; q++) {
+            yk[q] = yin[idx[q]];
+            F[q][0] = f1[idx[q]];
+            F[q][1] = f2[idx[q]];
+            F[q][2] = f3[idx[q]];
+            F[q][3] = SCH >= 45 ? f4[idx[q]] : make_double2(0.0, 0.0);
+            F[q][4] = SCH >= 55 ? f5[idx[q]] : make_double2(0.0, 0.0);
+        }
+#pragma unroll
+        for (int q = 0; q < 2; q++) {
+            double2 sp, sc;
+            abm_sums<SCH>(F[q][0], F[q][1], F[q][2], F[q][3], F[q][4], sp, sc);
+            const double2 yp = yk[q] + imul(sp, -dt);
+            y[idx[q]] = yp;
+            c[idx[q]] = yk[q] + imul(sc, -dt);
+            nrm += cnorm(yp);
+        }
+    }
+    nrm = block_sum(nrm, red) * dv;
+    if (threadIdx.x) return;
+    const double sc = 1.0 / sqrt(nrm);
+    s_out[a] = sc;
+    s2_out[a] = sc * sc;
+    if (nrm_out) nrm_out[a] = nrm;
+}
+
+struct RsH {
+    double mu_a, mu_b, dv, dta0;
+    int bdg;
+};
+
+// CORR 0: out = H psi - <H> psi, psi = in.
+// CORR 1: psi = s_a in (the normalised prediction), out = the normalised
+// corrected state of -i dt a0 (H psi - <H> psi) + c (out may be in: a state
+// is read whole before it is written).
+// <H> per state into e_out (and e_out2), or read from use_e; the corrected
+// state's norm into nrm_out where given.  H as in k_apply_h, with the transverse momenta of 1D
+// and 2D (kt, and kt2 in 1D) in the kinetic term.
+template <int CORR>
+__global__ void __launch_bounds__(RS_NT)
+rs_h(const double2 *in, double2 *out, const double2 *__restrict__ c, const double *__restrict__ pots,
+     const double *__restrict__ sc, const double *__restrict__ kt, const double *__restrict__ kt2, int n, int N,
+     RsPlan pl, RsH hp, const double2 *__restrict__ twg, int ntw, const double *__restrict__ kx,
+     const double *__restrict__ kin, const double *use_e, double *e_out, double *e_out2,
+     double *__restrict__ nrm_out)
+{
+    extern __shared__ double2 rs_sm[];
+    __shared__ double red[RS_NT / 64];
+    double2 *A = rs_sm, *tw = rs_sm + 2 * pl.npc;
+    const int a = blockIdx.x, tid = threadIdx.x, nt = blockDim.x;
+    const long gu = (long)a * N, gv = ((long)n + a) * N;
+    const double s = CORR ? sc[a] : 1.0;
+    for (int k = tid; k < ntw; k += nt) tw[k] = twg[k];
+    // point i of a component sits at i + i / ll: rows of the last axis, ll + 1 apart
+    const int pad = pl.dim > 1;
+    for (int i = tid; i < N; i += nt) {
+        const int pe = pad ? i + rs_div(i, pl.ll, pl.mll) : i;
+        A[pe] = in[gu + i] * s;
+        A[pl.npc + pe] = in[gv + i] * s;
+    }
+    __syncthreads();
+    rs_laplace(A, tw, pl, kx, kin);
+    double k2t = 0.0;
+    if (kt) k2t = kt[a] * kt[a];
+    if (kt2) k2t += kt2[a] * kt2[a];
+    // H psi over the Laplacian, <psi|H psi>
+    double e = 0.0;
+    for (int i = tid; i < N; i += nt) {
+        const int pe = pad ? i + rs_div(i, pl.ll, pl.mll) : i;
+        const double aa = hp.bdg ? -0.5 : pots[4 * N + i] * -0.5, ab = hp.bdg ? -0.5 : pots[5 * N + i] * -0.5;
+        const double Va = pots[i] - hp.mu_a - aa * k2t, Vb = pots[N + i] - hp.mu_b - ab * k2t;
+        const double2 D = make_double2(pots[2 * N + 2 * i], pots[2 * N + 2 * i + 1]);
+        const double2 tu = in[gu + i] * s, tv = in[gv + i] * s;
+        const double2 u = tu * Va + cmul(tv, D) + A[pe] * aa;
+        const double2 v = tv * (-Vb) + cmulc(D, tu) - A[pl.npc + pe] * ab;
+        A[pe] = u;
+        A[pl.npc + pe] = v;
+        e += cmulc(tu, u).x + cmulc(tv, v).x;
+    }
+    if (use_e) {
+        e = use_e[a];
+    } else {
+        e = block_sum(e, red) * hp.dv;
+        if (tid == 0) {
+            e_out[a] = e;
+            if (e_out2) e_out2[a] = e;
+        }
+    }
+    double nrm = 0.0;
+    for (int i = tid; i < N; i += nt) {
+        const int pe = pad ? i + rs_div(i, pl.ll, pl.mll) : i;
+        const double2 u = A[pe] - in[gu + i] * s * e, v = A[pl.npc + pe] - in[gv + i] * s * e;
+        if constexpr (CORR) {
+            const double2 yu = imul(u, -hp.dta0) + c[gu + i], yv = imul(v, -hp.dta0) + c[gv + i];
+            A[pe] = yu;
+            A[pl.npc + pe] = yv;
+            nrm += cnorm(yu) + cnorm(yv);
+        } else {
+            out[gu + i] = u;
+            out[gv + i] = v;
+        }
+    }
+    if constexpr (CORR) {
+        nrm = block_sum(nrm, red) * hp.dv;
+        const double r = 1.0 / sqrt(nrm);
+        if (tid == 0 && nrm_out) nrm_out[a] = nrm;
+        for (int i = tid; i < N; i += nt) {
+            const int pe = pad ? i + rs_div(i, pl.ll, pl.mll) : i;
+            out[gu + i] = A[pe] * r;
+            out[gv + i] = A[pl.npc + pe] * r;
+        }
+    }
+}
+
+// ---------------------------------------------------------------------------
+// host side
+// ---------------------------------------------------------------------------
+static unsigned magic(int d) { return d > 1 ? (unsigned)((1ull << 32) / (unsigned)d) + 1u : 0u; }
+
+// The radices of an axis: the fewest stages, then the smallest largest radix
+// (registers: the 12 values of a stage are 48 of the 128 that 1024 threads
+// leave).  -1: the length has another prime factor, or too many.
+static bool rs_split(int rem, int m, int top, int *R)
+{
+    if (m == 0) return rem == 1;
+    for (int q : {12, 9, 8, 6, 4, 3, 2})
+        if (q <= top && rem % q == 0) {
+            R[0] = q;
+            if (rs_split(rem / q, m - 1, top, R + 1)) return true;
+        }
+    return false;
+}
+static int rs_radices(int L, int *R)
+{
+    for (int m = 0; m <= RS_MAXST; m++)
+        for (int top : {2, 3, 4, 6, 8, 9, 12})
+            if (rs_split(L, m, top, R)) return m;
+    return -1;
+}
+
+static size_t rs_lds(const RsPlan &pl, int ntw) { return sizeof(double2) * (2 * (size_t)pl.npc + ntw); }
+
+int resident_setup(tdw_ctx *c)
+{
+    const int len[3] = {c->nx, c->ny, c->nz};
+    const int dim = c->dim, ll = len[dim - 1], row = dim > 1 ? ll + 1 : 1;
+    RsPlan pl;
+    pl.dim = dim;
+    pl.ll = ll;
+    pl.mll = magic(ll);
+    const size_t npc = dim == 1 ? (size_t)c->nx : c->N / ll * row;
+    const int ntw = len[0] + (dim > 1 ? len[1] : 0) + (dim > 2 ? len[2] : 0);
+    // the state, the twiddles and the static reduction slots within a CU's LDS
+    if (sizeof(double2) * (2 * npc + ntw) + 1024 > (size_t)c->max_lds) return 0;
+    pl.npc = (int)npc;
+    pl.inner = (int)(npc / c->nx);
+    std::vector<double2> tw;
+    std::vector<double> kk[3];
+    int t0 = 0;
+    for (int d = 0; d < dim; d++) {
+        RsAxis &ax = pl.ax[d];
+        const int L = len[d];
+        int R[RS_MAXST];
+        ax.L = L;
+        ax.nst = rs_radices(L, R);
+        if (ax.nst < 0 || (d == 0 && ax.nst < 1)) return 0;
+        ax.tw = t0;
+        t0 += L;
+        if (d == 0) {
+            ax.is = pl.inner;
+            ax.P = 2 * pl.inner;
+            ax.qd = pl.inner;
+            ax.qh = pl.npc;
+        } else if (d == dim - 1) {
+            ax.is = 1;
+            ax.P = 2 * (pl.npc / row);
+            ax.qd = 0;
+            ax.qh = row;
+        } else {
+            ax.is = row;
+            ax.P = 2 * c->nx * row;
+            ax.qd = row;
+            ax.qh = c->ny * row;
+        }
+        ax.mP = magic(ax.P);
+        ax.mqd = magic(ax.qd);
+        int sub = L, mul = 1;
+        for (int s = 0; s < ax.nst; s++) {
+            RsStage &st = ax.st[s];
+            st.tws = mul;
+            sub /= R[s];
+            mul *= R[s];
+            st.R = R[s];
+            st.sub = sub;
+            st.msub = magic(sub);
+        }
+        // -k^2 / N at each position of the digit-reversed spectrum
+        kk[d].resize(L);
+        for (int p = 0; p < L; p++) {
+            int f = 0, w = 1, rem = p, blk = L;
+            for (int s = 0; s < ax.nst; s++) {
+                blk /= R[s];
+                f += w * (rem / blk);
+                rem %= blk;
+                w *= R[s];
+            }
+            const double k = 2. * M_PI / c->Lphys[d] * (double)(f < L / 2 ? f : f - L);
+            kk[d][p] = -(k * k) / (double)c->N;
+        }
+        for (int t = 0; t < L; t++) {
+            const double an = 2.0 * M_PI * (double)t / (double)L;
+            tw.push_back(make_double2(cos(an), -sin(an)));
+        }
+    }
+    // tables: twiddles of all axes, then k_x^2, then the rest per point of an
+    // x plane (pads included)
+    std::vector<double> kt(kk[0]);
+    for (int i = 0; i < pl.inner; i++) {
+        const int z = i % row, y = i / row;
+        double v = 0.0;
+        if (dim == 2 && z < ll) v = kk[1][z];
+        if (dim == 3 && z < ll) v = kk[1][y] + kk[2][z];
+        kt.push_back(v);
+    }
+    const size_t btw = sizeof(double2) * tw.size(), bk = sizeof(double) * kt.size();
+    TDW_HIP(hipMalloc(&c->d_rtab, btw + bk));
+    TDW_HIP(hipMemcpy(c->d_rtab, tw.data(), btw, hipMemcpyHostToDevice));
+    TDW_HIP(hipMemcpy((char *)c->d_rtab + btw, kt.data(), bk, hipMemcpyHostToDevice));
+    c->rplan = new RsPlan(pl);
+    return 0;
+}
+
+void resident_release(tdw_ctx *c)
+{
+    if (c->d_rtab) hipFree(c->d_rtab);
+    c->d_rtab = nullptr;
+    delete c->rplan;
+    c->rplan = nullptr;
+}
+
+bool resident_supported(const tdw_ctx *c)
+{
+    return c->rplan && !varying_mass(c) && c->p.precision == TDW_FP64;
+}
+
+// Threads of a workgroup: 16 waves per CU (four per SIMD, what 103 VGPRs of
+// rs_h leave) over the workgroups that share it, as many as the LDS holds or
+// as the states give; a whole number of waves, no more than one point per
+// thread.  With 20 waves a second workgroup did not fit beside the first: 300
+// states of 36 x 18 took 26 us against 15 for 128.
+static int rs_threads(size_t lds, int n, int N)
+{
+    const int fit = lds ? (int)std::max<size_t>(1, (160 * 1024) / (lds + 256)) : 8;
+    const int wg = std::min(std::min(fit, 16), std::max(1, (n + 255) / 256));
+    const int nt = 64 * std::max(1, 16 / wg);
+    return std::min(nt, (N + 63) / 64 * 64);
+}
+
+template <int CORR>
+static int launch_h(tdw_ctx *c, int n, const double2 *in, double2 *out, const double2 *cc, const double *pots,
+                    const double *sc, const double *use_e, double *e_out, double *e_out2, double *nrm_out)
+{
+    const RsPlan &pl = *c->rplan;
+    const int N = (int)c->N, ntw = pl.ax[0].L + (pl.dim > 1 ? pl.ax[1].L : 0) + (pl.dim > 2 ? pl.ax[2].L : 0);
+    const double2 *tw = (const double2 *)c->d_rtab;
+    const double *kx = (const double *)(tw + ntw);
+    const double a0 = (c->p.scheme == TDW_AB3AM4) ? 9. / 24. : 251. / 720.;
+    const RsH hp{c->p.mu_a, c->p.mu_b, dvol_norm(c), c->p.dt * a0, c->p.functional == TDW_BDG};
+    const size_t lds = rs_lds(pl, ntw);
+    const double *kt = c->dim < 3 ? c->d_kt : nullptr, *kt2 = c->dim == 1 ? c->d_kt + n : nullptr;
+    TDW_TIMED(c, CORR ? "rs_hcorr" : "rs_h");
+    hipLaunchKernelGGL(rs_h<CORR>, dim3(n), dim3(rs_threads(lds, n, N)), lds, c->stream, in, out, cc, pots, sc, kt, kt2,
+                       n, N, pl, hp, tw, ntw, kx, kx + pl.ax[0].L, use_e, e_out, e_out2, nrm_out);
+    return (int)hipGetLastError();
+}
+
+int resident_h(tdw_ctx *c, int n, const double2 *in, double2 *out, const double *pots, double *qpe,
+               const double *use_e)
+{
+    return launch_h<0>(c, n, in, out, nullptr, pots, nullptr, use_e, qpe, nullptr, nullptr);
+}
+
+static int tape_copy(tdw_ctx *c, const double *src, double *dst, long nd)
+{
+    return (int)hipMemcpyAsync(dst, src, sizeof(double) * nd, hipMemcpyDeviceToDevice, c->stream);
+}
+
+int resident_step(tdw_ctx *c, tdw_state *s, int it, int grad_last, tdw_tape_step *tape, tdw_complex *y_out,
+                  double2 *cbuf, tdw_complex *f_next)
+{
+    const int n = s->n, N = (int)c->N;
+    const int h = c->p.scheme == TDW_AB3AM4 ? 3 : c->p.scheme == TDW_AB4AM5 ? 4 : 5;
+    TDW_TRY(fused_state_vecs(c));
+    double *qpe = s->qpe ? s->qpe : c->d_qpe;
+    const double2 *y0 = (const double2 *)s->wf, *f[5];
+    for (int j = 0; j < 5; j++) f[j] = (const double2 *)s->f[j];
+    double2 *y = y_out ? (double2 *)y_out : (double2 *)s->wf;
+    double2 *cc = cbuf ? cbuf : (double2 *)s->f[h - 1];
+    const double dv = dvol_norm(c);
+    {
+        TDW_TIMED(c, "rs_pred");
+        const int nt = rs_threads(0, n, N);
+        double *nrm = tape ? tape->scal : nullptr;
+#define RS_PRED(S)                                                                                                       hipLaunchKernelGGL(rs_pred<S>, dim3(n), dim3(nt), 0, c->stream, y0, y, cc, f[0], f[1], f[2], f[3], f[4], n, N,                        c->p.dt, dv, c->d_sp, c->d_s2, nrm)
+        if (h == 3) RS_PRED(34);
+        else if (h == 4) RS_PRED(45);
+        else RS_PRED(55);
+#undef RS_PRED
+        TDW_HIP(hipGetLastError());
+    }
+    if (y_out) s->wf = y_out;
+    TDW_TRY(densities(c, n, y, nullptr, nullptr, nullptr, nullptr, c->d_fbeta, c->d_s2, c->d_kt, c->d_cnt, s->dens, 0));
+    if (tape) TDW_TRY(tape_copy(c, s->dens, tape->dens_p, 12L * N));
+    TDW_TRY(step_potentials(c, it + 1, s->dens, s->pots));
+    TDW_TRY(hkf_fields(c, s->pots, true));
+    if (tape) TDW_TRY(tape_copy(c, s->pots, tape->pots_p, 12L * N));
+    const double *hp = h_view(c, it + 1, s->pots);
+    if (!hp) return TDW_EINVAL;
+    TDW_TRY(launch_h<1>(c, n, y, y, cc, hp, c->d_sp, nullptr, qpe, tape ? tape->scal + n : nullptr,
+                        tape ? tape->scal + 2 * n : nullptr));
+    // the corrected state: densities (a measurement step's with gradients,
+    // tau and j), potentials, the new history entry
+    if (grad_last && dens_grad_fused_supported(c)) {
+        // 3D lattices with the in-pass gradient densities (as the six-pass
+        // step does it: no derivative array is stored)
+        TDW_TRY(dens_grad_fused(c, n, y, c->d_fbeta, nullptr, s->dens));
+    } else {
+        if (grad_last)
+            TDW_TRY(derivatives(c, 2 * n, y, (double2 *)s->ddx, (double2 *)s->ddy, (double2 *)s->ddz,
+                                (double2 *)s->lap));
+        TDW_TRY(densities(c, n, y, (double2 *)s->ddx, (double2 *)s->ddy, (double2 *)s->ddz, (double2 *)s->lap,
+                          c->d_fbeta, nullptr, c->d_kt, c->d_cnt, s->dens, grad_last));
+    }
+    if (grad_last) TDW_TRY(density_tau(c, s->dens));
+    if (tape) TDW_TRY(tape_copy(c, s->dens, tape->dens_c, 12L * N));
+    TDW_TRY(step_potentials(c, it + 1, s->dens, s->pots));
+    TDW_TRY(hkf_fields(c, s->pots, true));
+    if (tape) TDW_TRY(tape_copy(c, s->pots, tape->pots_c, 12L * N));
+    hp = h_view(c, it + 1, s->pots);
+    if (!hp) return TDW_EINVAL;
+    tdw_complex *tmp = f_next ? f_next : s->f[h - 1];
+    for (int j = h - 1; j > 0; j--) s->f[j] = s->f[j - 1];
+    s->f[0] = tmp;
+    return launch_h<0>(c, n, y, (double2 *)s->f[0], nullptr, hp, nullptr, nullptr, qpe,
+                       tape ? tape->scal + 3 * n : nullptr, nullptr);
+}
+
+}  // namespace tdw

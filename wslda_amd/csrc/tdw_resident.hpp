@@ -1,0 +1,29 @@
+// tdw_resident.hpp -- the PECE step of lattices whose whole state fits in LDS.
+#pragma once
+#include "tdw_internal.hpp"
+
+namespace tdw {
+
+static constexpr int RS_MAXST = 6;    // stages per axis
+static constexpr int RS_NT = 1024;    // most threads per workgroup
+
+struct RsPlan;
+
+// plan and tables of the context's lattice (tdw_create); none where a state
+// does not fit, and no error then
+int resident_setup(tdw_ctx *c);
+void resident_release(tdw_ctx *c);
+// constant-mass H in FP64 on a lattice with a plan
+bool resident_supported(const tdw_ctx *c);
+// The step of tdw_step (same arrays, complete at its end; lap is not
+// written by a step without gradients).  The adjoint's taped step is the
+// same with tape: y to y_out (NULL: in place), the partial corrector to cbuf
+// (NULL: the oldest history entry), the new entry to f_next (NULL: the
+// dropped oldest entry).
+int resident_step(tdw_ctx *c, tdw_state *s, int it, int grad_last, tdw_tape_step *tape = nullptr,
+                  tdw_complex *y_out = nullptr, double2 *cbuf = nullptr, tdw_complex *f_next = nullptr);
+// out = H in - e in with <H> of in into qpe, or with use_e the given e (qpe
+// is then not written)
+int resident_h(tdw_ctx *c, int n, const double2 *in, double2 *out, const double *pots, double *qpe,
+               const double *use_e = nullptr);
+}  // namespace tdw
