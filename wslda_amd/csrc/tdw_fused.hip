@@ -124,6 +124,15 @@ __device__ __forceinline__ double xkin_energy(C (&r)[LX], double sig_kscale_half
 // by Parseval, unscaled by the state's normalisation (xpart, laid out as the
 // norm partials).
 // ---------------------------------------------------------------------------
+// Whether the predictor holds its lane's pencil of y in registers between the
+// transform and the update: up to 24 points fit beside the streams at two
+// waves per SIMD (240 VGPRs).  What is read again misses the L2 (every byte,
+// by the counters), while the third wave of 150 VGPRs only adds loads in
+// flight that the streams do not need.  24^3 x 4096: FP64 3.33 ms (10 S) ->
+// 3.13 ms (9 S), split 2.01 -> 1.94 ms.  At 32 points half a pencil fits and
+// gains nothing (1.77 -> 1.76 ms), so it is read twice there.
+template <int LX> constexpr bool pred_hold() { return LX <= 24; }
+
 template <int LX, int SCH, bool SP>
 __global__ void __launch_bounds__(FT)
 f_pred(double2 *__restrict__ y, hc_t<SP> *f1, const hc_t<SP> *f2, const hc_t<SP> *f3, const hc_t<SP> *f4,
@@ -144,10 +153,15 @@ f_pred(double2 *__restrict__ y, hc_t<SP> *f1, const hc_t<SP> *f2, const hc_t<SP>
         const double skh = (a2 < n ? 0.5 : -0.5) * kscale;
         const long base = a2 * N + j;
         HC r[LX];
-        if (pending) {
-            // the pencil of y (read again in the loop below, from cache)
+        constexpr bool HOLD = pred_hold<LX>();
+        double2 yh[HOLD ? LX : 1];
+        if constexpr (HOLD) {
 #pragma unroll
-            for (int i = 0; i < LX; i++) r[i] = cvt<HC>(y[base + (long)i * S]);
+            for (int i = 0; i < LX; i++) yh[i] = y[base + (long)i * S];
+        }
+        if (pending) {
+#pragma unroll
+            for (int i = 0; i < LX; i++) r[i] = cvt<HC>(HOLD ? yh[HOLD ? i : 0] : y[base + (long)i * S]);
             xkin_inplace<LX>(r, skh, 0.0);
             __builtin_amdgcn_sched_barrier(0);
         }
@@ -158,7 +172,7 @@ f_pred(double2 *__restrict__ y, hc_t<SP> *f1, const hc_t<SP> *f2, const hc_t<SP>
 #pragma unroll
         for (int i = 0; i < LX; i++) {
             const long idx = lb + (long)i * ls;
-            const double2 yk = y[idx] * s;
+            const double2 yk = (HOLD ? yh[HOLD ? i : 0] : y[idx]) * s;
             double2 F1 = to64(f1[idx]);
             if (pending) {
                 F1 = F1 + to64(r[i]) * s - yk * e;

@@ -26,8 +26,8 @@
 #include "tdw_fused.hpp"
 #include "tdw_internal.hpp"
 #include "tdw_physics.hpp"
-#include "tdw_regfft.hpp"
 #include "tdw_resident.hpp"
+#include "tdw_rsfft.hpp"
 
 #include <algorithm>
 #include <math.h>
@@ -35,112 +35,21 @@
 
 namespace tdw {
 
-// One radix-R stage of an axis: blocks of R * sub elements, tws = L / (R sub)
-// the step of its twiddles in the table of L.
-struct RsStage {
-    int R, sub, tws;
-    unsigned msub;   // division by sub
-};
-// An axis of the state in LDS.  Pencil q of P starts at q * qh (qd = 0) or at
-// (q / qd) * qh + q % qd; its elements lie `is` apart.
-struct RsAxis {
-    int L, nst, is, P, qd, qh, tw;
-    unsigned mP, mqd;
-    RsStage st[RS_MAXST];
-};
 struct RsPlan {
     int dim, inner, npc, ll;      // points per x plane (padded), padded points per component, last axis length
     unsigned mll;                 // division by the last axis length
     RsAxis ax[3];
 };
 
-// x / d for the small operands here (x d < 2^32), m = floor(2^32 / d) + 1
-__device__ __forceinline__ unsigned rs_div(unsigned x, unsigned d, unsigned m) { return d == 1 ? x : __umulhi(x, m); }
-
-// Mixed-radix transforms in place.  Forward stages are decimation in
-// frequency: R elements sub apart, DFT, times W_{R sub}^{j t}; the inverse
-// stages undo them in reverse order, so the spectrum is used in the
-// digit-reversed order it is left in and nothing is reordered.
-// KIND 0: forward stage; 1: inverse stage; 2: the last forward stage of the
-// x axis, the factor -(k_x^2 + k_y^2 + k_z^2) / N and the first inverse stage
-// in registers.  Consecutive lanes take consecutive pencils.
-template <int R, int KIND>
-__device__ __forceinline__ void rs_stage(double2 *A, const double2 *tw, const RsAxis &ax, const RsStage &st,
-                                         const double *__restrict__ kx, const double *__restrict__ kin)
-{
-    const unsigned tot = ax.P * (ax.L / R);
-    for (unsigned b = threadIdx.x; b < tot; b += blockDim.x) {
-        const unsigned jj = rs_div(b, ax.P, ax.mP), q = b - jj * ax.P;
-        const unsigned blk = rs_div(jj, st.sub, st.msub), j = jj - blk * st.sub;
-        unsigned qi = q, base = q * ax.qh;
-        if (ax.qd) {
-            const unsigned hi = rs_div(q, ax.qd, ax.mqd);
-            qi = q - hi * ax.qd;
-            base = hi * ax.qh + qi;
-        }
-        const unsigned i0 = blk * (R * st.sub) + j, step = st.sub * ax.is;
-        double2 *p = A + base + i0 * ax.is;
-        double2 v[R];
-#pragma unroll
-        for (int t = 0; t < R; t++) v[t] = p[t * step];
-        if constexpr (KIND == 1) {
-            if (st.sub > 1) {
-#pragma unroll
-                for (int t = 1; t < R; t++) {
-                    const double2 w = tw[j * t * st.tws];
-                    v[t] = cmul(v[t], make_double2(w.x, -w.y));
-                }
-            }
-            rf::dft_inplace<R, +1, double2>(v);
-        } else {
-            rf::dft_inplace<R, -1, double2>(v);
-            if constexpr (KIND == 0) {
-                if (st.sub > 1) {
-#pragma unroll
-                    for (int t = 1; t < R; t++) v[t] = cmul(v[t], tw[j * t * st.tws]);
-                }
-            } else {
-                const double ki = kin[qi];
-#pragma unroll
-                for (int t = 0; t < R; t++) v[t] = v[t] * (kx[i0 + t] + ki);
-                rf::dft_inplace<R, +1, double2>(v);
-            }
-        }
-#pragma unroll
-        for (int t = 0; t < R; t++) p[t * step] = v[t];
-    }
-    __syncthreads();
-}
-
-template <int KIND>
-__device__ __forceinline__ void rs_run(double2 *A, const double2 *tw, const RsAxis &ax, int s,
-                                       const double *__restrict__ kx, const double *__restrict__ kin)
-{
-    const RsStage st = ax.st[s];
-    switch (st.R) {
-    case 2: rs_stage<2, KIND>(A, tw + ax.tw, ax, st, kx, kin); break;
-    case 3: rs_stage<3, KIND>(A, tw + ax.tw, ax, st, kx, kin); break;
-    case 4: rs_stage<4, KIND>(A, tw + ax.tw, ax, st, kx, kin); break;
-    case 6: rs_stage<6, KIND>(A, tw + ax.tw, ax, st, kx, kin); break;
-    case 8: rs_stage<8, KIND>(A, tw + ax.tw, ax, st, kx, kin); break;
-    case 9: rs_stage<9, KIND>(A, tw + ax.tw, ax, st, kx, kin); break;
-    default: rs_stage<12, KIND>(A, tw + ax.tw, ax, st, kx, kin); break;
-    }
-}
-
-// Laplacian of both components in LDS, in place
+// Laplacian of both components in LDS, in place: the factor
+// -(k_x^2 + k_y^2 + k_z^2) / N on the spectrum, kx its x part per position of
+// the x axis, kin the rest per point of an x plane
 __device__ __forceinline__ void rs_laplace(double2 *A, const double2 *tw, const RsPlan &pl,
                                            const double *__restrict__ kx, const double *__restrict__ kin)
 {
-    for (int d = pl.dim - 1; d >= 0; d--) {
-        const int ns = d == 0 ? pl.ax[0].nst - 1 : pl.ax[d].nst;
-        for (int s = 0; s < ns; s++) rs_run<0>(A, tw, pl.ax[d], s, kx, kin);
-    }
-    rs_run<2>(A, tw, pl.ax[0], pl.ax[0].nst - 1, kx, kin);
-    for (int d = 0; d < pl.dim; d++) {
-        const int ns = d == 0 ? pl.ax[0].nst - 1 : pl.ax[d].nst;
-        for (int s = ns - 1; s >= 0; s--) rs_run<1>(A, tw, pl.ax[d], s, kx, kin);
-    }
+    for (int d = pl.dim - 1; d > 0; d--) rs_forward(A, tw, pl.ax[d]);
+    rs_filter(A, tw, pl.ax[0], [&](unsigned i, unsigned q, double2 &v) { v = v * (kx[i] + kin[q]); });
+    for (int d = 1; d < pl.dim; d++) rs_inverse(A, tw, pl.ax[d]);
 }
 
 // Predictor: y <- y_p (unnormalised), c <- the partial corrector, s = 1 /
@@ -277,29 +186,6 @@ rs_h(const double2 *in, double2 *out, const double2 *__restrict__ c, const doubl
 // ---------------------------------------------------------------------------
 // host side
 // ---------------------------------------------------------------------------
-static unsigned magic(int d) { return d > 1 ? (unsigned)((1ull << 32) / (unsigned)d) + 1u : 0u; }
-
-// The radices of an axis: the fewest stages, then the smallest largest radix
-// (registers: the 12 values of a stage are 48 of the 128 that 1024 threads
-// leave).  -1: the length has another prime factor, or too many.
-static bool rs_split(int rem, int m, int top, int *R)
-{
-    if (m == 0) return rem == 1;
-    for (int q : {12, 9, 8, 6, 4, 3, 2})
-        if (q <= top && rem % q == 0) {
-            R[0] = q;
-            if (rs_split(rem / q, m - 1, top, R + 1)) return true;
-        }
-    return false;
-}
-static int rs_radices(int L, int *R)
-{
-    for (int m = 0; m <= RS_MAXST; m++)
-        for (int top : {2, 3, 4, 6, 8, 9, 12})
-            if (rs_split(L, m, top, R)) return m;
-    return -1;
-}
-
 static size_t rs_lds(const RsPlan &pl, int ntw) { return sizeof(double2) * (2 * (size_t)pl.npc + ntw); }
 
 int resident_setup(tdw_ctx *c)
@@ -309,7 +195,7 @@ int resident_setup(tdw_ctx *c)
     RsPlan pl;
     pl.dim = dim;
     pl.ll = ll;
-    pl.mll = magic(ll);
+    pl.mll = rs_magic(ll);
     const size_t npc = dim == 1 ? (size_t)c->nx : c->N / ll * row;
     const int ntw = len[0] + (dim > 1 ? len[1] : 0) + (dim > 2 ? len[2] : 0);
     // the state, the twiddles and the static reduction slots within a CU's LDS
@@ -322,52 +208,16 @@ int resident_setup(tdw_ctx *c)
     for (int d = 0; d < dim; d++) {
         RsAxis &ax = pl.ax[d];
         const int L = len[d];
-        int R[RS_MAXST];
-        ax.L = L;
-        ax.nst = rs_radices(L, R);
-        if (ax.nst < 0 || (d == 0 && ax.nst < 1)) return 0;
-        ax.tw = t0;
+        bool ok;
+        if (d == 0) ok = rs_axis(ax, L, pl.inner, 2 * pl.inner, pl.inner, pl.npc, t0);
+        else if (d == dim - 1) ok = rs_axis(ax, L, 1, 2 * (pl.npc / row), 0, row, t0);
+        else ok = rs_axis(ax, L, row, 2 * c->nx * row, row, c->ny * row, t0);
+        if (!ok || (d == 0 && ax.nst < 1)) return 0;
         t0 += L;
-        if (d == 0) {
-            ax.is = pl.inner;
-            ax.P = 2 * pl.inner;
-            ax.qd = pl.inner;
-            ax.qh = pl.npc;
-        } else if (d == dim - 1) {
-            ax.is = 1;
-            ax.P = 2 * (pl.npc / row);
-            ax.qd = 0;
-            ax.qh = row;
-        } else {
-            ax.is = row;
-            ax.P = 2 * c->nx * row;
-            ax.qd = row;
-            ax.qh = c->ny * row;
-        }
-        ax.mP = magic(ax.P);
-        ax.mqd = magic(ax.qd);
-        int sub = L, mul = 1;
-        for (int s = 0; s < ax.nst; s++) {
-            RsStage &st = ax.st[s];
-            st.tws = mul;
-            sub /= R[s];
-            mul *= R[s];
-            st.R = R[s];
-            st.sub = sub;
-            st.msub = magic(sub);
-        }
-        // -k^2 / N at each position of the digit-reversed spectrum
-        kk[d].resize(L);
-        for (int p = 0; p < L; p++) {
-            int f = 0, w = 1, rem = p, blk = L;
-            for (int s = 0; s < ax.nst; s++) {
-                blk /= R[s];
-                f += w * (rem / blk);
-                rem %= blk;
-                w *= R[s];
-            }
-            const double k = 2. * M_PI / c->Lphys[d] * (double)(f < L / 2 ? f : f - L);
-            kk[d][p] = -(k * k) / (double)c->N;
+        // -k^2 / N at each position of the spectrum
+        for (int f : rs_order(ax)) {
+            const double k = rs_k(f, L, c->Lphys[d]);
+            kk[d].push_back(-(k * k) / (double)c->N);
         }
         for (int t = 0; t < L; t++) {
             const double an = 2.0 * M_PI * (double)t / (double)L;

@@ -4,7 +4,6 @@
 
 namespace tdw {
 
-static constexpr int RS_MAXST = 6;    // stages per axis
 static constexpr int RS_NT = 1024;    // most threads per workgroup
 
 struct RsPlan;
