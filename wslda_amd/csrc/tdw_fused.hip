@@ -131,10 +131,14 @@ __device__ __forceinline__ double xkin_energy(C (&r)[LX], double sig_kscale_half
 // flight that the streams do not need.  24^3 x 4096: FP64 3.33 ms (10 S) ->
 // 3.13 ms (9 S), split 2.01 -> 1.94 ms.  At 32 points half a pencil fits and
 // gains nothing (1.77 -> 1.76 ms), so it is read twice there.
+// waves per SIMD asked for: pencils of 36 and 48 points would take a few
+// registers more than the 256 that leave two
+constexpr int x_waves(int LX) { return LX >= 36 ? 2 : 1; }
+
 template <int LX> constexpr bool pred_hold() { return LX <= 24; }
 
 template <int LX, int SCH, bool SP>
-__global__ void __launch_bounds__(FT)
+__global__ void __launch_bounds__(FT, x_waves(LX))
 f_pred(double2 *__restrict__ y, hc_t<SP> *f1, const hc_t<SP> *f2, const hc_t<SP> *f3, const hc_t<SP> *f4,
        const hc_t<SP> *f5, hc_t<SP> *fold, double *__restrict__ xpart,
        const double *__restrict__ sk, const double *__restrict__ ek, int pending, int n, long N, int S, double dt,
@@ -216,7 +220,7 @@ f_pred(double2 *__restrict__ y, hc_t<SP> *f1, const hc_t<SP> *f2, const hc_t<SP>
 // entry).
 // ---------------------------------------------------------------------------
 template <int LX, bool SP>
-__global__ void __launch_bounds__(FT)
+__global__ void __launch_bounds__(FT, x_waves(LX))
 f_corr(double2 *__restrict__ y, const hc_t<SP> *hin, const hc_t<SP> *__restrict__ cin,
        double *__restrict__ xpart, const double *__restrict__ sp_, const double *__restrict__ ep_, int n, long N,
        int S, double dta0, double kscale, int wave, double *__restrict__ part, float2 *y32)
@@ -547,8 +551,9 @@ f_hyz_big(const hc_t<SP> *__restrict__ y, const hc_t<SP> *__restrict__ T, hc_t<S
     typedef hc_t<SP> C;
     constexpr int E = LY * LZ;              // points of one plane
     constexpr int EP = LY * (LZ + 1);       // one component's plane in LDS, row stride LZ + 1
-    constexpr int KM = E / NT;              // owned points per thread
-    static_assert(E % NT == 0 && (NC == 1 || NC == 2), "plane split");
+    constexpr int KM = (E + NT - 1) / NT;   // owned points per thread
+    constexpr bool FULL = E % NT == 0;
+    static_assert(NC == 1 || NC == 2, "plane split");
     __shared__ C twy[LY], twz[LZ];
     __shared__ double zt[LZ];
     __shared__ double red[NT / 64];
@@ -574,6 +579,7 @@ f_hyz_big(const hc_t<SP> *__restrict__ y, const hc_t<SP> *__restrict__ T, hc_t<S
 #pragma unroll
     for (int k = 0; k < KM; k++) {
         const int e = tid + k * NT;
+        if (!FULL && e >= E) continue;
         Xu[k] = yu[e];
         Xv[k] = yv[e];
     }
@@ -585,6 +591,7 @@ f_hyz_big(const hc_t<SP> *__restrict__ y, const hc_t<SP> *__restrict__ T, hc_t<S
 #pragma unroll
         for (int k = 0; k < KM; k++) {
             const int e = tid + k * NT;
+            if (!FULL && e >= E) continue;
             const int pe = (e / LZ) * (LZ + 1) + e % LZ;
             if constexpr (NC == 2) {
                 A[pe] = Xu[k];
@@ -604,6 +611,7 @@ f_hyz_big(const hc_t<SP> *__restrict__ y, const hc_t<SP> *__restrict__ T, hc_t<S
 #pragma unroll
         for (int k = 0; k < KM; k++) {
             const int e = tid + k * NT;
+            if (!FULL && e >= E) continue;
             const int pe = (e / LZ) * (LZ + 1) + e % LZ;
             const double2 pu = to64(Xu[k]) * s, pv = to64(Xv[k]) * s;
             const double2 D = make_double2(Db[2 * e], Db[2 * e + 1]);
@@ -695,7 +703,7 @@ f_fixup(double2 *__restrict__ y, hc_t<SP> *__restrict__ f0, const double *__rest
 // and the newest history entry completed, f0 += s sigma (-1/2 D_x) y - e y_k
 // (x-pencils, as the predictor does it)
 template <int LX, bool SP>
-__global__ void __launch_bounds__(FT)
+__global__ void __launch_bounds__(FT, x_waves(LX))
 f_fixup_x(double2 *__restrict__ y, hc_t<SP> *__restrict__ f0, const double *__restrict__ sk,
           const double *__restrict__ ek, int n, long N, int S, double kscale)
 {
@@ -710,12 +718,19 @@ f_fixup_x(double2 *__restrict__ y, hc_t<SP> *__restrict__ f0, const double *__re
 #pragma unroll
     for (int i = 0; i < LX; i++) r[i] = cvt<HC>(y[base + (long)i * S]);
     xkin_inplace<LX>(r, (a2 < n ? 0.5 : -0.5) * kscale, 0.0);
+    // as in the corrector: loads kept out of the transforms, addresses formed
+    // here (registers)
+    __builtin_amdgcn_sched_barrier(0);
+    long lb = base;
+    int ls = S;
+    asm volatile("" : "+v"(lb), "+s"(ls));
 #pragma unroll
     for (int i = 0; i < LX; i++) {
-        const long idx = base + (long)i * S;
+        const long idx = lb + (long)i * ls;
         const double2 v = y[idx] * s;
         y[idx] = v;
         f0[idx] = cvt<HC>(to64(f0[idx]) + to64(r[i]) * s - v * e);
+        if (i % 4 == 3) __builtin_amdgcn_sched_barrier(0);
     }
 }
 
@@ -768,6 +783,11 @@ template <bool SP> struct HyzBig {
     static constexpr int NT = SP ? 512 : 1024;
 };
 
+// threads of the yz pass of the 18^2, 36^2 and 48^2 planes: two to six points
+// each, so that the workgroups that the LDS holds (48^2: two of 75 KB) have
+// the registers too
+constexpr int ext_nt(int ny) { return ny == 18 ? 192 : ny == 36 ? 448 : 384; }
+
 template <bool SP> struct FusedFns {
     typedef hc_t<SP> HC;
     typedef void (*pred_fn)(double2 *, HC *, const HC *, const HC *, const HC *, const HC *, HC *, double *,
@@ -793,8 +813,17 @@ template <bool SP> struct FusedFns {
         case 16: *p = pick_pred<16>(sch); *cf = f_corr<16, SP>; return true;
         case 24: *p = pick_pred<24>(sch); *cf = f_corr<24, SP>; return true;
         case 32: *p = pick_pred<32>(sch); *cf = f_corr<32, SP>; return true;
-        default: return false;
+        default: break;
         }
+        if constexpr (!SP) {
+            switch (nx) {
+            case 18: *p = pick_pred<18>(sch); *cf = f_corr<18, SP>; return true;
+            case 36: *p = pick_pred<36>(sch); *cf = f_corr<36, SP>; return true;
+            case 48: *p = pick_pred<48>(sch); *cf = f_corr<48, SP>; return true;
+            default: break;
+            }
+        }
+        return false;
     }
 
     static bool fix(int nx, fix_fn *f)
@@ -805,8 +834,17 @@ template <bool SP> struct FusedFns {
         case 16: *f = f_fixup_x<16, SP>; return true;
         case 24: *f = f_fixup_x<24, SP>; return true;
         case 32: *f = f_fixup_x<32, SP>; return true;
-        default: return false;
+        default: break;
         }
+        if constexpr (!SP) {
+            switch (nx) {
+            case 18: *f = f_fixup_x<18, SP>; return true;
+            case 36: *f = f_fixup_x<36, SP>; return true;
+            case 48: *f = f_fixup_x<48, SP>; return true;
+            default: break;
+            }
+        }
+        return false;
     }
 
     template <bool TX> static bool hyz_t(int ny, int nz, hyz_fn *h)
@@ -829,6 +867,11 @@ template <bool SP> struct FusedFns {
         if (ny == 8 && nz == 12) { *h = f_hyz<8, 12, SP, TX>; return true; }
         if (ny == 12 && nz == 6) { *h = f_hyz<12, 6, SP, TX>; return true; }
         if (ny == 32 && nz == 96) { *h = f_hyz_big<32, 96, SP, TX, HyzBig<SP>::NC, HyzBig<SP>::NT>; return true; }
+        if constexpr (!SP && !TX) {
+            if (ny == 18 && nz == 18) { *h = f_hyz_big<18, 18, SP, TX, 2, ext_nt(18)>; return true; }
+            if (ny == 36 && nz == 36) { *h = f_hyz_big<36, 36, SP, TX, 2, ext_nt(36)>; return true; }
+            if (ny == 48 && nz == 48) { *h = f_hyz_big<48, 48, SP, TX, 2, ext_nt(48)>; return true; }
+        }
         return false;
     }
 
@@ -838,6 +881,8 @@ template <bool SP> struct FusedFns {
 
 static bool split_mode(const tdw_ctx *c) { return c->p.precision == TDW_SPLIT; }
 
+static bool ext_plane(const tdw_ctx *c) { return c->ny == c->nz && (c->ny == 18 || c->ny == 36 || c->ny == 48); }
+
 // planes above 1024 points (the tube section) run f_hyz_big with its own
 // thread counts; FP64 24^2 and 32^2 planes run it with nt_hyz's
 static bool hyz_big(const tdw_ctx *c) { return c->ny * c->nz > 1024; }
@@ -845,6 +890,7 @@ static bool hyz_big(const tdw_ctx *c) { return c->ny * c->nz > 1024; }
 // threads of the yz pass in the precision SP of its arrays
 template <bool SP> static int hyz_nt(const tdw_ctx *c)
 {
+    if (ext_plane(c)) return ext_nt(c->ny);
     if (!hyz_big(c)) return nt_hyz(c->ny * c->nz);
     return HyzBig<SP>::NT;
 }
@@ -853,7 +899,7 @@ template <bool SP> static int hyz_nt(const tdw_ctx *c)
 template <bool SP> static size_t hyz_lds(const tdw_ctx *c)
 {
     const size_t plane = (SP ? sizeof(float2) : sizeof(double2)) * (size_t)c->ny * (c->nz + 1);
-    if (!hyz_big(c)) return 2 * plane;
+    if (!hyz_big(c) || ext_plane(c)) return 2 * plane;
     return HyzBig<SP>::NC * plane;
 }
 
@@ -863,13 +909,32 @@ bool fused_supported(const tdw_ctx *c)
     // the fused passes apply the constant-effective-mass Hamiltonian
     if (varying_mass(c)) return false;
     if (c->p.precision != TDW_FP64 && c->p.precision != TDW_SPLIT) return false;
-    FusedFns<false>::pred_fn p;
-    FusedFns<false>::corr_fn cf;
     FusedFns<false>::hyz_fn h;
-    if (!FusedFns<false>::xpass(c->nx, c->p.scheme, &p, &cf)) return false;
+    // (the FP32 passes: every length the FP64 ones have but 18, 36 and 48)
+    FusedFns<true>::pred_fn p;
+    FusedFns<true>::corr_fn cf;
+    if (!FusedFns<true>::xpass(c->nx, c->p.scheme, &p, &cf)) return false;
     if (!FusedFns<false>::hyz(c->ny, c->nz, true, &h)) return false;
     // the FP64 yz pass runs in both forms (H of FP64 vectors, gradient steps)
     return hyz_lds<false>(c) <= (size_t)c->max_lds && hyz_lds<true>(c) <= (size_t)c->max_lds;
+}
+
+// Lattices with 18, 36 or 48 points along x, or planes of 18^2, 36^2 or 48^2:
+// the six FP64 passes exist, but not those of split precision, of H alone
+// (fused_apply_h) or of the in-pass gradients, so fused_supported says no and
+// every other entry treats them as before; tdw_step_fused runs the passes and
+// completes the arrays at the end of each step (4 S), since callers there
+// have always got complete arrays.  48^3 x 200 per step: 9.6 ms kernel by
+// kernel, 3.9 ms with
+// the passes (plain step).
+static bool fused_ext(const tdw_ctx *c)
+{
+    if (c->dim != 3 || varying_mass(c) || c->p.precision != TDW_FP64 || fused_supported(c)) return false;
+    FusedFns<false>::pred_fn p;
+    FusedFns<false>::corr_fn cf;
+    FusedFns<false>::hyz_fn h;
+    return FusedFns<false>::xpass(c->nx, c->p.scheme, &p, &cf) && FusedFns<false>::hyz(c->ny, c->nz, false, &h) &&
+           hyz_lds<false>(c) <= (size_t)c->max_lds;
 }
 
 static int nhist(const tdw_ctx *c) { return c->p.scheme == TDW_AB3AM4 ? 3 : c->p.scheme == TDW_AB4AM5 ? 4 : 5; }
@@ -1166,7 +1231,9 @@ int fused_step(tdw_ctx *c, tdw_state *s, int it, int grad_last)
         // hold FP32 values, which the FP64 step cannot continue from
         if (split_mode(c)) return TDW_EINVAL;
         TDW_TRY(fused_finalize(c, s));
-        return tdw_step(c, s, it, grad_last);
+        if (!fused_ext(c)) return tdw_step(c, s, it, grad_last);
+        TDW_TRY(fused_step_t<false>(c, s, it, grad_last));
+        return fused_finalize(c, s);
     }
     if (split_mode(c)) return fused_step_t<true>(c, s, it, grad_last);
     return fused_step_t<false>(c, s, it, grad_last);
