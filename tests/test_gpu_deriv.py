@@ -1,0 +1,69 @@
+"""Laplacian and derivatives of 3D arrays on lattices with compiled axis
+lengths, against numpy's FFT: every length, x lengths whose planes do not fill
+the last tile or workgroup, one array and several, out of place and in place.
+
+Tolerance: 1e-12 of the largest value, as for the other building blocks (an
+FFT of L points errs by a few eps sqrt(log L) of the spectrum's norm times
+k_max^2, here some 1e-14 of the largest value)."""
+import numpy as np
+import pytest
+
+from oracle import pyoracle as po
+from tests import tdgauss
+from tests.test_gpu_parity import TOL, cuda, rel, say
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def torch():
+    import torch as t
+    if not t.cuda.is_available():
+        pytest.skip("no HIP device")
+    return t
+
+
+def kax(n, d, first=False):
+    i = np.arange(n)
+    k = 2 * np.pi / (n * d) * np.where(i < n // 2, i, i - n)
+    if first:
+        k[n // 2] = 0.0
+    return k
+
+
+@pytest.mark.parametrize("shape", [(8, 12, 12), (12, 16, 16), (16, 18, 18), (18, 24, 24), (24, 32, 32), (32, 36, 36),
+                                   (36, 12, 12), (48, 48, 48), (18, 18, 18), (6, 32, 96), (48, 8, 12), (36, 6, 8)])
+@pytest.mark.parametrize("m", [1, 3])
+def test_derivatives_3d_lengths(torch, shape, m):
+    from wslda_amd import td
+    say("case: derivatives shape=%s m=%d" % (shape, m))
+    nx, ny, nz = shape
+    cfg = po.make_cfg(3, nx, ny, nz, dx=0.9)
+    cfg.dy, cfg.dz = 1.1, 1.3
+    N = nx * ny * nz
+    r = np.random.default_rng(nx + ny + m)
+    a = r.normal(size=(m, N)) + 1j * r.normal(size=(m, N))
+    ctx = td.TDContext(tdgauss.to_params(cfg, td.FP64), m, 0)
+    f = np.fft.fftn(a.reshape(m, *shape), axes=(1, 2, 3))
+    d = (0.9, 1.1, 1.3)
+    K = [kax(n, h).reshape([-1 if e == i else 1 for e in range(3)]) for i, (n, h) in enumerate(zip(shape, d))]
+    K1 = [kax(n, h, True).reshape([-1 if e == i else 1 for e in range(3)]) for i, (n, h) in enumerate(zip(shape, d))]
+    back = lambda g: np.fft.ifftn(g, axes=(1, 2, 3)).reshape(m, N)
+    lap = back(-(K[0] ** 2 + K[1] ** 2 + K[2] ** 2) * f)
+    t = cuda(torch, a)
+    out = torch.zeros_like(t)
+    ctx.compute_laplace(t, out)
+    ctx.sync()
+    assert rel(out.cpu().numpy(), lap) < TOL
+    D = [torch.zeros_like(t) for _ in range(3)]
+    out.zero_()
+    ctx.compute_derivatives(t, D[0], D[1], D[2], out)
+    ctx.sync()
+    assert rel(out.cpu().numpy(), lap) < TOL
+    for i in range(3):
+        assert rel(D[i].cpu().numpy(), back(1j * K1[i] * f)) < TOL, i
+    assert rel(t.cpu().numpy(), a) == 0.0
+    ctx.compute_laplace(t, t)
+    ctx.sync()
+    assert rel(t.cpu().numpy(), lap) < TOL
+    ctx.close()

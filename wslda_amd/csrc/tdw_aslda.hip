@@ -16,6 +16,7 @@
 // lap(alpha psi): 5 S per state instead of 14 S.  The gradient of psi along
 // an axis has its Nyquist mode set to zero, as the reference's derivatives
 // do (pca_derivative.cu:169-171).
+#include "tdw_axis.hpp"
 #include "tdw_fft.hpp"
 #include "tdw_fused.hpp"
 #include "tdw_physics.hpp"
@@ -30,86 +31,6 @@ static constexpr int AT = 256;
 // storage of the passes' inputs and outputs: FP64, or FP32 in the
 // split-precision step (the transforms in FP32, the sums in FP64)
 template <bool SP> using ac_t = typename std::conditional<SP, float2, double2>::type;
-
-// ---------------------------------------------------------------------------
-// In-place derivatives along one axis of P pencils held in LDS (L = R1*R2,
-// n = n1*R2 + n2, frequency f = k1 + R1*k2 at position k1*R2 + n2 between
-// the stages; consecutive lanes take consecutive pencils, so layouts whose
-// pencils start one element apart, or a padded row apart, are read without
-// LDS bank conflicts).  A receives the second derivative (factor -k2s m^2, the
-// inverse transform's 1/L folded into k2s); with GRAD, B (same layout)
-// receives the first derivative (factor i k1s m, Nyquist mode zero).  Pencil q starts at
-// (q / QD) * QH + (q % QD) * QL, element stride IS.
-// ---------------------------------------------------------------------------
-template <int L, int P, int QD, int QH, int QL, int IS, int NT, bool GRAD, typename C = double2>
-__device__ __forceinline__ void axis_d12(C *A, C *B, const C *tw, int tid, double k1s, double k2s)
-{
-    typedef decltype(C().x) R;
-    constexpr int R1 = rf::fac2<L>::R1, R2 = rf::fac2<L>::R2;
-    static_assert(R2 > 1, "axis_d12 needs L = R1 * R2 with R2 > 1");
-    // stage 1: R1-point DFTs over n1, twiddle W_L^{n2 k1}
-    for (int b = tid; b < P * R2; b += NT) {
-        const int n2 = b / P, q = b - n2 * P;
-        C *pa = A + (q / QD) * QH + (q % QD) * QL;
-        C v[R1];
-#pragma unroll
-        for (int n1 = 0; n1 < R1; n1++) v[n1] = pa[(n1 * R2 + n2) * IS];
-        rf::small_dft<R1, -1, C>::run(v);
-#pragma unroll
-        for (int k1 = 1; k1 < R1; k1++) v[k1] = cmul(v[k1], tw[(n2 * k1) % L]);
-#pragma unroll
-        for (int k1 = 0; k1 < R1; k1++) pa[(k1 * R2 + n2) * IS] = v[k1];
-    }
-    __syncthreads();
-    // stage 2: R2-point DFTs over n2, the derivative factors, inverse R2 DFTs
-    for (int b = tid; b < P * R1; b += NT) {
-        const int k1 = b / P, q = b - k1 * P;
-        const int off = (q / QD) * QH + (q % QD) * QL;
-        C *pa = A + off;
-        C v[R2], g[R2];
-#pragma unroll
-        for (int n2 = 0; n2 < R2; n2++) v[n2] = pa[(k1 * R2 + n2) * IS];
-        rf::small_dft<R2, -1, C>::run(v);
-#pragma unroll
-        for (int k2 = 0; k2 < R2; k2++) {
-            const int f = k1 + R1 * k2;
-            const int m = (f < L / 2) ? f : f - L;
-            if constexpr (GRAD) g[k2] = (f == L / 2) ? cvt<C>(make_double2(0.0, 0.0)) : imul(v[k2], (R)(k1s * (double)m));
-            v[k2] = v[k2] * (R)(-k2s * (double)(m * m));
-        }
-        rf::small_dft<R2, +1, C>::run(v);
-        if constexpr (GRAD) rf::small_dft<R2, +1, C>::run(g);
-#pragma unroll
-        for (int n2 = 0; n2 < R2; n2++) {
-            C wc = tw[(n2 * k1) % L];
-            wc.y = -wc.y;
-            pa[(k1 * R2 + n2) * IS] = n2 == 0 ? v[n2] : cmul(v[n2], wc);
-            if constexpr (GRAD) B[off + (k1 * R2 + n2) * IS] = n2 == 0 ? g[n2] : cmul(g[n2], wc);
-        }
-    }
-    __syncthreads();
-    // stage 3: inverse R1-point DFTs over k1
-    for (int b = tid; b < P * R2; b += NT) {
-        const int n2 = b / P, q = b - n2 * P;
-        const int off = (q / QD) * QH + (q % QD) * QL;
-        C v[R1];
-        C *pa = A + off;
-#pragma unroll
-        for (int k1 = 0; k1 < R1; k1++) v[k1] = pa[(k1 * R2 + n2) * IS];
-        rf::small_dft<R1, +1, C>::run(v);
-#pragma unroll
-        for (int n1 = 0; n1 < R1; n1++) pa[(n1 * R2 + n2) * IS] = v[n1];
-        if constexpr (GRAD) {
-            C *pb = B + off;
-#pragma unroll
-            for (int k1 = 0; k1 < R1; k1++) v[k1] = pb[(k1 * R2 + n2) * IS];
-            rf::small_dft<R1, +1, C>::run(v);
-#pragma unroll
-            for (int n1 = 0; n1 < R1; n1++) pb[(n1 * R2 + n2) * IS] = v[n1];
-        }
-    }
-    __syncthreads();
-}
 
 // ---------------------------------------------------------------------------
 // x pass: T = K_x (u) / K'_x (v).  One workgroup per (state component, block

@@ -185,6 +185,9 @@ int launch_outer(tdw_ctx *c, int m, const double2 *in, double2 *T, double2 *ddx,
     size_t lds = sizeof(double2) * ((size_t)L + (size_t)(mode ? 3 : 2) * TP * L);
     if (lds > (size_t)c->max_lds) return TDW_ESIZE;
     TDW_TIMED(c, mode ? "fft_outer_deriv" : "fft_outer");
+    int done;
+    TDW_TRY(deriv3d_outer(c, m, in, T, ddx, mode, &done));
+    if (done) return 0;
     if (mode == 0)
         hipLaunchKernelGGL(k_outer<0>, dim3(nblk), dim3(NTHR), lds, c->stream, in, T, ddx, m,
                            (long)c->N, S, TP, c->ax[0], c->d_tw[0], c->Lphys[0]);
@@ -227,6 +230,12 @@ int launch_inner(tdw_ctx *c, int m, const double2 *in, const double2 *T, double2
     if (c->dim == 1) return TDW_EINVAL;
     long nblk = (long)m * c->nx;   // inner blocks of S points
     if (c->dim == 3) {
+        int done;
+        {
+            TDW_TIMED(c, mode ? "fft_inner_deriv" : "fft_inner");
+            TDW_TRY(deriv3d_inner(c, m, in, T, out, ddy, ddz, mode, &done));
+        }
+        if (done) return 0;
         if (mode == 0) return launch_inner_k<0, 2>(c, nblk, 1, in, T, out, ddy, ddz);
         return launch_inner_k<1, 2>(c, nblk, 1, in, T, out, ddy, ddz);
     }

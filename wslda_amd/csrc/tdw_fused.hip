@@ -32,6 +32,7 @@
 // densities and the yz pass read that copy.  The corrector reads c and the
 // copy, writes the FP64 y and an FP32 copy of it (into H's buffer, which it
 // has consumed) for the second density and yz passes.
+#include "tdw_axis.hpp"
 #include "tdw_fft.hpp"
 #include "tdw_fused.hpp"
 #include "tdw_physics.hpp"
@@ -49,20 +50,6 @@ static constexpr int FT = 256;
 // scratch: FP64 in the plain form; FP32 in the split-precision form, where
 // the state y stays FP64 and every update of it is done in FP64.
 template <bool SP> using hc_t = typename std::conditional<SP, float2, double2>::type;
-
-template <int LX, typename C>
-__device__ __forceinline__ void dxx_inplace(C (&r)[LX], double kscale)
-{
-    // D_x = F^-1 (-k^2/LX) F ; kscale = (2 pi / Lx)^2 / LX
-    typedef decltype(r[0].x) R;
-    rf::fft<LX, -1, C>(r);
-#pragma unroll
-    for (int i = 0; i < LX; i++) {
-        const int m = (i < LX / 2) ? i : i - LX;
-        r[i] = r[i] * (R)(-kscale * (double)(m * m));
-    }
-    rf::fft<LX, +1, C>(r);
-}
 
 // wave: S % 64 == 0, so every wave lies inside one component and Ptot % 64 == 0
 __device__ __forceinline__ void put_norm_part(double nrm, bool wave, long P, long Ptot, double *part)
@@ -302,128 +289,6 @@ constexpr int nt_hyz(int E)
     return E % 256 == 0 ? 256 : E % 192 == 0 ? 192 : E <= 64 ? 64 : E <= 128 ? 128 : E <= 192 ? 192 : 256;
 }
 
-// In-place transforms along one axis of P pencils held in LDS, for
-// L = R1*R2: with n = n1*R2 + n2 and f = k1 + R1*k2,
-//   X[f] = sum_n2 W_R2^{n2 k2} W_L^{n2 k1} sum_n1 x[n1 R2 + n2] W_R1^{n1 k1},
-// stage 1 (per n2): R1-point DFT over n1, twiddle W_L^{n2 k1}, stored at k1*R2 + n2;
-// stage 2 (per k1): R2-point DFT over n2 -> X[k1 + R1 k2], times mul(m(f), q)
-//   for pencil q, inverse R2-point DFT and the conjugate twiddle, stored at
-//   k1*R2 + n2;
-// stage 3 (per n2): inverse R1-point DFT over k1, stored at n1*R2 + n2.
-// MODE 0 runs all three (with mul = -ks m^2 the second derivative); MODE 1
-// stops after the forward R2-point DFT and leaves X[k1 + R1 k2] at position
-// k1*R2 + k2; MODE 2 starts from that layout and runs the inverse half.
-// Every stage reads and writes the same positions, so one buffer suffices.
-// Consecutive lanes take consecutive pencils: with pencils one element or one
-// padded row apart, a wave's LDS accesses fall in distinct banks.
-
-// frequency index m(f) in (-L/2, L/2] of the DFT output at position p (MODE 1 layout)
-template <int L> __host__ __device__ constexpr int axis_freq(int p)
-{
-    constexpr int R1 = rf::fac2<L>::R1, R2 = rf::fac2<L>::R2;
-    const int f = R2 > 1 ? p / R2 + R1 * (p % R2) : p;
-    return f < L / 2 ? f : f - L;
-}
-
-struct KsMul {
-    double ks;
-    __device__ double operator()(int m, int) const { return -ks * (double)(m * m); }
-};
-
-template <int L, int P, int QD, int QH, int QL, int IS, int NT, int MODE, typename C, typename MUL>
-__device__ __forceinline__ void dft_axis(C *A, const C *tw, int tid, MUL mul)
-{
-    typedef decltype(C().x) Rl;
-    constexpr int R1 = rf::fac2<L>::R1, R2 = rf::fac2<L>::R2;
-    // stage 1
-    if constexpr (R2 > 1 && MODE != 2) {
-        for (int b = tid; b < P * R2; b += NT) {
-            const int n2 = b / P, q = b - n2 * P;
-            C *pa = A + (q / QD) * QH + (q % QD) * QL;
-            C v[R1];
-#pragma unroll
-            for (int n1 = 0; n1 < R1; n1++) v[n1] = pa[(n1 * R2 + n2) * IS];
-            rf::dft_inplace<R1, -1, C>(v);
-#pragma unroll
-            for (int k1 = 1; k1 < R1; k1++) v[k1] = cmul(v[k1], tw[(n2 * k1) % L]);
-#pragma unroll
-            for (int k1 = 0; k1 < R1; k1++) pa[(k1 * R2 + n2) * IS] = v[k1];
-        }
-        __syncthreads();
-    }
-    // stage 2 (for R2 == 1 the whole transform)
-    for (int b = tid; b < P * R1; b += NT) {
-        const int k1 = b / P, q = b - k1 * P;
-        C *pa = A + (q / QD) * QH + (q % QD) * QL;
-        if constexpr (R2 > 1) {
-            C v[R2];
-#pragma unroll
-            for (int n2 = 0; n2 < R2; n2++) v[n2] = pa[(k1 * R2 + n2) * IS];
-            if constexpr (MODE != 2) {
-                rf::dft_inplace<R2, -1, C>(v);
-                if constexpr (MODE == 1) {
-#pragma unroll
-                    for (int k2 = 0; k2 < R2; k2++) pa[(k1 * R2 + k2) * IS] = v[k2];
-                    continue;
-                }
-#pragma unroll
-                for (int k2 = 0; k2 < R2; k2++) {
-                    const int f = k1 + R1 * k2;
-                    const int m = (f < L / 2) ? f : f - L;
-                    v[k2] = v[k2] * (Rl)mul(m, q);
-                }
-            }
-            rf::dft_inplace<R2, +1, C>(v);
-#pragma unroll
-            for (int n2 = 0; n2 < R2; n2++) {
-                C w = tw[(n2 * k1) % L];
-                w.y = -w.y;
-                pa[(k1 * R2 + n2) * IS] = n2 == 0 ? v[n2] : cmul(v[n2], w);
-            }
-        } else if (k1 == 0) {
-            // R2 == 1: one group per pencil holds the whole pencil
-            C v[R1];
-#pragma unroll
-            for (int n = 0; n < R1; n++) v[n] = pa[n * IS];
-            if constexpr (MODE != 2) {
-                rf::dft_inplace<R1, -1, C>(v);
-                if constexpr (MODE == 0) {
-#pragma unroll
-                    for (int f = 0; f < R1; f++) {
-                        const int m = (f < L / 2) ? f : f - L;
-                        v[f] = v[f] * (Rl)mul(m, q);
-                    }
-                }
-            }
-            if constexpr (MODE != 1) rf::dft_inplace<R1, +1, C>(v);
-#pragma unroll
-            for (int n = 0; n < R1; n++) pa[n * IS] = v[n];
-        }
-    }
-    __syncthreads();
-    // stage 3
-    if constexpr (R2 > 1 && MODE != 1) {
-        for (int b = tid; b < P * R2; b += NT) {
-            const int n2 = b / P, q = b - n2 * P;
-            C *pa = A + (q / QD) * QH + (q % QD) * QL;
-            C v[R1];
-#pragma unroll
-            for (int k1 = 0; k1 < R1; k1++) v[k1] = pa[(k1 * R2 + n2) * IS];
-            rf::dft_inplace<R1, +1, C>(v);
-#pragma unroll
-            for (int n1 = 0; n1 < R1; n1++) pa[(n1 * R2 + n2) * IS] = v[n1];
-        }
-        __syncthreads();
-    }
-}
-
-// second derivative along one axis, in place (ks = (2 pi / L_phys)^2 / L)
-template <int L, int P, int QD, int QH, int QL, int IS, int NT, typename C>
-__device__ __forceinline__ void lap_axis(C *A, const C *tw, int tid, double ks)
-{
-    dft_axis<L, P, QD, QH, QL, IS, NT, 0>(A, tw, tid, KsMul{ks});
-}
-
 struct HParams {
     double mu_a, mu_b;
     int bdg;
@@ -525,15 +390,6 @@ f_hyz(const hc_t<SP> *__restrict__ y, const hc_t<SP> *__restrict__ T, hc_t<SP> *
     ssum = block_sum(ssum, red);
     if (tid == 0) part[blockIdx.x] = ssum;
 }
-
-// multiplier of the y pass of a 2D transform: -(k_y^2 + k_z^2) / (LY LZ),
-// with the z part per position of the z-transformed row in zt
-struct YZMul {
-    double ky;
-    const double *zt;
-    int lz;
-    __device__ double operator()(int m, int q) const { return -(ky * (double)(m * m) + zt[q % lz]); }
-};
 
 // yz pass with D_y + D_z as one 2D transform in place (forward along z;
 // forward, scale and inverse along y; inverse along z), NC components in LDS
@@ -638,24 +494,6 @@ f_hyz_big(const hc_t<SP> *__restrict__ y, const hc_t<SP> *__restrict__ T, hc_t<S
     }
     ssum = block_sum(ssum, red);
     if (tid == 0) part[blockIdx.x] = ssum;
-}
-
-// T = D_x in (x-pencils, one lane per pencil): the x-pass of an H
-// application to arbitrary vectors (the adjoint's)
-template <int LX>
-__global__ void __launch_bounds__(FT)
-f_dx(const double2 *__restrict__ in, double2 *__restrict__ T, int n, long N, int S, double kscale)
-{
-    const long P = (long)blockIdx.x * FT + threadIdx.x;
-    if (P >= 2L * n * S) return;
-    const long a2 = P / S, j = P - a2 * S;
-    const long base = a2 * N + j;
-    double2 r[LX];
-#pragma unroll
-    for (int i = 0; i < LX; i++) r[i] = in[base + (long)i * S];
-    dxx_inplace<LX>(r, kscale);
-#pragma unroll
-    for (int i = 0; i < LX; i++) T[base + (long)i * S] = r[i];
 }
 
 // out -= e_a in (the <H> subtraction, pca_kernels.cu:806-832)
@@ -924,9 +762,8 @@ bool fused_supported(const tdw_ctx *c)
 // (fused_apply_h) or of the in-pass gradients, so fused_supported says no and
 // every other entry treats them as before; tdw_step_fused runs the passes and
 // completes the arrays at the end of each step (4 S), since callers there
-// have always got complete arrays.  48^3 x 200 per step: 9.6 ms kernel by
-// kernel, 3.9 ms with
-// the passes (plain step).
+// have always got complete arrays.  48^3 x 200: 9.6 ms per plain step kernel
+// by kernel, 3.9 ms with the passes.
 static bool fused_ext(const tdw_ctx *c)
 {
     if (c->dim != 3 || varying_mass(c) || c->p.precision != TDW_FP64 || fused_supported(c)) return false;
@@ -1161,7 +998,7 @@ static int fused_step_t(tdw_ctx *c, tdw_state *s, int it, int grad_last, tdw_tap
 }
 
 // H applied to arbitrary FP64 vectors on the fused passes: T = D_x in
-// (f_dx), then the yz pass adding T (scale 1).  With qpe: <H> per state into
+// (launch_outer), then the yz pass adding T (scale 1).  With qpe: <H> per state into
 // qpe and out -= <H> in (apply_h); without: H in only (apply_h_only).  With
 // use_e: out -= use_e in, a known <H> (qpe is then not written).
 int fused_apply_h(tdw_ctx *c, int n, const double2 *in, double2 *out, double2 *T, const double *pots, double *qpe,
@@ -1171,23 +1008,7 @@ int fused_apply_h(tdw_ctx *c, int n, const double2 *in, double2 *out, double2 *T
     if (!fused_supported(c)) return TDW_EINVAL;
     TDW_TRY(fused_state_vecs(c));
     TDW_TRY(ensure_f(c, (size_t)n * c->nx));
-    const int S = c->S;
-    const double kxs = pow(2.0 * M_PI / c->Lphys[0], 2) / c->nx;
-    void (*dx)(const double2 *, double2 *, int, long, int, double) = nullptr;
-    switch (c->nx) {
-    case 8: dx = f_dx<8>; break;
-    case 12: dx = f_dx<12>; break;
-    case 16: dx = f_dx<16>; break;
-    case 24: dx = f_dx<24>; break;
-    case 32: dx = f_dx<32>; break;
-    default: return TDW_EINVAL;
-    }
-    {
-        TDW_TIMED(c, "f_dx");
-        hipLaunchKernelGGL(dx, dim3((2L * n * S + FT - 1) / FT), dim3(FT), 0, c->stream, in, T, n, (long)c->N, S,
-                           kxs);
-        TDW_HIP(hipGetLastError());
-    }
+    TDW_TRY(launch_outer(c, 2 * n, in, T, nullptr, 0));
     TDW_TRY(hyz<false>(c, n, in, T, out, pots, nullptr, (qpe && !use_e) ? qpe : c->d_ep, nullptr));
     const double *e = use_e ? use_e : qpe;
     if (e) {

@@ -143,6 +143,11 @@ int h2d(tdw_ctx *c, int n, const double2 *in, double2 *out, const double *pots, 
 // Inner (y[,z]) pass: out = T + D_y(in) + D_z(in) [ddy, ddz].  T may be NULL.
 int launch_inner(tdw_ctx *c, int m, const double2 *in, const double2 *T, double2 *out,
                  double2 *ddy, double2 *ddz, int mode);
+// The same passes of 3D lattices with compiled axis lengths (tdw_deriv.hip);
+// *done = 0 where the lattice has none (nothing launched).
+int deriv3d_outer(tdw_ctx *c, int m, const double2 *in, double2 *T, double2 *ddx, int mode, int *done);
+int deriv3d_inner(tdw_ctx *c, int m, const double2 *in, const double2 *T, double2 *out, double2 *ddy, double2 *ddz,
+                  int mode, int *done);
 }  // namespace tdw
 
 #define TDW_TRY(x)                                  \
