@@ -53,7 +53,7 @@ struct tdw_ctx {
     double *d_qpe;                       // n <H>
     double *d_esum;                      // energies (TDW_NITEMS)
     double2 *d_T;    size_t T_cap;       // laplacian scratch (complex elements)
-    double2 *d_rtmp;                     // N complex (real-field transforms)
+    double2 *d_rtmp;                     // 2N complex (real-field transforms)
     double *d_vext;                      // 2N
     void *ref_workarea;                  // set_workspace_for_cufftPlan()
     // fused-path state
@@ -69,7 +69,7 @@ struct tdw_ctx {
     double *d_adjv;                      // 4n per-state scalars of the backward step
     // ASLDA (allocated on first use)
     double *d_hx;                        // 4N: lap alpha_a, lap alpha_b, div A_a, div A_b
-    double2 *d_ascr;                     // 4N complex: derivative scratch of the real fields
+    double2 *d_ascr;                     // 34N complex: the real fields of H and their derivatives
     double2 *d_aw;   size_t aw_cap;      // lap(alpha psi) (complex elements)
     // grid-field helpers (tdw_grid.hip, allocated on first use)
     double2 *d_gscr;                     // 6N complex
