@@ -54,6 +54,7 @@ def problem(dim, shape, n, scheme, functional, seed=5):
 CASES = [
     (1, (2, 4, 4), 5), (1, (54, 4, 4), 300), (1, (256, 4, 4), 40), (1, (432, 4, 4), 6),
     (2, (8, 12, 6), 270), (2, (36, 18, 4), 20), (2, (6, 128, 4), 9), (2, (48, 54, 4), 7), (2, (64, 64, 4), 5),
+    (2, (32, 32, 4), 300), (2, (32, 64, 4), 6), (2, (64, 32, 4), 6),
     (2, (72, 72, 4), 4),       # the state (166 KB) does not fit: the plane-wise step
     (3, (12, 12, 12), 30), (3, (8, 6, 4), 600), (3, (16, 16, 16), 6), (3, (4, 18, 24), 12),
 ]

@@ -664,11 +664,8 @@ static int adj_forward(tdw_ctx *c, tdw_state *s, int it, tdw_complex *y_out, dou
     const int k = cf.h;
     const long N = (long)c->N;
     double *qpe = s->qpe ? s->qpe : c->d_qpe;
-    // the call sequence of tdw_step (pca.c:1401-1570), non-gradient form;
-    // the densities of a non-gradient step do not read the Laplacian, and 2D
-    // lattices with a plane kernel form it inside the H application
-    const bool plane = h2d_supported(c);
-    const bool fused = !plane && fused_supported(c);
+    // the call sequence of tdw_step (pca.c:1401-1570), non-gradient form
+    const bool fused = fused_supported(c);
     if (fused && s->ddx && s->ddy) {
         // 3D lattices of the fused step: its passes (finalised at the end of
         // the step), with the tape read from its own per-state scalars
@@ -689,18 +686,17 @@ static int adj_forward(tdw_ctx *c, tdw_state *s, int it, tdw_complex *y_out, dou
     // ddy as the D_x scratch (the Laplacian array is then not formed)
     double2 *hT = (fused && s->ddy) ? D2(s->ddy) : nullptr;
     TDW_TRY(normalize(c, n, D2(s->wf), t->scal));
-    if (!plane && !hT) TDW_TRY(laplace(c, 2 * n, D2(s->wf), D2(s->lap)));
+    if (!hT) TDW_TRY(laplace(c, 2 * n, D2(s->wf), D2(s->lap)));
     TDW_TRY(densities(c, n, D2(s->wf), nullptr, nullptr, nullptr, D2(s->lap), c->d_fbeta, nullptr, c->d_kt, c->d_cnt,
                       s->dens, 0));
     TDW_TRY(copy_d(c, s->dens, t->dens_p, 12 * N));
     TDW_TRY(potentials(c, it + 1, s->dens, s->pots));
     TDW_TRY(copy_d(c, s->pots, t->pots_p, 12 * N));
-    if (plane) TDW_TRY(apply_h_plane(c, it + 1, n, D2(s->wf), D2(s->lap), s->pots, c->d_kt, nullptr, t->scal + n));
-    else if (hT) TDW_TRY(fused_apply_h(c, n, D2(s->wf), D2(s->lap), hT, s->pots, t->scal + n));
+    if (hT) TDW_TRY(fused_apply_h(c, n, D2(s->wf), D2(s->lap), hT, s->pots, t->scal + n));
     else TDW_TRY(apply_h(c, it + 1, n, D2(s->wf), D2(s->lap), CD2(s->lap), s->pots, c->d_kt, nullptr, t->scal + n));
     TDW_TRY(abm4(c, n, CD2(s->lap), D2(s->wf), flast));
     TDW_TRY(normalize(c, n, D2(s->wf), t->scal + 2 * n));
-    if (!plane && !hT) TDW_TRY(laplace(c, 2 * n, D2(s->wf), D2(s->lap)));
+    if (!hT) TDW_TRY(laplace(c, 2 * n, D2(s->wf), D2(s->lap)));
     TDW_TRY(densities(c, n, D2(s->wf), nullptr, nullptr, nullptr, D2(s->lap), c->d_fbeta, nullptr, c->d_kt, c->d_cnt,
                       s->dens, 0));
     TDW_TRY(copy_d(c, s->dens, t->dens_c, 12 * N));
@@ -709,9 +705,7 @@ static int adj_forward(tdw_ctx *c, tdw_state *s, int it, tdw_complex *y_out, dou
     tdw_complex *tmp = f_next ? f_next : s->f[k - 1];
     for (int j = k - 1; j > 0; j--) s->f[j] = s->f[j - 1];
     s->f[0] = tmp;
-    if (plane)
-        TDW_TRY(apply_h_plane(c, it + 1, n, D2(s->wf), D2(s->f[0]), s->pots, c->d_kt, nullptr, t->scal + 3 * n));
-    else if (hT)
+    if (hT)
         TDW_TRY(fused_apply_h(c, n, D2(s->wf), D2(s->f[0]), hT, s->pots, t->scal + 3 * n));
     else
         TDW_TRY(apply_h(c, it + 1, n, D2(s->wf), D2(s->f[0]), CD2(s->lap), s->pots, c->d_kt, nullptr, t->scal + 3 * n));
@@ -754,8 +748,7 @@ extern "C" int tdw_adj_forward_step_to(tdw_ctx *c, tdw_state *s, int it, tdw_com
 
 // The history entry taped step `it` left, rebuilt from y after the step and
 // the step's tape: H(pots_c) y1 with the H application that step used, minus
-// the <H> it recorded (scal[3n..4n)).  2D plane lattices subtract inside the
-// plane pass, the others with the step's own subtraction kernel.
+// the <H> it recorded (scal[3n..4n)).
 extern "C" int tdw_adj_history_entry(tdw_ctx *c, int it, const tdw_tape_step *t, const tdw_complex *y1,
                                      tdw_complex *fnew, tdw_complex *scratch)
 {
@@ -765,10 +758,7 @@ extern "C" int tdw_adj_history_entry(tdw_ctx *c, int it, const tdw_tape_step *t,
     const int n = t->n;
     const double *e_c = t->scal + 3 * n;
     if (resident_supported(c)) return resident_h(c, n, CD2(y1), D2(fnew), t->pots_c, nullptr, e_c);
-    const bool plane = h2d_supported(c);
-    const bool fused = !plane && fused_supported(c);
-    if (plane) return apply_h_plane(c, it + 1, n, CD2(y1), D2(fnew), t->pots_c, c->d_kt, e_c, nullptr);
-    if (fused) return fused_apply_h(c, n, CD2(y1), D2(fnew), D2(scratch), t->pots_c, nullptr, e_c);
+    if (fused_supported(c)) return fused_apply_h(c, n, CD2(y1), D2(fnew), D2(scratch), t->pots_c, nullptr, e_c);
     TDW_TRY(laplace(c, 2 * n, CD2(y1), D2(scratch)));
     return apply_h(c, it + 1, n, CD2(y1), D2(fnew), CD2(scratch), t->pots_c, c->d_kt, e_c, nullptr);
 }
@@ -797,9 +787,12 @@ extern "C" int tdw_adj_backward_step(tdw_ctx *c, tdw_adj_state *A, int it, const
     TimerScope ts(c, "adj_step");
 
     // history refresh f_new = H(U') y' - e' y'  (mu = dL/df_new)
-    const bool plane = h2d_supported(c);
-    const bool fused = !plane && fused_supported(c);
-    if (plane) TDW_TRY(apply_h_only_plane(c, n, MU, W1, t->pots_c, c->d_kt, CD2(y1), dv, sv1));
+    // (the same H as the forward step's: the gradient is small against the
+    // sums it comes from, and 64 x 64 lattices with H rounded differently in
+    // the two directions had an error of 2.2e-14 in it for 4e-15)
+    const bool res = resident_supported(c);
+    const bool fused = !res && fused_supported(c);
+    if (res) TDW_TRY(resident_h_only(c, n, MU, W1, t->pots_c, CD2(y1), sv1));
     else {
         TDW_TRY(sdot(c, n, MU, CD2(y1), dv, sv1));
         if (fused) TDW_TRY(fused_apply_h(c, n, MU, W1, W2, t->pots_c, nullptr));
@@ -840,7 +833,7 @@ extern "C" int tdw_adj_backward_step(tdw_ctx *c, tdw_adj_state *A, int it, const
         TDW_HIP(hipGetLastError());
     }
     // F_p = H(U_p) yh_p - e_p yh_p
-    if (plane) TDW_TRY(apply_h_only_plane(c, n, W0, W1, t->pots_p, c->d_kt));
+    if (res) TDW_TRY(resident_h_only(c, n, W0, W1, t->pots_p));
     else if (fused) TDW_TRY(fused_apply_h(c, n, W0, W1, W2, t->pots_p, nullptr));
     else {
         TDW_TRY(laplace(c, 2 * n, W0, W2));

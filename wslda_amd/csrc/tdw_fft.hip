@@ -373,87 +373,6 @@ k_lap2d(const double2 *in, double2 *out, long N, const double2 *__restrict__ twx
     for (int e = tid; e < NX * NY; e += NTHR) out[r0 + e] = A[(e / NY) * NYP + (e % NY)];
 }
 
-// H applied to one plane (one component of one state) per workgroup, with
-// the Laplacian kept in LDS: plane p < n is u_p, p >= n is v_{p-n}; the
-// other component is read pointwise.  The pointwise part is that of
-// apply_hamiltonian_2d (as in k_apply_h), with kz the state's transverse
-// momentum and alpha = 1 for BdG:
-//   (H psi)_u =  (V_a - mu_a + alpha_a kz^2/2) u + Delta v  - alpha_a/2 lap u
-//   (H psi)_v = -(V_b - mu_b + alpha_b kz^2/2) v + Delta* u + alpha_b/2 lap v
-// part[p] = Re sum_i conj(psi_p) (H psi)_p; with dotw, also
-// part2[p] = Re sum_i conj(psi_p) dotw_p.  With esub, out = (H - esub_a) psi
-// (the <H> subtraction with a known <H>, in the same pass).  out must not
-// alias in (the other component is read from in).
-template <int NX, int NY>
-__global__ void __launch_bounds__(NTHR)
-k_h2d(const double2 *__restrict__ in, double2 *__restrict__ out, long N, int n, const double2 *__restrict__ twx_g,
-      const double2 *__restrict__ twy_g, double ksx, double ksy, const double *__restrict__ pots,
-      const double *__restrict__ kt, int bdg, double mu_a, double mu_b, double *__restrict__ part,
-      const double2 *__restrict__ dotw, double *__restrict__ part2, const double *__restrict__ esub)
-{
-    constexpr int NYP = NY + 1, E = NX * NY, KM = (E + NTHR - 1) / NTHR;
-    extern __shared__ double2 lds2[];
-    __shared__ double2 twx[NX], twy[NY];
-    __shared__ double red[NTHR / 64];
-    double2 *A = lds2;
-    const int tid = threadIdx.x;
-    const int p = blockIdx.x;
-    const int comp = p >= n ? 1 : 0;
-    const int a = p - comp * n;
-    const long own = (long)p * N, oth = (long)(comp ? a : n + a) * N;
-    for (int k = tid; k < NX; k += NTHR) twx[k] = twx_g[k];
-    for (int k = tid; k < NY; k += NTHR) twy[k] = twy_g[k];
-    // the plane stays in registers for the pointwise part; the other
-    // component is fetched while the transforms run
-    double2 X[KM], Y[KM];
-#pragma unroll
-    for (int k = 0; k < KM; k++) {
-        const int e = tid + k * NTHR;
-        if (e < E) {
-            X[k] = in[own + e];
-            A[(e / NY) * NYP + (e % NY)] = X[k];
-        }
-    }
-#pragma unroll
-    for (int k = 0; k < KM; k++) {
-        const int e = tid + k * NTHR;
-        if (e < E) Y[k] = in[oth + e];
-    }
-    __syncthreads();
-    lap_plane<NX, NY>(A, twx, twy, tid, ksx, ksy);
-    const double k2t = kt ? kt[a] * kt[a] : 0.0;
-    const double es = esub ? esub[a] : 0.0;
-    double s = 0.0, s2 = 0.0;
-#pragma unroll
-    for (int k = 0; k < KM; k++) {
-        const int e = tid + k * NTHR;
-        if (e >= E) continue;
-        const double2 lp = A[(e / NY) * NYP + (e % NY)];
-        const double2 x = X[k], y = Y[k];
-        const double2 D = make_double2(pots[2 * N + 2 * e], pots[2 * N + 2 * e + 1]);
-        double2 r;
-        if (!comp) {
-            const double aa = bdg ? -0.5 : pots[4 * N + e] * -0.5;
-            const double Va = pots[e] - mu_a + (-1.0 * aa * k2t);
-            r = x * Va + cmul(y, D) + lp * aa;
-        } else {
-            const double ab = bdg ? -0.5 : pots[5 * N + e] * -0.5;
-            const double Vb = pots[N + e] - mu_b + (-1.0 * ab * k2t);
-            r = x * (-Vb) + cmulc(D, y) - lp * ab;
-        }
-        s += cmulc(x, r).x;
-        if (esub) r = r - x * es;
-        out[own + e] = r;
-        if (dotw) s2 += cmulc(x, dotw[own + e]).x;
-    }
-    s = block_sum(s, red);
-    if (tid == 0) part[p] = s;
-    if (dotw) {
-        s2 = block_sum(s2, red);
-        if (tid == 0) part2[p] = s2;
-    }
-}
-
 typedef void (*lap2d_fn)(const double2 *, double2 *, long, const double2 *, const double2 *, double, double);
 
 static bool lap2d_for(const tdw_ctx *c, lap2d_fn *f, size_t *lds)
@@ -486,51 +405,6 @@ int lap2d(tdw_ctx *c, int m, const double2 *in, double2 *out, int *done)
     const double ksx = pow(2.0 * M_PI / c->Lphys[0], 2) / N, ksy = pow(2.0 * M_PI / c->Lphys[1], 2) / N;
     hipLaunchKernelGGL(f, dim3(m), dim3(NTHR), lds, c->stream, in, out, (long)c->N, c->d_tw[0], c->d_tw[1], ksx,
                        ksy);
-    TDW_HIP(hipGetLastError());
-    return 0;
-}
-
-typedef void (*h2d_fn)(const double2 *, double2 *, long, int, const double2 *, const double2 *, double, double,
-                       const double *, const double *, int, double, double, double *, const double2 *, double *,
-                       const double *);
-
-static bool h2d_for(const tdw_ctx *c, h2d_fn *f, size_t *lds)
-{
-    if (c->dim != 2 || c->nx != c->ny) return false;
-    switch (c->nx) {
-    case 8: *f = k_h2d<8, 8>; break;
-    case 12: *f = k_h2d<12, 12>; break;
-    case 16: *f = k_h2d<16, 16>; break;
-    case 24: *f = k_h2d<24, 24>; break;
-    case 32: *f = k_h2d<32, 32>; break;
-    case 64: *f = k_h2d<64, 64>; break;
-    default: return false;
-    }
-    *lds = sizeof(double2) * (size_t)c->nx * (c->ny + 1);
-    return *lds <= (size_t)c->max_lds;
-}
-
-bool h2d_supported(const tdw_ctx *c)
-{
-    // the plane kernel applies the constant-effective-mass Hamiltonian
-    if (varying_mass(c)) return false;
-    h2d_fn f;
-    size_t lds;
-    return h2d_for(c, &f, &lds);
-}
-
-int h2d(tdw_ctx *c, int n, const double2 *in, double2 *out, const double *pots, const double *kt, double *part,
-        const double2 *dotw, double *part2, const double *esub)
-{
-    h2d_fn f;
-    size_t lds;
-    if (!h2d_for(c, &f, &lds) || in == out) return TDW_EINVAL;
-    TDW_TIMED(c, "h2d");
-    const double N = (double)c->N;
-    const double ksx = pow(2.0 * M_PI / c->Lphys[0], 2) / N, ksy = pow(2.0 * M_PI / c->Lphys[1], 2) / N;
-    hipLaunchKernelGGL(f, dim3(2 * n), dim3(NTHR), lds, c->stream, in, out, (long)c->N, n, c->d_tw[0], c->d_tw[1],
-                       ksx, ksy, pots, kt, c->p.functional == TDW_BDG, c->p.mu_a, c->p.mu_b, part, dotw, part2,
-                       esub);
     TDW_HIP(hipGetLastError());
     return 0;
 }

@@ -831,47 +831,6 @@ int apply_h(tdw_ctx *c, int it, int n, const double2 *in, double2 *out, const do
     return (int)hipGetLastError();
 }
 
-// qpe[a] = dv (part[a] + part[n + a]): <H> from the per-plane sums of h2d
-__global__ void k_plane_pairs(const double *__restrict__ part, int n, double dv, double *__restrict__ qpe)
-{
-    const int a = blockIdx.x * blockDim.x + threadIdx.x;
-    if (a < n) qpe[a] = dv * (part[a] + part[n + a]);
-}
-
-// apply_h for 2D lattices with a one-pass plane kernel: the Laplacian of in
-// is formed in LDS and not stored (lap of apply_h is not needed)
-int apply_h_plane(tdw_ctx *c, int it, int n, const double2 *in, double2 *out, const double *pots, const double *kt,
-                  const double *useqpe, double *d_qpe)
-{
-    (void)it;
-    TDW_TRY(ensure_part(c, (size_t)2 * n));
-    if (useqpe) {
-        // a known <H>: subtracted inside the plane pass
-        TDW_TRY(h2d(c, n, in, out, pots, kt, c->d_part, nullptr, nullptr, useqpe));
-        if (d_qpe && d_qpe != useqpe)
-            TDW_HIP(hipMemcpyAsync(d_qpe, useqpe, sizeof(double) * n, hipMemcpyDeviceToDevice, c->stream));
-        return 0;
-    }
-    TDW_TRY(h2d(c, n, in, out, pots, kt, c->d_part));
-    TDW_TIMED(c, "apply_h");
-    hipLaunchKernelGGL(k_plane_pairs, dim3((n + 255) / 256), dim3(256), 0, c->stream, c->d_part, n, dvol_norm(c),
-                       d_qpe);
-    const long N = (long)c->N, tot = 2L * n * N;
-    hipLaunchKernelGGL(k_sub_qpe, dim3((tot + NT - 1) / NT), dim3(NT), 0, c->stream, in, out, n, N, d_qpe);
-    return (int)hipGetLastError();
-}
-
-int apply_h_only_plane(tdw_ctx *c, int n, const double2 *in, double2 *out, const double *pots, const double *kt,
-                       const double2 *dotw, double dscale, double *d_dot)
-{
-    TDW_TRY(ensure_part(c, (size_t)4 * n));
-    TDW_TRY(h2d(c, n, in, out, pots, kt, c->d_part, dotw, dotw ? c->d_part + 2 * n : nullptr));
-    if (dotw)
-        hipLaunchKernelGGL(k_plane_pairs, dim3((n + 255) / 256), dim3(256), 0, c->stream, c->d_part + 2 * n, n, dscale,
-                           d_dot);
-    return (int)hipGetLastError();
-}
-
 // out = H in, without the <H> sums and subtraction (the adjoint applies H to
 // its own vectors and subtracts in its next pass)
 int apply_h_only(tdw_ctx *c, int n, const double2 *in, double2 *out, const double2 *lap, const double *pots,

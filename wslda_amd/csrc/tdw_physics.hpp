@@ -168,13 +168,6 @@ int apply_h(tdw_ctx *c, int it, int n, const double2 *in, double2 *out, const do
             const double *pots, const double *kt, const double *useqpe, double *d_qpe);
 int apply_h_only(tdw_ctx *c, int n, const double2 *in, double2 *out, const double2 *lap, const double *pots,
                  const double *kt);
-// the same two on 2D lattices with a one-pass plane kernel (h2d_supported):
-// the Laplacian of in is formed in LDS; out must differ from in
-int apply_h_plane(tdw_ctx *c, int it, int n, const double2 *in, double2 *out, const double *pots, const double *kt,
-                  const double *useqpe, double *d_qpe);
-// With dotw, also d_dot[a] = dscale Re<in_a, dotw_a> (both components).
-int apply_h_only_plane(tdw_ctx *c, int n, const double2 *in, double2 *out, const double *pots, const double *kt,
-                       const double2 *dotw = nullptr, double dscale = 0.0, double *d_dot = nullptr);
 // ASLDA: out = alpha_s psi_s (in place allowed)
 int alpha_wf(tdw_ctx *c, int n, const double2 *in, double2 *out, const double *pots);
 // ASLDA H application with the <H> subtraction: ddx..ddz the gradients of in

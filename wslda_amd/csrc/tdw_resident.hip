@@ -104,6 +104,7 @@ struct RsH {
 // CORR 1: psi = s_a in (the normalised prediction), out = the normalised
 // corrected state of -i dt a0 (H psi - <H> psi) + c (out may be in: a state
 // is read whole before it is written).
+// CORR 2: out = H psi, psi = in (out is not in); with c, e_out = dv Re <in|c>.
 // <H> per state into e_out (and e_out2), or read from use_e; the corrected
 // state's norm into nrm_out where given.  H as in k_apply_h, with the transverse momenta of 1D
 // and 2D (kt, and kt2 in 1D) in the kinetic term.
@@ -120,7 +121,7 @@ rs_h(const double2 *in, double2 *out, const double2 *__restrict__ c, const doubl
     double2 *A = rs_sm, *tw = rs_sm + 2 * pl.npc;
     const int a = blockIdx.x, tid = threadIdx.x, nt = blockDim.x;
     const long gu = (long)a * N, gv = ((long)n + a) * N;
-    const double s = CORR ? sc[a] : 1.0;
+    const double s = CORR == 1 ? sc[a] : 1.0;
     for (int k = tid; k < ntw; k += nt) tw[k] = twg[k];
     // point i of a component sits at i + i / ll: rows of the last axis, ll + 1 apart
     const int pad = pl.dim > 1;
@@ -144,9 +145,21 @@ rs_h(const double2 *in, double2 *out, const double2 *__restrict__ c, const doubl
         const double2 tu = in[gu + i] * s, tv = in[gv + i] * s;
         const double2 u = tu * Va + cmul(tv, D) + A[pe] * aa;
         const double2 v = tv * (-Vb) + cmulc(D, tu) - A[pl.npc + pe] * ab;
+        if constexpr (CORR == 2) {
+            out[gu + i] = u;
+            out[gv + i] = v;
+            if (c) e += cmulc(tu, c[gu + i]).x + cmulc(tv, c[gv + i]).x;
+            continue;
+        }
         A[pe] = u;
         A[pl.npc + pe] = v;
         e += cmulc(tu, u).x + cmulc(tv, v).x;
+    }
+    if constexpr (CORR == 2) {
+        if (!c) return;
+        e = block_sum(e, red) * hp.dv;
+        if (tid == 0) e_out[a] = e;
+        return;
     }
     if (use_e) {
         e = use_e[a];
@@ -161,7 +174,7 @@ rs_h(const double2 *in, double2 *out, const double2 *__restrict__ c, const doubl
     for (int i = tid; i < N; i += nt) {
         const int pe = pad ? i + rs_div(i, pl.ll, pl.mll) : i;
         const double2 u = A[pe] - in[gu + i] * s * e, v = A[pl.npc + pe] - in[gv + i] * s * e;
-        if constexpr (CORR) {
+        if constexpr (CORR == 1) {
             const double2 yu = imul(u, -hp.dta0) + c[gu + i], yv = imul(v, -hp.dta0) + c[gv + i];
             A[pe] = yu;
             A[pl.npc + pe] = yv;
@@ -171,7 +184,7 @@ rs_h(const double2 *in, double2 *out, const double2 *__restrict__ c, const doubl
             out[gv + i] = v;
         }
     }
-    if constexpr (CORR) {
+    if constexpr (CORR == 1) {
         nrm = block_sum(nrm, red) * hp.dv;
         const double r = 1.0 / sqrt(nrm);
         if (tid == 0 && nrm_out) nrm_out[a] = nrm;
@@ -184,9 +197,212 @@ rs_h(const double2 *in, double2 *out, const double2 *__restrict__ c, const doubl
 }
 
 // ---------------------------------------------------------------------------
+// The same for 2D planes of 32 or 64 points a side, on the matrix cores.
+//
+// The transforms of rs_h read and write the state seven times in LDS, behind
+// as many barriers, and one 64 x 64 state occupies a CU alone.  The second
+// derivative along an axis of L points is a circulant L x L matrix, real and
+// even; with p = x_j + x_{j + L/2}, m = x_j - x_{j + L/2} it falls into two
+// L/2 x L/2 products, P p and M m (y_i = P p + M m, y_{i + L/2} = P p - M m),
+// contractions for v_mfma_f64_16x16x4.  A wave owns the points (ix, iy) of
+// one component with ix in a 16-row tile or that plus LX/2, iy in a tile or
+// that plus LY/2.  d^2/dx^2 takes the matrix as the A operand and the plane as
+// B, d^2/dy^2 the plane as A and the matrix as B, so both leave the wave's own
+// points in the same registers (row lane / 16 + 4 r, column lane % 16): the
+// plane is written to LDS once, read four times over, never overwritten, and
+// all that follows (H psi, <H>, corrector, norm) stays in registers.
+// More multiplications (64 per point and component at 64 x 64) but no index
+// arithmetic and one barrier before H: at 64 x 64 the corrector form of 1024
+// states 169 -> 128 us, the plain one 141 -> 99, of 192 states 39 -> 28 and
+// 35 -> 25; 32 x 32 and 32 x 64 gain as much.  One 512-thread workgroup per CU
+// at 64 x 64 (133 KB of LDS, 254 registers), bound by its load and store
+// phases, which nothing overlaps.
+// ---------------------------------------------------------------------------
+typedef double dbl4 __attribute__((ext_vector_type(4)));
+
+// a tile's offsets, opaque to the compiler; the previous tile is done with
+__device__ __forceinline__ bool mm_tile(int &i, int &j)
+{
+    __builtin_amdgcn_sched_barrier(0);
+    asm volatile("" : "+v"(i), "+v"(j));
+    return true;
+}
+
+template <int LX, int LY, int CORR>
+__global__ void __launch_bounds__(64 * 2 * (LX / 32) * (LY / 32), 2)
+rs_mm(const double2 *in, double2 *out, const double2 *__restrict__ c, const double *__restrict__ pots,
+      const double *__restrict__ sc, const double *__restrict__ kt, int n, RsH hp, const double *__restrict__ mx,
+      const double *__restrict__ my, const double *use_e, double *e_out, double *e_out2, double *__restrict__ nrm_out)
+{
+    constexpr int HX = LX / 2, HY = LY / 2, TX = HX / 16, TY = HY / 16, W = 2 * TX * TY, NT = 64 * W;
+    constexpr int N = LX * LY, RS = LY + 1, NPC = LX * RS;
+    extern __shared__ double2 rs_sm[];
+    __shared__ double red[W];
+    const int a = blockIdx.x, tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
+    const int cmp = w / (TX * TY), tx = (w / TY) % TX, ty = w % TY;
+    const long gu = (long)a * N, gv = ((long)n + a) * N;
+    const double s = CORR == 1 ? sc[a] : 1.0;
+#pragma unroll 4
+    for (int i = tid; i < N; i += NT) {
+        const int pe = i + i / LY;
+        rs_sm[pe] = in[gu + i] * s;
+        rs_sm[NPC + pe] = in[gv + i] * s;
+    }
+    const double2 *X = rs_sm + cmp * NPC, *Y = rs_sm + (1 - cmp) * NPC;   // own component, the other
+    const int lr = lane >> 4, lc = lane & 15;
+    // lap[h][g]: points (ix + h HX, iy + g HY), four rows each; re and im
+    dbl4 lre[2][2], lim[2][2];
+    __syncthreads();
+    // along x: the matrix times the plane, columns iy
+    {
+        const double *M = mx + (long)tx * (HX / 4) * 128 + lane;
+        dbl4 P[2][2], Q[2][2];   // [column tile][re, im]
+#pragma unroll
+        for (int g = 0; g < 2; g++)
+#pragma unroll
+            for (int q = 0; q < 2; q++) P[g][q] = Q[g][q] = dbl4{0.0, 0.0, 0.0, 0.0};
+#pragma unroll 2
+        for (int ks = 0; ks < HX / 4; ks++) {
+            const double mp = M[ks * 128], mm = M[ks * 128 + 64];
+            const double2 *x = X + (4 * ks + lr) * RS + 16 * ty + lc;
+#pragma unroll
+            for (int g = 0; g < 2; g++) {
+                const double2 u = x[g * HY], v = x[g * HY + HX * RS];
+                P[g][0] = __builtin_amdgcn_mfma_f64_16x16x4f64(mp, u.x + v.x, P[g][0], 0, 0, 0);
+                P[g][1] = __builtin_amdgcn_mfma_f64_16x16x4f64(mp, u.y + v.y, P[g][1], 0, 0, 0);
+                Q[g][0] = __builtin_amdgcn_mfma_f64_16x16x4f64(mm, u.x - v.x, Q[g][0], 0, 0, 0);
+                Q[g][1] = __builtin_amdgcn_mfma_f64_16x16x4f64(mm, u.y - v.y, Q[g][1], 0, 0, 0);
+            }
+        }
+#pragma unroll
+        for (int g = 0; g < 2; g++) {
+            lre[0][g] = P[g][0] + Q[g][0];
+            lim[0][g] = P[g][1] + Q[g][1];
+            lre[1][g] = P[g][0] - Q[g][0];
+            lim[1][g] = P[g][1] - Q[g][1];
+        }
+    }
+    __builtin_amdgcn_sched_barrier(0);
+    // along y: the plane times the matrix, rows ix
+    {
+        const double *M = my + (long)ty * (HY / 4) * 128 + lane;
+        dbl4 P[2][2], Q[2][2];   // [row tile][re, im]
+#pragma unroll
+        for (int h = 0; h < 2; h++)
+#pragma unroll
+            for (int q = 0; q < 2; q++) P[h][q] = Q[h][q] = dbl4{0.0, 0.0, 0.0, 0.0};
+#pragma unroll 2
+        for (int ks = 0; ks < HY / 4; ks++) {
+            const double mp = M[ks * 128], mm = M[ks * 128 + 64];
+            const double2 *x = X + (16 * tx + lc) * RS + 4 * ks + lr;
+#pragma unroll
+            for (int h = 0; h < 2; h++) {
+                const double2 u = x[h * HX * RS], v = x[h * HX * RS + HY];
+                P[h][0] = __builtin_amdgcn_mfma_f64_16x16x4f64(u.x + v.x, mp, P[h][0], 0, 0, 0);
+                P[h][1] = __builtin_amdgcn_mfma_f64_16x16x4f64(u.y + v.y, mp, P[h][1], 0, 0, 0);
+                Q[h][0] = __builtin_amdgcn_mfma_f64_16x16x4f64(u.x - v.x, mm, Q[h][0], 0, 0, 0);
+                Q[h][1] = __builtin_amdgcn_mfma_f64_16x16x4f64(u.y - v.y, mm, Q[h][1], 0, 0, 0);
+            }
+        }
+#pragma unroll
+        for (int h = 0; h < 2; h++) {
+            lre[h][0] += P[h][0] + Q[h][0];
+            lim[h][0] += P[h][1] + Q[h][1];
+            lre[h][1] += P[h][0] - Q[h][0];
+            lim[h][1] += P[h][1] - Q[h][1];
+        }
+    }
+    const double k2t = kt ? kt[a] * kt[a] : 0.0;
+    const long own = cmp ? gv : gu;
+    const double *V = pots + cmp * N, *al = pots + (4 + cmp) * N;
+    const double sg = cmp ? -1.0 : 1.0, mu = cmp ? hp.mu_b : hp.mu_a;
+    // The wave's points, one 16 x 16 tile (four rows r) at a time: tile (h, g)
+    // starts h HX rows and g HY columns on, rows are 4 apart.  The offsets are
+    // formed per tile and kept opaque, else all sixteen points' addresses are
+    // (registers).
+    const int i0 = (16 * tx + lr) * LY + 16 * ty + lc, j0 = (16 * tx + lr) * RS + 16 * ty + lc;
+#define MM_TILES(h, g, i, j)                                                                     \
+    _Pragma("unroll") for (int h = 0; h < 2; h++)                                                \
+        _Pragma("unroll") for (int g = 0; g < 2; g++)                                            \
+            if (int i = i0 + h * HX * LY + g * HY, j = j0 + h * HX * RS + g * HY; mm_tile(i, j))
+    // H psi over the Laplacian, <psi|H psi>
+    const double2 *co = CORR && c ? c + own : nullptr;
+    double2 *oo = out + own;
+    double e = 0.0;
+    MM_TILES(h, g, i, j) {
+#pragma unroll
+        for (int r = 0; r < 4; r++) {
+            const int ir = i + 4 * r * LY, jr = j + 4 * r * RS;
+            const double2 x = X[jr], y = Y[jr];
+            const double av = al[ir];
+            const double aa = hp.bdg ? -0.5 : av * -0.5;
+            const double Vv = sg * (V[ir] - mu - aa * k2t);
+            const double2 Dv = ((const double2 *)(pots + 2 * N))[ir];
+            const double2 t = x * Vv + cmul(y, make_double2(Dv.x, sg * Dv.y)) +
+                              make_double2(lre[h][g][r], lim[h][g][r]) * (sg * aa);
+            if constexpr (CORR == 2) {
+                oo[ir] = t;
+                if (co) e += cmulc(x, co[ir]).x;
+            } else {
+                lre[h][g][r] = t.x;
+                lim[h][g][r] = t.y;
+                e += cmulc(x, t).x;
+            }
+        }
+    }
+    if constexpr (CORR == 2) {
+        if (!co) return;
+        e = block_sum(e, red) * hp.dv;
+        if (tid == 0) e_out[a] = e;
+        return;
+    }
+    if (use_e) {
+        e = use_e[a];
+    } else {
+        e = block_sum(e, red) * hp.dv;
+        if (tid == 0) {
+            e_out[a] = e;
+            if (e_out2) e_out2[a] = e;
+        }
+    }
+    double nrm = 0.0;
+    MM_TILES(h, g, i, j) {
+#pragma unroll
+        for (int r = 0; r < 4; r++) {
+            const int ir = i + 4 * r * LY;
+            double2 t = make_double2(lre[h][g][r], lim[h][g][r]) - X[j + 4 * r * RS] * e;
+            if constexpr (CORR == 1) {
+                t = imul(t, -hp.dta0) + co[ir];
+                lre[h][g][r] = t.x;
+                lim[h][g][r] = t.y;
+                nrm += cnorm(t);
+            } else {
+                oo[ir] = t;
+            }
+        }
+    }
+    if constexpr (CORR == 1) {
+        nrm = block_sum(nrm, red) * hp.dv;
+        const double q = 1.0 / sqrt(nrm);
+        if (tid == 0 && nrm_out) nrm_out[a] = nrm;
+        MM_TILES(h, g, i, j) {
+#pragma unroll
+            for (int r = 0; r < 4; r++) oo[i + 4 * r * LY] = make_double2(lre[h][g][r], lim[h][g][r]) * q;
+        }
+    }
+#undef MM_TILES
+}
+
+// ---------------------------------------------------------------------------
 // host side
 // ---------------------------------------------------------------------------
 static size_t rs_lds(const RsPlan &pl, int ntw) { return sizeof(double2) * (2 * (size_t)pl.npc + ntw); }
+
+// 2D planes of the matrix-core form: tiles of 16 in both halves of an axis
+static bool mm_plane(const tdw_ctx *c)
+{
+    return c->dim == 2 && (c->nx == 32 || c->nx == 64) && (c->ny == 32 || c->ny == 64);
+}
 
 int resident_setup(tdw_ctx *c)
 {
@@ -234,6 +450,28 @@ int resident_setup(tdw_ctx *c)
         if (dim == 3 && z < ll) v = kk[1][y] + kk[2][z];
         kt.push_back(v);
     }
+    // the halves of the second-derivative circulants in rs_mm's operand order
+    if (mm_plane(c))
+        for (int d = 0; d < 2; d++) {
+            const int L = len[d], H = L / 2;
+            // summed in extended precision, else the rounding of the sums (not
+            // that of the entries) is what the operator differs by
+            std::vector<long double> cs(L), cc(L, 0.0L);
+            for (int t = 0; t < L; t++) cs[t] = cosl(2.0L * 3.141592653589793238462643383L * t / L);
+            for (int x = 0; x < L; x++)
+                for (int f = 0; f < L; f++) {
+                    const long double k = rs_k(f, L, c->Lphys[d]);
+                    cc[x] -= k * k / L * cs[(f * x) % L];
+                }
+            for (int t = 0; t < H / 16; t++)
+                for (int ks = 0; ks < H / 4; ks++)
+                    for (int pm = 0; pm < 2; pm++)
+                        for (int l = 0; l < 64; l++) {
+                            const int x = 16 * t + l % 16 - (4 * ks + l / 16) + L;
+                            const long double v = cc[x % L], h = cc[(x + H) % L];
+                            kt.push_back((double)(0.5L * (pm ? v - h : v + h)));
+                        }
+        }
     const size_t btw = sizeof(double2) * tw.size(), bk = sizeof(double) * kt.size();
     TDW_HIP(hipMalloc(&c->d_rtab, btw + bk));
     TDW_HIP(hipMemcpy(c->d_rtab, tw.data(), btw, hipMemcpyHostToDevice));
@@ -281,6 +519,24 @@ static int launch_h(tdw_ctx *c, int n, const double2 *in, double2 *out, const do
     const size_t lds = rs_lds(pl, ntw);
     const double *kt = c->dim < 3 ? c->d_kt : nullptr, *kt2 = c->dim == 1 ? c->d_kt + n : nullptr;
     TDW_TIMED(c, CORR ? "rs_hcorr" : "rs_h");
+    if (mm_plane(c)) {
+        const double *mx = kx + pl.ax[0].L + pl.inner;
+        const double *my = mx + (size_t)(c->nx / 32) * (c->nx / 8) * 128;
+        const dim3 g(n), b(128 * (c->nx / 32) * (c->ny / 32));
+        const size_t sm = sizeof(double2) * 2 * (size_t)pl.npc;
+#define RS_MM(LX, LY)                                                                                               \
+    hipLaunchKernelGGL((rs_mm<LX, LY, CORR>), g, b, sm, c->stream, in, out, cc, pots, sc, kt, n, hp, mx, my, use_e, \
+                       e_out, e_out2, nrm_out)
+        if (c->nx == 32) {
+            if (c->ny == 32) RS_MM(32, 32);
+            else RS_MM(32, 64);
+        } else {
+            if (c->ny == 32) RS_MM(64, 32);
+            else RS_MM(64, 64);
+        }
+#undef RS_MM
+        return (int)hipGetLastError();
+    }
     hipLaunchKernelGGL(rs_h<CORR>, dim3(n), dim3(rs_threads(lds, n, N)), lds, c->stream, in, out, cc, pots, sc, kt, kt2,
                        n, N, pl, hp, tw, ntw, kx, kx + pl.ax[0].L, use_e, e_out, e_out2, nrm_out);
     return (int)hipGetLastError();
@@ -290,6 +546,12 @@ int resident_h(tdw_ctx *c, int n, const double2 *in, double2 *out, const double 
                const double *use_e)
 {
     return launch_h<0>(c, n, in, out, nullptr, pots, nullptr, use_e, qpe, nullptr, nullptr);
+}
+
+int resident_h_only(tdw_ctx *c, int n, const double2 *in, double2 *out, const double *pots, const double2 *dotw,
+                    double *d_dot)
+{
+    return launch_h<2>(c, n, in, out, dotw, pots, nullptr, nullptr, d_dot, nullptr, nullptr);
 }
 
 static int tape_copy(tdw_ctx *c, const double *src, double *dst, long nd)

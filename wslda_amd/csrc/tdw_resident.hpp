@@ -25,4 +25,7 @@ int resident_step(tdw_ctx *c, tdw_state *s, int it, int grad_last, tdw_tape_step
 // is then not written)
 int resident_h(tdw_ctx *c, int n, const double2 *in, double2 *out, const double *pots, double *qpe,
                const double *use_e = nullptr);
+// out = H in (out is not in); with dotw, d_dot[a] = dv Re <in_a|dotw_a>
+int resident_h_only(tdw_ctx *c, int n, const double2 *in, double2 *out, const double *pots,
+                    const double2 *dotw = nullptr, double *d_dot = nullptr);
 }  // namespace tdw
