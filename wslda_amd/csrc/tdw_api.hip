@@ -204,6 +204,7 @@ extern "C" int tdw_create(const tdw_params *p, int nwf, int device, tdw_ctx **ou
         free(ones);
     }
     if (!e) e = resident_setup(c);
+    if (!e) e = aslda_setup(c);
     if (!e) e = project_attach(c);
     if (e) {
         tdw_destroy(c);
@@ -222,7 +223,7 @@ extern "C" int tdw_destroy(tdw_ctx *c)
         if (c->d_tw[k]) hipFree(c->d_tw[k]);
         if (c->d_tw32[k]) hipFree(c->d_tw32[k]);
     }
-    void *bufs[] = {c->d_fbeta, c->d_kt, c->d_cnt, c->d_part, c->d_nrm, c->d_qpe, c->d_esum,
+    void *bufs[] = {c->d_mmt, c->d_fbeta, c->d_kt, c->d_cnt, c->d_part, c->d_nrm, c->d_qpe, c->d_esum,
                     c->d_T, c->d_rtmp, c->d_vext, c->d_scale, c->d_adjv, c->d_hx, c->d_ascr, c->d_aw,
                     c->d_gscr};
     for (void *b : bufs)

@@ -20,6 +20,7 @@
 #include "tdw_fft.hpp"
 #include "tdw_fused.hpp"
 #include "tdw_physics.hpp"
+#include "tdw_planemm.hpp"
 #include "tdw_regfft.hpp"
 
 #include <type_traits>
@@ -233,6 +234,209 @@ ah_yz(const ac_t<SP> *__restrict__ y, const ac_t<SP> *__restrict__ T, ac_t<SP> *
     if (tid == 0) part[blockIdx.x] = ssum;
 }
 
+// The same for FP64 planes of 24 or 32 points a side, on the matrix cores.
+// The transforms of ah_yz read and write each point some seventy times in LDS
+// (six derivatives of each component, forward and inverse in two stages), and
+// that bounds them.  Here psi and alpha psi are written to LDS once and read
+// twice, as the operands of tdw_planemm.hpp: one wave per component holds a
+// quarter of its plane and the three images (rows and columns past L / 2 of the
+// 16 x 16 tile are padding at 24: 44 % of the products, still the shorter
+// form).  1656 states of 24^3: 986 -> 870 us, 300 of 32^3 a whole step 1.18x
+// faster.  Two waves per SIMD (244 registers), the FP64 pipe (products and
+// sums) busy three quarters of the time; without the factors and tables loaded
+// ahead of the products that hide them it took 1227 us.
+// mt: second- and first-derivative tables of y, then of z (d_mmt).
+// The tiles of a wave's points: row image h, column image g, offset i in the
+// plane and j in its LDS copy; rows are 4 apart, R of them inside the tile.
+#define MM_TILES(h, g, i, j)                                                                     \
+    _Pragma("unroll") for (int h = 0; h < 2; h++)                                                \
+        _Pragma("unroll") for (int g = 0; g < 2; g++)                                            \
+            if (int i = i0 + h * H * L + g * H, j = j0 + h * H * RS + g * H; mm_tile(i, j))
+
+template <int L>
+__global__ void __launch_bounds__(128, 2)
+ah_yz_mm(const double2 *__restrict__ y, const double2 *__restrict__ T, double2 *__restrict__ out,
+         const double *__restrict__ pots, const double *__restrict__ hx, int n, long N, int NX,
+         const double *__restrict__ mt, double mu_a, double mu_b, double *__restrict__ part,
+         const double *__restrict__ sc)
+{
+    constexpr int H = L / 2, RS = L + 1, E = L * L, EP = L * RS, R = (H + 3) / 4, NT = 128, MT = (L / 8) * 128;
+    static_assert(H % 4 == 0 && H <= 16, "one 16 x 16 tile per quarter plane");
+    __shared__ double red[NT / 64];
+    extern __shared__ double2 lds_raw[];
+    double2 *A = lds_raw, *B = lds_raw + 2 * EP;
+    const int tid = threadIdx.x, lane = tid & 63, cmp = tid >> 6;
+    const int a = blockIdx.x / NX;
+    const int x = blockIdx.x - a * NX;
+    const long g0 = (long)x * E, gu = (long)a * N + g0, gv = ((long)n + a) * N + g0;
+    const double ys = sc ? sc[a] : 1.0;
+    // all loads first; points past the plane's end repeat its last one
+    constexpr int KM = (E + NT - 1) / NT;
+    double2 xu[KM], xv[KM];
+    double xa[KM], xb[KM];
+#pragma unroll
+    for (int k = 0; k < KM; k++) {
+        const int e = min(tid + k * NT, E - 1);
+        xu[k] = y[gu + e];
+        xv[k] = y[gv + e];
+        xa[k] = pots[4 * N + g0 + e];
+        xb[k] = pots[5 * N + g0 + e];
+    }
+    const int lr = lane >> 4, lc = lane & 15, cl = lc < H ? lc : H - 1;
+    const int i0 = lr * L + cl, j0 = lr * RS + cl;
+    const long own = cmp ? gv : gu;
+    const double2 *X = A + cmp * EP, *Y = A + (1 - cmp) * EP, *XA = B + cmp * EP;
+    const double *al = pots + (4 + cmp) * N + g0;
+    const double q = cmp ? 0.25 : -0.25;
+    dbl4 ore[2][2], oim[2][2];
+    const double2 *Tp = T + own;
+#pragma unroll
+    for (int h = 0; h < 2; h++)
+#pragma unroll
+        for (int g = 0; g < 2; g++) {
+            ore[h][g] = oim[h][g] = dbl4{0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+            for (int r = 0; r < R; r++) {
+                const double2 t = Tp[i0 + (h * H + 4 * r) * L + g * H];
+                ore[h][g][r] = t.x;
+                oim[h][g][r] = t.y;
+            }
+        }
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int k = 0; k < KM; k++) {
+        const int e = min(tid + k * NT, E - 1), pe = e + e / L;
+        const double2 u = xu[k] * ys, v = xv[k] * ys;
+        A[pe] = u;
+        A[EP + pe] = v;
+        B[pe] = u * xa[k];
+        B[EP + pe] = v * xb[k];
+    }
+    MmTab<H> t2, t1;   // of the second and the first derivative
+    mm_load<H>(mt + lane, t2);
+    mm_load<H>(mt + MT + lane, t1);
+    __syncthreads();
+    MmAcc acc;
+    // the points' factors, loaded ahead of the products that hide the wait
+    double fa[2][2][R], fd[2][2][R];
+    auto load = [&](const double *src, double (&f)[2][2][R]) {
+        int i = i0;
+        asm volatile("" : "+v"(i));
+#pragma unroll
+        for (int h = 0; h < 2; h++)
+#pragma unroll
+            for (int g = 0; g < 2; g++)
+#pragma unroll
+                for (int r = 0; r < R; r++) f[h][g][r] = src[i + (h * H + 4 * r) * L + g * H];
+        __builtin_amdgcn_sched_barrier(0);
+    };
+    load(al, fa);
+    load(pots + (7 + 3 * cmp) * N + g0, fd);
+#pragma unroll
+    for (int ax = 0; ax < 2; ax++) {
+        const int xo = ax ? cl * RS + lr : lr * RS + cl;
+        // psi: second derivative
+        if (ax) mm_product<false, H, RS, H>(X + xo, t2, acc);
+        else mm_product<true, H, RS, H>(X + xo, t2, acc);
+#pragma unroll
+        for (int h = 0; h < 2; h++)
+#pragma unroll
+            for (int g = 0; g < 2; g++) {
+                const dbl4 re = ax ? mm_inner_at(acc, h, g, 0) : mm_outer_at(acc, h, g, 0);
+                const dbl4 im = ax ? mm_inner_at(acc, h, g, 1) : mm_outer_at(acc, h, g, 1);
+#pragma unroll
+                for (int r = 0; r < R; r++) {
+                    const double f = q * fa[h][g][r];
+                    ore[h][g][r] += f * re[r];
+                    oim[h][g][r] += f * im[r];
+                }
+                mm_keep(ore[h][g]);
+                mm_keep(oim[h][g]);
+            }
+        // first derivative, -i A_d d_d psi
+        __builtin_amdgcn_sched_barrier(0);
+        if (ax) mm_product<false, H, RS, H>(X + xo, t1, acc);
+        else mm_product<true, H, RS, H>(X + xo, t1, acc);
+#pragma unroll
+        for (int h = 0; h < 2; h++)
+#pragma unroll
+            for (int g = 0; g < 2; g++) {
+                const dbl4 re = ax ? mm_inner_at(acc, h, g, 0) : mm_outer_at(acc, h, g, 0);
+                const dbl4 im = ax ? mm_inner_at(acc, h, g, 1) : mm_outer_at(acc, h, g, 1);
+#pragma unroll
+                for (int r = 0; r < R; r++) {
+                    ore[h][g][r] += fd[h][g][r] * im[r];
+                    oim[h][g][r] -= fd[h][g][r] * re[r];
+                }
+                mm_keep(ore[h][g]);
+                mm_keep(oim[h][g]);
+            }
+        // alpha psi: second derivative
+        __builtin_amdgcn_sched_barrier(0);
+        MmTab<H> tn = t2;
+        if (!ax) {
+            // the inner axis' factors and tables
+            load(pots + (8 + 3 * cmp) * N + g0, fd);
+            mm_load<H>(mt + 2 * MT + lane, tn);
+            mm_load<H>(mt + 3 * MT + lane, t1);
+            __builtin_amdgcn_sched_barrier(0);
+        }
+        if (ax) mm_product<false, H, RS, H>(XA + xo, t2, acc);
+        else mm_product<true, H, RS, H>(XA + xo, t2, acc);
+        t2 = tn;
+#pragma unroll
+        for (int h = 0; h < 2; h++)
+#pragma unroll
+            for (int g = 0; g < 2; g++) {
+                ore[h][g] += (ax ? mm_inner_at(acc, h, g, 0) : mm_outer_at(acc, h, g, 0)) * q;
+                oim[h][g] += (ax ? mm_inner_at(acc, h, g, 1) : mm_outer_at(acc, h, g, 1)) * q;
+                mm_keep(ore[h][g]);
+                mm_keep(oim[h][g]);
+            }
+    }
+    // the pointwise terms, the partner component and <psi|H psi>
+    const double *V = pots + cmp * N + g0, *lap = hx + cmp * N + g0, *dva = hx + (2 + cmp) * N + g0;
+    const double2 *D = (const double2 *)(pots + 2 * N) + g0;
+    const double mu = cmp ? mu_b : mu_a, sg = cmp ? -1.0 : 1.0;
+    double2 *op = out + own;
+    double ssum = 0.0;
+    // half of the points at a time, all of a half's loads first
+#pragma unroll
+    for (int h = 0; h < 2; h++) {
+        int i = i0 + h * H * L, j = j0 + h * H * RS;
+        mm_tile(i, j);
+        double fv[2][R], fl[2][R], fc[2][R];
+        double2 Dv[2][R];
+#pragma unroll
+        for (int g = 0; g < 2; g++)
+#pragma unroll
+            for (int r = 0; r < R; r++) {
+                const int ir = i + g * H + 4 * r * L;
+                fv[g][r] = V[ir];
+                fl[g][r] = lap[ir];
+                fc[g][r] = dva[ir];
+                Dv[g][r] = D[ir];
+            }
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int g = 0; g < 2; g++)
+#pragma unroll
+            for (int r = 0; r < R; r++) {
+                const int ir = i + g * H + 4 * r * L, jr = j + g * H + 4 * r * RS;
+                const double2 px = X[jr], py = Y[jr];
+                double2 t = cmul(px, make_double2(sg * (fv[g][r] - mu + 0.25 * fl[g][r]), -0.5 * fc[g][r]));
+                t = t + cmul(py, make_double2(Dv[g][r].x, sg * Dv[g][r].y));
+                t = t + make_double2(ore[h][g][r], oim[h][g][r]);
+                if (lc < H) {
+                    op[ir] = t;
+                    ssum += cmulc(px, t).x;
+                }
+            }
+    }
+    ssum = block_sum(ssum, red);
+    if (tid == 0) part[blockIdx.x] = ssum;
+}
+
 // ---------------------------------------------------------------------------
 // Densities with gradients without storing the gradients: an x pass and a
 // yz pass over the state, each workgroup looping over a chunk of G states
@@ -418,6 +622,113 @@ dg_yz(const ac_t<SP> *__restrict__ y, const double *__restrict__ fbeta, const do
     }
 }
 
+// The same for FP64 planes of 24 or 32 points a side on the matrix cores (as
+// ah_yz_mm): a wave per (chunk, x plane, component), the next state's plane
+// loaded while the products of this one run.  1656 states of 24^3: 548 ->
+// 474 us, bound by the FP64 pipe and its two waves per SIMD (256 registers).
+template <int L>
+__global__ void __launch_bounds__(64, 2)
+dg_yz_mm(const double2 *__restrict__ y, const double *__restrict__ fbeta, const double *__restrict__ wgt, int n, long N,
+         int NX, int G, const double *__restrict__ mt, double *__restrict__ part)
+{
+    constexpr int H = L / 2, RS = L + 1, E = L * L, EP = L * RS, R = (H + 3) / 4, KM = E / 64, MT = (L / 8) * 128;
+    static_assert(H % 4 == 0 && H <= 16 && E % 64 == 0, "one 16 x 16 tile per quarter plane");
+    __shared__ double2 X[EP];
+    const int lane = threadIdx.x;
+    const int cmp = blockIdx.x & 1, blk = blockIdx.x >> 1;
+    const int ch = blk / NX;
+    const int x = blk - ch * NX;
+    const int a0 = ch * G, a1 = min(n, a0 + G);
+    const long g0 = (long)x * E, gc = cmp ? (long)n * N + g0 : g0;
+    const int lr = lane >> 4, lc = lane & 15, cl = lc < H ? lc : H - 1;
+    const int i0 = lr * L + cl, j0 = lr * RS + cl;
+    double ta[2][2][R], jy[2][2][R], jz[2][2][R];
+#pragma unroll
+    for (int h = 0; h < 2; h++)
+#pragma unroll
+        for (int g = 0; g < 2; g++)
+#pragma unroll
+            for (int r = 0; r < R; r++) ta[h][g][r] = jy[h][g][r] = jz[h][g][r] = 0.0;
+    double2 nx[KM];
+#pragma unroll
+    for (int k = 0; k < KM; k++) nx[k] = a0 < a1 ? y[gc + (long)a0 * N + lane + 64 * k] : make_double2(0.0, 0.0);
+    for (int a = a0; a < a1; a++) {
+        const double fb = fbeta[a] * 10000.;
+        double w = cmp ? 10000. - fb : fb;
+        if (wgt) w *= wgt[a];
+        const double wj = cmp ? -w : w;
+        __syncthreads();
+#pragma unroll
+        for (int k = 0; k < KM; k++) {
+            const int e = lane + 64 * k;
+            X[e + e / L] = nx[k];
+        }
+        __syncthreads();
+        if (a + 1 < a1) {
+            const double2 *yn = y + gc + (long)(a + 1) * N + lane;
+#pragma unroll
+            for (int k = 0; k < KM; k++) nx[k] = yn[64 * k];
+        }
+        MmAcc acc;
+#pragma unroll
+        for (int ax = 0; ax < 2; ax++) {
+            const double *m2 = mt + 2 * ax * MT + lane, *m1 = m2 + MT;
+            const int xo = ax ? cl * RS + lr : lr * RS + cl;
+            __builtin_amdgcn_sched_barrier(0);
+            if (ax) mm_product<false, H, RS, H>(X + xo, m2, acc);
+            else mm_product<true, H, RS, H>(X + xo, m2, acc);
+            MM_TILES(h, g, i, j) {
+                const dbl4 re = ax ? mm_inner_at(acc, h, g, 0) : mm_outer_at(acc, h, g, 0);
+                const dbl4 im = ax ? mm_inner_at(acc, h, g, 1) : mm_outer_at(acc, h, g, 1);
+#pragma unroll
+                for (int r = 0; r < R; r++) {
+                    ta[h][g][r] += cmulc(X[j + 4 * r * RS], make_double2(re[r], im[r])).x * w;
+                    mm_keep(ta[h][g][r]);
+                }
+            }
+            __builtin_amdgcn_sched_barrier(0);
+            if (ax) mm_product<false, H, RS, H>(X + xo, m1, acc);
+            else mm_product<true, H, RS, H>(X + xo, m1, acc);
+            MM_TILES(h, g, i, j) {
+                const dbl4 re = ax ? mm_inner_at(acc, h, g, 0) : mm_outer_at(acc, h, g, 0);
+                const dbl4 im = ax ? mm_inner_at(acc, h, g, 1) : mm_outer_at(acc, h, g, 1);
+#pragma unroll
+                for (int r = 0; r < R; r++) {
+                    const double v = cmulc(X[j + 4 * r * RS], make_double2(re[r], im[r])).y * wj;
+                    double &t = ax ? jz[h][g][r] : jy[h][g][r];
+                    t += v;
+                    mm_keep(t);
+                }
+            }
+        }
+    }
+    if (lc >= H) return;
+    double *p = part + (long)ch * 6 * N + g0;
+    MM_TILES(h, g, i, j) {
+#pragma unroll
+        for (int r = 0; r < R; r++) {
+            const int ir = i + 4 * r * L;
+            p[cmp * N + ir] = ta[h][g][r];
+            p[(2 + 2 * cmp) * N + ir] = jy[h][g][r];
+            p[(3 + 2 * cmp) * N + ir] = jz[h][g][r];
+        }
+    }
+}
+#undef MM_TILES
+
+// FP64 planes of the matrix-core forms, and their tables
+static bool amm_plane(const tdw_ctx *c) { return c->dim == 3 && c->ny == c->nz && (c->ny == 24 || c->ny == 32); }
+
+int aslda_setup(tdw_ctx *c)
+{
+    if (!amm_plane(c)) return 0;
+    std::vector<double> t;
+    for (int d = 1; d < 3; d++)
+        for (int order = 2; order > 0; order--) mm_tables(c->ny, c->Lphys[d], order, t);
+    TDW_HIP(hipMalloc(&c->d_mmt, sizeof(double) * t.size()));
+    return (int)hipMemcpy(c->d_mmt, t.data(), sizeof(double) * t.size(), hipMemcpyHostToDevice);
+}
+
 template <bool SP> struct AFns {
     typedef ac_t<SP> C;
     typedef void (*ahx_fn)(const C *, C *, const double *, int, long, int, const C *, double, double, const double *);
@@ -540,8 +851,17 @@ static int dens_grad_t(tdw_ctx *c, int n, const ac_t<SP> *wf, const double *fbet
     const size_t lds = sizeof(typename F::C) * 4 * (size_t)c->ny * (c->nz + 1);
     const double k1y = 2.0 * M_PI / c->Lphys[1] / c->ny, k2y = pow(2.0 * M_PI / c->Lphys[1], 2) / c->ny;
     const double k1z = 2.0 * M_PI / c->Lphys[2] / c->nz, k2z = pow(2.0 * M_PI / c->Lphys[2], 2) / c->nz;
-    hipLaunchKernelGGL(fy, dim3((unsigned)((long)nchunk * c->nx)), dim3(nt), lds, c->stream, wf, fbeta, wgt, n, N,
-                       c->nx, G, F::tw(c, 1), F::tw(c, 2), k1y, k2y, k1z, k2z, pyz_part);
+    bool mm = false;
+    if constexpr (!SP)
+        if (c->d_mmt) {
+            mm = true;
+            const auto fm = c->ny == 24 ? dg_yz_mm<24> : dg_yz_mm<32>;
+            hipLaunchKernelGGL(fm, dim3((unsigned)(2L * nchunk * c->nx)), dim3(64), 0, c->stream, wf, fbeta, wgt, n, N,
+                               c->nx, G, c->d_mmt, pyz_part);
+        }
+    if (!mm)
+        hipLaunchKernelGGL(fy, dim3((unsigned)((long)nchunk * c->nx)), dim3(nt), lds, c->stream, wf, fbeta, wgt, n, N,
+                           c->nx, G, F::tw(c, 1), F::tw(c, 2), k1y, k2y, k1z, k2z, pyz_part);
     TDW_TRY((int)hipGetLastError());
     const ChunkSrc fx_src{px_part, 8, {2, 3, 0, 4, 6, -1, -1, 1, 5, 7, -1, -1}};
     const ChunkSrc fy_src{pyz_part, 6, {-1, -1, -1, 0, -1, 2, 3, -1, 1, -1, 4, 5}};
@@ -589,6 +909,13 @@ static int aslda_h_t(tdw_ctx *c, int n, const ac_t<SP> *in, ac_t<SP> *out, ac_t<
         const size_t lds = sizeof(typename F::C) * 4 * (size_t)c->ny * (c->nz + 1);
         const double k1y = 2.0 * M_PI / c->Lphys[1] / c->ny, k2y = pow(2.0 * M_PI / c->Lphys[1], 2) / c->ny;
         const double k1z = 2.0 * M_PI / c->Lphys[2] / c->nz, k2z = pow(2.0 * M_PI / c->Lphys[2], 2) / c->nz;
+        if constexpr (!SP)
+            if (c->d_mmt) {
+                const auto fm = c->ny == 24 ? ah_yz_mm<24> : ah_yz_mm<32>;
+                hipLaunchKernelGGL(fm, dim3((unsigned)((long)n * c->nx)), dim3(128), lds, c->stream, in, T, out, pots,
+                                   hx, n, N, c->nx, c->d_mmt, c->p.mu_a, c->p.mu_b, part, sc);
+                return row_sums(c, part, n, c->nx, dvol_norm(c), d_qpe);
+            }
         hipLaunchKernelGGL(fy, dim3((unsigned)((long)n * c->nx)), dim3(nt), lds, c->stream, in, T, out, pots, hx, n, N,
                            c->nx, F::tw(c, 1), F::tw(c, 2), k1y, k2y, k1z, k2z, c->p.mu_a, c->p.mu_b, part, sc);
         TDW_TRY(row_sums(c, part, n, c->nx, dvol_norm(c), d_qpe));

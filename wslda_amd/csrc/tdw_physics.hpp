@@ -186,6 +186,9 @@ int abm4q(tdw_ctx *c, int n, const double2 *hy, double2 *y, const double2 *fl, c
 // hx the grid fields of aslda_fields, part n*NX doubles; with sc (n
 // per-state factors) H acts on sc_a in_a
 bool aslda_h_fused_supported(const tdw_ctx *c);
+// tables of the context's yz planes (tdw_create), none where they have no
+// matrix-core form
+int aslda_setup(tdw_ctx *c);
 // hx = [lap alpha_a, lap alpha_b, div A_a, div A_b] of the potentials into c->d_hx
 int aslda_fields(tdw_ctx *c, const double *pots);
 int aslda_h_fused(tdw_ctx *c, int n, const double2 *in, double2 *out, double2 *T, const double *pots,

@@ -27,6 +27,7 @@
 #include "tdw_internal.hpp"
 #include "tdw_physics.hpp"
 #include "tdw_resident.hpp"
+#include "tdw_planemm.hpp"
 #include "tdw_rsfft.hpp"
 
 #include <algorithm>
@@ -200,17 +201,11 @@ rs_h(const double2 *in, double2 *out, const double2 *__restrict__ c, const doubl
 // The same for 2D planes of 32 or 64 points a side, on the matrix cores.
 //
 // The transforms of rs_h read and write the state seven times in LDS, behind
-// as many barriers, and one 64 x 64 state occupies a CU alone.  The second
-// derivative along an axis of L points is a circulant L x L matrix, real and
-// even; with p = x_j + x_{j + L/2}, m = x_j - x_{j + L/2} it falls into two
-// L/2 x L/2 products, P p and M m (y_i = P p + M m, y_{i + L/2} = P p - M m),
-// contractions for v_mfma_f64_16x16x4.  A wave owns the points (ix, iy) of
-// one component with ix in a 16-row tile or that plus LX/2, iy in a tile or
-// that plus LY/2.  d^2/dx^2 takes the matrix as the A operand and the plane as
-// B, d^2/dy^2 the plane as A and the matrix as B, so both leave the wave's own
-// points in the same registers (row lane / 16 + 4 r, column lane % 16): the
-// plane is written to LDS once, read four times over, never overwritten, and
-// all that follows (H psi, <H>, corrector, norm) stays in registers.
+// as many barriers, and one 64 x 64 state occupies a CU alone.  Here the second
+// derivatives are the products of tdw_planemm.hpp: a wave owns the points
+// (ix, iy) of one component with ix in a 16-row tile or that plus LX/2, iy in a
+// tile or that plus LY/2, and all that follows (H psi, <H>, corrector, norm)
+// stays in its registers.
 // More multiplications (64 per point and component at 64 x 64) but no index
 // arithmetic and one barrier before H: at 64 x 64 the corrector form of 1024
 // states 169 -> 128 us, the plain one 141 -> 99, of 192 states 39 -> 28 and
@@ -218,16 +213,6 @@ rs_h(const double2 *in, double2 *out, const double2 *__restrict__ c, const doubl
 // at 64 x 64 (133 KB of LDS, 254 registers), bound by its load and store
 // phases, which nothing overlaps.
 // ---------------------------------------------------------------------------
-typedef double dbl4 __attribute__((ext_vector_type(4)));
-
-// a tile's offsets, opaque to the compiler; the previous tile is done with
-__device__ __forceinline__ bool mm_tile(int &i, int &j)
-{
-    __builtin_amdgcn_sched_barrier(0);
-    asm volatile("" : "+v"(i), "+v"(j));
-    return true;
-}
-
 template <int LX, int LY, int CORR>
 __global__ void __launch_bounds__(64 * 2 * (LX / 32) * (LY / 32), 2)
 rs_mm(const double2 *in, double2 *out, const double2 *__restrict__ c, const double *__restrict__ pots,
@@ -253,65 +238,24 @@ rs_mm(const double2 *in, double2 *out, const double2 *__restrict__ c, const doub
     // lap[h][g]: points (ix + h HX, iy + g HY), four rows each; re and im
     dbl4 lre[2][2], lim[2][2];
     __syncthreads();
-    // along x: the matrix times the plane, columns iy
-    {
-        const double *M = mx + (long)tx * (HX / 4) * 128 + lane;
-        dbl4 P[2][2], Q[2][2];   // [column tile][re, im]
+    MmAcc acc;
+    mm_product<true, HX, RS, HY>(X + lr * RS + 16 * ty + lc, mx + (long)tx * (HX / 4) * 128 + lane, acc);
 #pragma unroll
-        for (int g = 0; g < 2; g++)
-#pragma unroll
-            for (int q = 0; q < 2; q++) P[g][q] = Q[g][q] = dbl4{0.0, 0.0, 0.0, 0.0};
-#pragma unroll 2
-        for (int ks = 0; ks < HX / 4; ks++) {
-            const double mp = M[ks * 128], mm = M[ks * 128 + 64];
-            const double2 *x = X + (4 * ks + lr) * RS + 16 * ty + lc;
-#pragma unroll
-            for (int g = 0; g < 2; g++) {
-                const double2 u = x[g * HY], v = x[g * HY + HX * RS];
-                P[g][0] = __builtin_amdgcn_mfma_f64_16x16x4f64(mp, u.x + v.x, P[g][0], 0, 0, 0);
-                P[g][1] = __builtin_amdgcn_mfma_f64_16x16x4f64(mp, u.y + v.y, P[g][1], 0, 0, 0);
-                Q[g][0] = __builtin_amdgcn_mfma_f64_16x16x4f64(mm, u.x - v.x, Q[g][0], 0, 0, 0);
-                Q[g][1] = __builtin_amdgcn_mfma_f64_16x16x4f64(mm, u.y - v.y, Q[g][1], 0, 0, 0);
-            }
-        }
+    for (int h = 0; h < 2; h++)
 #pragma unroll
         for (int g = 0; g < 2; g++) {
-            lre[0][g] = P[g][0] + Q[g][0];
-            lim[0][g] = P[g][1] + Q[g][1];
-            lre[1][g] = P[g][0] - Q[g][0];
-            lim[1][g] = P[g][1] - Q[g][1];
+            lre[h][g] = mm_outer_at(acc, h, g, 0);
+            lim[h][g] = mm_outer_at(acc, h, g, 1);
         }
-    }
     __builtin_amdgcn_sched_barrier(0);
-    // along y: the plane times the matrix, rows ix
-    {
-        const double *M = my + (long)ty * (HY / 4) * 128 + lane;
-        dbl4 P[2][2], Q[2][2];   // [row tile][re, im]
+    mm_product<false, HY, RS, HX>(X + (16 * tx + lc) * RS + lr, my + (long)ty * (HY / 4) * 128 + lane, acc);
 #pragma unroll
-        for (int h = 0; h < 2; h++)
+    for (int h = 0; h < 2; h++)
 #pragma unroll
-            for (int q = 0; q < 2; q++) P[h][q] = Q[h][q] = dbl4{0.0, 0.0, 0.0, 0.0};
-#pragma unroll 2
-        for (int ks = 0; ks < HY / 4; ks++) {
-            const double mp = M[ks * 128], mm = M[ks * 128 + 64];
-            const double2 *x = X + (16 * tx + lc) * RS + 4 * ks + lr;
-#pragma unroll
-            for (int h = 0; h < 2; h++) {
-                const double2 u = x[h * HX * RS], v = x[h * HX * RS + HY];
-                P[h][0] = __builtin_amdgcn_mfma_f64_16x16x4f64(u.x + v.x, mp, P[h][0], 0, 0, 0);
-                P[h][1] = __builtin_amdgcn_mfma_f64_16x16x4f64(u.y + v.y, mp, P[h][1], 0, 0, 0);
-                Q[h][0] = __builtin_amdgcn_mfma_f64_16x16x4f64(u.x - v.x, mm, Q[h][0], 0, 0, 0);
-                Q[h][1] = __builtin_amdgcn_mfma_f64_16x16x4f64(u.y - v.y, mm, Q[h][1], 0, 0, 0);
-            }
+        for (int g = 0; g < 2; g++) {
+            lre[h][g] += mm_inner_at(acc, h, g, 0);
+            lim[h][g] += mm_inner_at(acc, h, g, 1);
         }
-#pragma unroll
-        for (int h = 0; h < 2; h++) {
-            lre[h][0] += P[h][0] + Q[h][0];
-            lim[h][0] += P[h][1] + Q[h][1];
-            lre[h][1] += P[h][0] - Q[h][0];
-            lim[h][1] += P[h][1] - Q[h][1];
-        }
-    }
     const double k2t = kt ? kt[a] * kt[a] : 0.0;
     const long own = cmp ? gv : gu;
     const double *V = pots + cmp * N, *al = pots + (4 + cmp) * N;
@@ -452,26 +396,7 @@ int resident_setup(tdw_ctx *c)
     }
     // the halves of the second-derivative circulants in rs_mm's operand order
     if (mm_plane(c))
-        for (int d = 0; d < 2; d++) {
-            const int L = len[d], H = L / 2;
-            // summed in extended precision, else the rounding of the sums (not
-            // that of the entries) is what the operator differs by
-            std::vector<long double> cs(L), cc(L, 0.0L);
-            for (int t = 0; t < L; t++) cs[t] = cosl(2.0L * 3.141592653589793238462643383L * t / L);
-            for (int x = 0; x < L; x++)
-                for (int f = 0; f < L; f++) {
-                    const long double k = rs_k(f, L, c->Lphys[d]);
-                    cc[x] -= k * k / L * cs[(f * x) % L];
-                }
-            for (int t = 0; t < H / 16; t++)
-                for (int ks = 0; ks < H / 4; ks++)
-                    for (int pm = 0; pm < 2; pm++)
-                        for (int l = 0; l < 64; l++) {
-                            const int x = 16 * t + l % 16 - (4 * ks + l / 16) + L;
-                            const long double v = cc[x % L], h = cc[(x + H) % L];
-                            kt.push_back((double)(0.5L * (pm ? v - h : v + h)));
-                        }
-        }
+        for (int d = 0; d < 2; d++) mm_tables(len[d], c->Lphys[d], 2, kt);
     const size_t btw = sizeof(double2) * tw.size(), bk = sizeof(double) * kt.size();
     TDW_HIP(hipMalloc(&c->d_rtab, btw + bk));
     TDW_HIP(hipMemcpy(c->d_rtab, tw.data(), btw, hipMemcpyHostToDevice));
@@ -521,7 +446,7 @@ static int launch_h(tdw_ctx *c, int n, const double2 *in, double2 *out, const do
     TDW_TIMED(c, CORR ? "rs_hcorr" : "rs_h");
     if (mm_plane(c)) {
         const double *mx = kx + pl.ax[0].L + pl.inner;
-        const double *my = mx + (size_t)(c->nx / 32) * (c->nx / 8) * 128;
+        const double *my = mx + mm_doubles(c->nx);
         const dim3 g(n), b(128 * (c->nx / 32) * (c->ny / 32));
         const size_t sm = sizeof(double2) * 2 * (size_t)pl.npc;
 #define RS_MM(LX, LY)                                                                                               \
