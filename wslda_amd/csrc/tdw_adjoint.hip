@@ -18,6 +18,7 @@
 #include "tdw_internal.hpp"
 #include "tdw_physics.hpp"
 #include "tdw_resident.hpp"
+#include <algorithm>
 
 namespace tdw {
 
@@ -53,6 +54,12 @@ static AbmCoef abm_coef(int scheme)
         k.a0 = 251. / 720.;
     }
     return k;
+}
+
+__global__ void k_copy_d(const double *__restrict__ s, double *__restrict__ d, long n)
+{
+    const long i = (long)blockIdx.x * AT + threadIdx.x;
+    if (i < n) d[i] = s[i];
 }
 
 // ---------------------------------------------------------------------------
@@ -163,33 +170,28 @@ __global__ void k_cross_final(const double *__restrict__ part, int nchunk, long 
 }
 
 // ---------------------------------------------------------------------------
-// transpose of the potential update at one point: dual numbers over the
-// inputs (rho_a, rho_b, Re nu, Im nu, u_a, u_b, Va_prev, Vb_prev); lU holds
+// transpose of the potential update at one point (ad::slda_vjp); lU holds
 // dL/d(Va, Vb, Re D, Im D) in 4 planes of N.  Also accumulates dL/dtheta of
-// the Gaussian parameters through u_a, u_b (block partials).
+// the Gaussian parameters through u_a, u_b (block partials of the parameters
+// in use).  A serial chain of divisions and logarithms over the 15 mixing
+// steps bounds it: 64 x 64 points 51 -> 37 us with four tangents through the
+// loop instead of eight and the sums of the Gaussians in use only.
 // ---------------------------------------------------------------------------
 __global__ void __launch_bounds__(AT)
 k_pot_vjp(FParams f, VextDev V, long N, const double *__restrict__ dens, const double *__restrict__ pots_prev,
           const double *__restrict__ lU, const double *__restrict__ dens_add, double *__restrict__ lD,
           double *__restrict__ lUprev, double *__restrict__ gpart)
 {
-    typedef Dual<8> D8;
     __shared__ double red[AT / 64];
     const long i = (long)blockIdx.x * blockDim.x + threadIdx.x;
     double lua = 0.0, lub = 0.0;
     if (i < N) {
         double ua, ub;
         vext_point(V, i, ua, ub);
-        const D8 na = dvar<8>(dens[2 * N + i], 0), nb = dvar<8>(dens[7 * N + i], 1);
-        const Cx<D8> nu = cx<D8>(dvar<8>(dens[2 * i], 2), dvar<8>(dens[2 * i + 1], 3));
-        const D8 dua = dvar<8>(ua, 4), dub = dvar<8>(ub, 5);
-        D8 Va = dvar<8>(pots_prev[i], 6), Vb = dvar<8>(pots_prev[N + i], 7);
-        Cx<D8> del;
-        ad::slda_point(f, na, nb, nu, dua, dub, Va, Vb, del);
-        const double l0 = lU[i], l1 = lU[N + i], l2 = lU[2 * N + i], l3 = lU[3 * N + i];
+        const double l[4] = {lU[i], lU[N + i], lU[2 * N + i], lU[3 * N + i]};
         double g[8];
-#pragma unroll
-        for (int k = 0; k < 8; k++) g[k] = l0 * Va.d[k] + l1 * Vb.d[k] + l2 * del.x.d[k] + l3 * del.y.d[k];
+        ad::slda_vjp(f, dens[2 * N + i], dens[7 * N + i], dens[2 * i], dens[2 * i + 1], ua, ub, pots_prev[i],
+                     pots_prev[N + i], l, g);
         double d0 = g[0], d1 = g[1], d2 = g[2], d3 = g[3];
         if (dens_add) {
             d0 += dens_add[i];
@@ -215,9 +217,9 @@ k_pot_vjp(FParams f, VextDev V, long N, const double *__restrict__ dens, const d
     const double y = V.dim >= 2 ? V.dy * (iy - V.ny / 2) : 0.0;
     const double z = V.dim >= 3 ? V.dz * (iz - V.nz / 2) : 0.0;
     const double lg = lua + (V.v.flip_b ? -lub : lub);   // dL/dg, g = the Gaussian sum
-    for (int k = 0; k < TDW_MAX_GAUSS; k++) {
+    for (int k = 0; k < min(V.v.ngauss, TDW_MAX_GAUSS); k++) {
         double t[7] = {0, 0, 0, 0, 0, 0, 0};
-        if (k < V.v.ngauss && i < N) {
+        if (i < N) {
             const double X = x - V.v.cx[k], Y = y - V.v.cy[k], Z = z - V.v.cz[k];
             const double E = V.s * exp(V.v.wx[k] * (X * X) + V.v.wy[k] * (Y * Y) + V.v.wz[k] * (Z * Z));
             const double A = V.v.amp[k];
@@ -507,12 +509,6 @@ k_hist_dt(double2 *ly, const double2 *__restrict__ w1, const double2 *__restrict
     }
 }
 
-__global__ void k_copy_d(const double *__restrict__ s, double *__restrict__ d, long n)
-{
-    const long i = (long)blockIdx.x * AT + threadIdx.x;
-    if (i < n) d[i] = s[i];
-}
-
 // ---------------------------------------------------------------------------
 // host side
 // ---------------------------------------------------------------------------
@@ -564,7 +560,8 @@ static int pot_vjp(tdw_ctx *c, int it, const double *dens, const double *pots_pr
     TDW_TRY(ensure_part(c, (size_t)nblk * NTHETA));
     hipLaunchKernelGGL(k_pot_vjp, dim3(nblk), dim3(PT), 0, c->stream, fparams(c), make_vext(c, it), N, dens,
                        pots_prev, lU, dens_add, lD, lUprev, c->d_part);
-    hipLaunchKernelGGL(k_gsum, dim3(NTHETA), dim3(AT), 0, c->stream, c->d_part, nblk, theta_grad);
+    const int np = 7 * std::min(make_vext(c, it).v.ngauss, TDW_MAX_GAUSS);
+    if (np) hipLaunchKernelGGL(k_gsum, dim3(np), dim3(AT), 0, c->stream, c->d_part, nblk, theta_grad);
     return (int)hipGetLastError();
 }
 

@@ -114,39 +114,70 @@ __host__ __device__ __forceinline__ R mf_corr(const FParams &f, const R &p0x, co
     return S<R>::c(0.0);
 }
 
-// SLDA potentials at one point; Va, Vb enter as the previous potentials (the
-// start of the 15-step mixing loop) and leave as the new ones.
-template <typename R>
-__host__ __device__ __forceinline__ void slda_point(const FParams &f, const R &na, const R &nb, const Cx<R> &nu,
-                                                    const R &ua, const R &ub, R &Va, R &Vb, Cx<R> &delta)
+// Transpose of the SLDA potentials at one point: l = dL/d(Va, Vb, Re delta,
+// Im delta) to gr = dL/d(na, nb, Re nu, Im nu, ua, ub, Va_prev, Vb_prev).
+//
+// The 15-step mixing loop reaches its inputs through four of them only: c =
+// Va_const + Vb_const, n = na + nb, |nu|^2 and s0 = Va_prev + Vb_prev.  Both
+// potentials receive the same X(Va + Vb) per step, so with Y the mixed sum of
+// the X, Va = A Va_prev + (1 - A) Va_const + Y with A = (1 - mix)^15, and four
+// tangents of Va + Vb, Y and g carry the loop instead of eight of each
+// variable.  The loop's values are those of the potentials' own update, so it
+// takes the branches that update took.
+__host__ __device__ __forceinline__ void slda_vjp(const FParams &f, double na, double nb, double nux, double nuy,
+                                                  double ua, double ub, double Va, double Vb, const double (&l)[4],
+                                                  double (&gr)[8])
 {
+    typedef Dual<4> D;
     const double alph_plus = TDW_A0;
-    R Va_const = ua + der_funD(f, na, nb, 0);
-    R Vb_const = ub + der_funD(f, na, nb, 1);
-    const R t3 = der_tildeC(f, na, nb) / alph_plus;
-    const R t5 = tildeC(f, na, nb);
-    R lkF = S<R>::c(0.0);
-    if (f.mf) lkF = ad_pow(3.0 * M_PI * M_PI * (na + nb), 1.0 / 3.0);
-    R g = S<R>::c(0.0);
-    const R nu2 = nu.x * nu.x + nu.y * nu.y;
+    const Dual<2> ea = dvar<2>(na, 0), eb = dvar<2>(nb, 1);
+    const Dual<2> fa = der_funD(f, ea, eb, 0), fb = der_funD(f, ea, eb, 1);
+    const double Va_const = ua + fa.v, Vb_const = ub + fb.v;
+    // tangents: 0 c, 1 n, 2 |nu|^2, 3 s0
+    const D dn = dvar<4>(na + nb, 1), z = dconst<4>(0.0);
+    const D t3 = der_tildeC(f, dn, z) / alph_plus;
+    const D t5 = tildeC(f, dn, z);
+    D lkF = z;
+    if (f.mf) lkF = ad_pow(3.0 * M_PI * M_PI * dn, 1.0 / 3.0);
+    const D nu2 = dvar<4>(nux * nux + nuy * nuy, 2);
+    D g = z, Y = z;
+    double sd[4] = {0.0, 0.0, 0.0, 1.0};   // of Va + Vb
+    double A = 1.0;
     for (int k = 0; k < TDW_UD_SCITERS; k++) {
-        R t7 = (f.mu_a - Va + f.mu_b - Vb) / 2.0;
-        Cx<R> wz, p0;
+        D t7;
+        t7.v = (f.mu_a - Va + f.mu_b - Vb) / 2.0;
+#pragma unroll
+        for (int j = 0; j < 4; j++) t7.d[j] = -0.5 * sd[j];
+        Cx<D> wz, p0;
         const bool real = reg_wz(f, t7, alph_plus, wz, p0);
-        const R d = t5 - wz.x;
+        const D d = t5 - wz.x;
         g = real ? alph_plus / d : alph_plus * d / (d * d + wz.y * wz.y);
-        R t7b = (g * g) * nu2;
-        R Vanew = Va_const - t3 * t7b;
-        R Vbnew = Vb_const - t3 * t7b;
-        if (f.mf) {
-            R dl = mf_corr(f, p0.x, g, lkF, na + nb, alph_plus);
-            Vanew = Vanew + dl * t7b;
-            Vbnew = Vbnew + dl * t7b;
+        const D t7b = (g * g) * nu2;
+        D X = -(t3 * t7b);
+        if (f.mf) X = X + mf_corr(f, p0.x, g, lkF, dn, alph_plus) * t7b;
+        Va = TDW_UD_MIX * (Va_const + X.v) + (1.0 - TDW_UD_MIX) * Va;
+        Vb = TDW_UD_MIX * (Vb_const + X.v) + (1.0 - TDW_UD_MIX) * Vb;
+#pragma unroll
+        for (int j = 0; j < 4; j++) {
+            sd[j] = TDW_UD_MIX * (2.0 * X.d[j] + (j == 0 ? 1.0 : 0.0)) + (1.0 - TDW_UD_MIX) * sd[j];
+            Y.d[j] = TDW_UD_MIX * X.d[j] + (1.0 - TDW_UD_MIX) * Y.d[j];
         }
-        Va = TDW_UD_MIX * Vanew + (1.0 - TDW_UD_MIX) * Va;
-        Vb = TDW_UD_MIX * Vbnew + (1.0 - TDW_UD_MIX) * Vb;
+        A *= 1.0 - TDW_UD_MIX;
     }
-    delta = cx<R>(-nu.x * g, -nu.y * g);
+    // delta = -nu g
+    const double lY = l[0] + l[1], lg = -(l[2] * nux + l[3] * nuy);
+    double w[4];
+#pragma unroll
+    for (int j = 0; j < 4; j++) w[j] = lY * Y.d[j] + lg * g.d[j];
+    const double la = l[0] * (1.0 - A) + w[0], lb = l[1] * (1.0 - A) + w[0];
+    gr[0] = la * fa.d[0] + lb * fb.d[0] + w[1];
+    gr[1] = la * fa.d[1] + lb * fb.d[1] + w[1];
+    gr[2] = 2.0 * nux * w[2] - l[2] * g.v;
+    gr[3] = 2.0 * nuy * w[2] - l[3] * g.v;
+    gr[4] = la;
+    gr[5] = lb;
+    gr[6] = l[0] * A + w[3];
+    gr[7] = l[1] * A + w[3];
 }
 
 }  // namespace ad
