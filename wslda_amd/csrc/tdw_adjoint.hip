@@ -56,12 +56,6 @@ static AbmCoef abm_coef(int scheme)
     return k;
 }
 
-__global__ void k_copy_d(const double *__restrict__ s, double *__restrict__ d, long n)
-{
-    const long i = (long)blockIdx.x * AT + threadIdx.x;
-    if (i < n) d[i] = s[i];
-}
-
 // ---------------------------------------------------------------------------
 // per-state sums: part[a * gridDim.x + blk] over a chunk of points
 // ---------------------------------------------------------------------------
@@ -588,12 +582,6 @@ static int dens_t(tdw_ctx *c, int n, const double2 *psi, double2 *out, const dou
     return (int)hipGetLastError();
 }
 
-static int copy_d(tdw_ctx *c, const double *s, double *d, long n)
-{
-    hipLaunchKernelGGL(k_copy_d, dim3((n + AT - 1) / AT), dim3(AT), 0, c->stream, s, d, n);
-    return (int)hipGetLastError();
-}
-
 // points per thread of the fused one-workgroup-per-state kernels; 0: the
 // state does not fit one workgroup (the separate passes run)
 static int fused_kp(long N)
@@ -686,9 +674,8 @@ static int adj_forward(tdw_ctx *c, tdw_state *s, int it, tdw_complex *y_out, dou
     if (!hT) TDW_TRY(laplace(c, 2 * n, D2(s->wf), D2(s->lap)));
     TDW_TRY(densities(c, n, D2(s->wf), nullptr, nullptr, nullptr, D2(s->lap), c->d_fbeta, nullptr, c->d_kt, c->d_cnt,
                       s->dens, 0));
-    TDW_TRY(copy_d(c, s->dens, t->dens_p, 12 * N));
     TDW_TRY(potentials(c, it + 1, s->dens, s->pots));
-    TDW_TRY(copy_d(c, s->pots, t->pots_p, 12 * N));
+    TDW_TRY(tape_fields(c, s->dens, t->dens_p, s->pots, t->pots_p));
     if (hT) TDW_TRY(fused_apply_h(c, n, D2(s->wf), D2(s->lap), hT, s->pots, t->scal + n));
     else TDW_TRY(apply_h(c, it + 1, n, D2(s->wf), D2(s->lap), CD2(s->lap), s->pots, c->d_kt, nullptr, t->scal + n));
     TDW_TRY(abm4(c, n, CD2(s->lap), D2(s->wf), flast));
@@ -696,9 +683,8 @@ static int adj_forward(tdw_ctx *c, tdw_state *s, int it, tdw_complex *y_out, dou
     if (!hT) TDW_TRY(laplace(c, 2 * n, D2(s->wf), D2(s->lap)));
     TDW_TRY(densities(c, n, D2(s->wf), nullptr, nullptr, nullptr, D2(s->lap), c->d_fbeta, nullptr, c->d_kt, c->d_cnt,
                       s->dens, 0));
-    TDW_TRY(copy_d(c, s->dens, t->dens_c, 12 * N));
     TDW_TRY(potentials(c, it + 1, s->dens, s->pots));
-    TDW_TRY(copy_d(c, s->pots, t->pots_c, 12 * N));
+    TDW_TRY(tape_fields(c, s->dens, t->dens_c, s->pots, t->pots_c));
     tdw_complex *tmp = f_next ? f_next : s->f[k - 1];
     for (int j = k - 1; j > 0; j--) s->f[j] = s->f[j - 1];
     s->f[0] = tmp;

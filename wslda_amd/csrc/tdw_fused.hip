@@ -856,11 +856,6 @@ static int hyz(tdw_ctx *c, int n, const hc_t<SP> *y, const hc_t<SP> *T, hc_t<SP>
 // in the tape's slots); cbuf: the partial corrector's buffer instead of the
 // oldest history entry (which then stays intact); f_next: the new history
 // entry's buffer instead of the dropped oldest one.
-static int tape_copy(tdw_ctx *c, const double *src, double *dst, long nd)
-{
-    return (int)hipMemcpyAsync(dst, src, sizeof(double) * nd, hipMemcpyDeviceToDevice, c->stream);
-}
-
 template <bool SP>
 static int fused_step_t(tdw_ctx *c, tdw_state *s, int it, int grad_last, tdw_tape_step *tape = nullptr,
                         double2 *cbuf = nullptr, tdw_complex *f_next = nullptr)
@@ -912,10 +907,9 @@ static int fused_step_t(tdw_ctx *c, tdw_state *s, int it, int grad_last, tdw_tap
     else
         TDW_TRY(densities(c, n, y, nullptr, nullptr, nullptr, nullptr, c->d_fbeta, c->d_s2, c->d_kt, c->d_cnt,
                           s->dens, 0));
-    if (tape) TDW_TRY(tape_copy(c, s->dens, tape->dens_p, 12 * N));
     TDW_TRY(step_potentials(c, it + 1, s->dens, s->pots));
     TDW_TRY(hkf_fields(c, s->pots, true));
-    if (tape) TDW_TRY(tape_copy(c, s->pots, tape->pots_p, 12 * N));
+    if (tape) TDW_TRY(tape_fields(c, s->dens, tape->dens_p, s->pots, tape->pots_p));
     const double *hp = h_view(c, it + 1, s->pots);
     if (!hp) return TDW_EINVAL;
     TDW_TRY(hyz<SP>(c, n, yp, T, H, hp, c->d_sp, c->d_ep, tape ? tape->scal + n : nullptr, xpart, per, c->d_s2));
@@ -937,10 +931,9 @@ static int fused_step_t(tdw_ctx *c, tdw_state *s, int it, int grad_last, tdw_tap
         else
             TDW_TRY(densities(c, n, y, nullptr, nullptr, nullptr, nullptr, c->d_fbeta, c->d_s2, c->d_kt, c->d_cnt,
                               s->dens, 0));
-        if (tape) TDW_TRY(tape_copy(c, s->dens, tape->dens_c, 12 * N));
         TDW_TRY(step_potentials(c, it + 1, s->dens, s->pots));
         TDW_TRY(hkf_fields(c, s->pots, true));
-        if (tape) TDW_TRY(tape_copy(c, s->pots, tape->pots_c, 12 * N));
+        if (tape) TDW_TRY(tape_fields(c, s->dens, tape->dens_c, s->pots, tape->pots_c));
         hp = h_view(c, it + 1, s->pots);
         if (!hp) return TDW_EINVAL;
         tdw_complex *tmp = f_next ? f_next : s->f[h - 1];
@@ -948,7 +941,8 @@ static int fused_step_t(tdw_ctx *c, tdw_state *s, int it, int grad_last, tdw_tap
         s->f[0] = tmp;
         double *e2 = tape ? tape->scal + 3 * n : (qpe != c->d_qpe ? qpe : nullptr);
         TDW_TRY(hyz<SP>(c, n, yc, T, (HC *)s->f[0], hp, c->d_scale, c->d_qpe, e2, xpart, per, c->d_s2));
-        if (tape && qpe != c->d_qpe) TDW_TRY(tape_copy(c, c->d_qpe, qpe, n));
+        if (tape && qpe != c->d_qpe)
+            TDW_HIP(hipMemcpyAsync(qpe, c->d_qpe, sizeof(double) * n, hipMemcpyDeviceToDevice, c->stream));
         // pending: y unscaled, and f[0] without the x kinetic part and the
         // <H> subtraction (the next predictor or tdw_finalize adds both)
         c->pending = 1;

@@ -158,6 +158,27 @@ int row_sums(tdw_ctx *c, const double *part, int n, int nchunk, double scale, do
     return (int)hipGetLastError();
 }
 
+// One launch for both arrays: two copies of 393 KB each (64 x 64) cost a queue
+// entry apiece, which a taped step of few states waits for: a gradient over 192
+// states of 64 x 64 (60 taped half-steps) 14.9 -> 14.6 ms.
+__global__ void __launch_bounds__(NT)
+k_tape_fields(const double *__restrict__ d, double *__restrict__ td, const double *__restrict__ p,
+              double *__restrict__ tp, long m)
+{
+    const long i = (long)blockIdx.x * NT + threadIdx.x;
+    if (i >= m) return;
+    td[i] = d[i];
+    tp[i] = p[i];
+}
+
+int tape_fields(tdw_ctx *c, const double *dens, double *tdens, const double *pots, double *tpots)
+{
+    const long m = 12L * c->N;
+    hipLaunchKernelGGL(k_tape_fields, dim3((unsigned)((m + NT - 1) / NT)), dim3(NT), 0, c->stream, dens, tdens, pots,
+                       tpots, m);
+    return (int)hipGetLastError();
+}
+
 __global__ void __launch_bounds__(NT)
 k_scale_states(double2 *__restrict__ wf, int n, long N, const double *__restrict__ nrm)
 {

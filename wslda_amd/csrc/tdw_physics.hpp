@@ -130,6 +130,8 @@ int spin_fold(tdw_ctx *c, double *dens);
 int copy_f64(tdw_ctx *c, const double *src, double *dst, long n);
 // out[a] = scale * sum of the m values of row a of part (n rows)
 int row_sums(tdw_ctx *c, const double *part, int n, int m, double scale, double *out);
+// a taped half-step's densities and potentials (12N doubles each) to its tape
+int tape_fields(tdw_ctx *c, const double *dens, double *tdens, const double *pots, double *tpots);
 // partial densities of state chunks: nf fields of N points per chunk, f[o]
 // the field that contributes to output o of the density block (-1: none)
 struct ChunkSrc {

@@ -479,11 +479,6 @@ int resident_h_only(tdw_ctx *c, int n, const double2 *in, double2 *out, const do
     return launch_h<2>(c, n, in, out, dotw, pots, nullptr, nullptr, d_dot, nullptr, nullptr);
 }
 
-static int tape_copy(tdw_ctx *c, const double *src, double *dst, long nd)
-{
-    return (int)hipMemcpyAsync(dst, src, sizeof(double) * nd, hipMemcpyDeviceToDevice, c->stream);
-}
-
 int resident_step(tdw_ctx *c, tdw_state *s, int it, int grad_last, tdw_tape_step *tape, tdw_complex *y_out,
                   double2 *cbuf, tdw_complex *f_next)
 {
@@ -509,10 +504,9 @@ int resident_step(tdw_ctx *c, tdw_state *s, int it, int grad_last, tdw_tape_step
     }
     if (y_out) s->wf = y_out;
     TDW_TRY(densities(c, n, y, nullptr, nullptr, nullptr, nullptr, c->d_fbeta, c->d_s2, c->d_kt, c->d_cnt, s->dens, 0));
-    if (tape) TDW_TRY(tape_copy(c, s->dens, tape->dens_p, 12L * N));
     TDW_TRY(step_potentials(c, it + 1, s->dens, s->pots));
     TDW_TRY(hkf_fields(c, s->pots, true));
-    if (tape) TDW_TRY(tape_copy(c, s->pots, tape->pots_p, 12L * N));
+    if (tape) TDW_TRY(tape_fields(c, s->dens, tape->dens_p, s->pots, tape->pots_p));
     const double *hp = h_view(c, it + 1, s->pots);
     if (!hp) return TDW_EINVAL;
     TDW_TRY(launch_h<1>(c, n, y, y, cc, hp, c->d_sp, nullptr, qpe, tape ? tape->scal + n : nullptr,
@@ -531,10 +525,9 @@ int resident_step(tdw_ctx *c, tdw_state *s, int it, int grad_last, tdw_tape_step
                           c->d_fbeta, nullptr, c->d_kt, c->d_cnt, s->dens, grad_last));
     }
     if (grad_last) TDW_TRY(density_tau(c, s->dens));
-    if (tape) TDW_TRY(tape_copy(c, s->dens, tape->dens_c, 12L * N));
     TDW_TRY(step_potentials(c, it + 1, s->dens, s->pots));
     TDW_TRY(hkf_fields(c, s->pots, true));
-    if (tape) TDW_TRY(tape_copy(c, s->pots, tape->pots_c, 12L * N));
+    if (tape) TDW_TRY(tape_fields(c, s->dens, tape->dens_c, s->pots, tape->pots_c));
     hp = h_view(c, it + 1, s->pots);
     if (!hp) return TDW_EINVAL;
     tdw_complex *tmp = f_next ? f_next : s->f[h - 1];
