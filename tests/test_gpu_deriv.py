@@ -67,3 +67,31 @@ def test_derivatives_3d_lengths(torch, shape, m):
     ctx.sync()
     assert rel(t.cpu().numpy(), lap) < TOL
     ctx.close()
+
+
+@pytest.mark.parametrize("shape", [(32, 32), (32, 64), (64, 32), (64, 64)])
+@pytest.mark.parametrize("m", [1, 3])
+def test_derivatives_2d_planes(torch, shape, m):
+    """The one-pass derivatives of 2D planes on the matrix cores."""
+    from wslda_amd import td
+    say("case: derivatives shape=%s m=%d" % (shape, m))
+    nx, ny = shape
+    cfg = po.make_cfg(2, nx, ny, 4, dx=0.9)
+    cfg.dy = 1.1
+    r = np.random.default_rng(nx + ny + m)
+    a = r.normal(size=(m, nx * ny)) + 1j * r.normal(size=(m, nx * ny))
+    ctx = td.TDContext(tdgauss.to_params(cfg, td.FP64), m, 0)
+    f = np.fft.fftn(a.reshape(m, nx, ny), axes=(1, 2))
+    k = lambda first: (kax(nx, 0.9, first).reshape(-1, 1), kax(ny, 1.1, first).reshape(1, -1))
+    back = lambda g: np.fft.ifftn(g, axes=(1, 2)).reshape(m, nx * ny)
+    kx, ky = k(False)
+    gx, gy = k(True)
+    t = cuda(torch, a)
+    D = [torch.zeros_like(t) for _ in range(3)]
+    ctx.compute_derivatives(t, D[0], D[1], None, D[2])
+    ctx.sync()
+    assert rel(D[0].cpu().numpy(), back(1j * gx * f)) < TOL
+    assert rel(D[1].cpu().numpy(), back(1j * gy * f)) < TOL
+    assert rel(D[2].cpu().numpy(), back(-(kx ** 2 + ky ** 2) * f)) < TOL
+    assert rel(t.cpu().numpy(), a) == 0.0
+    ctx.close()

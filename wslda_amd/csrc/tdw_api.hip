@@ -103,6 +103,11 @@ int derivatives(tdw_ctx *c, int m, const double2 *in, double2 *ddx, double2 *ddy
 {
     if (m <= 0) return 0;
     if (lap == in || ddx == in) return TDW_EINVAL;
+    if (c->dim == 2 && ddx && ddy && lap) {
+        int done;
+        TDW_TRY(plane_derivatives(c, m, in, ddx, ddy, lap, &done));
+        if (done) return 0;
+    }
     TDW_TRY(launch_outer(c, m, in, lap, ddx, 1));
     if (c->dim == 1) return 0;
     return launch_inner(c, m, in, lap, lap, ddy, c->dim == 3 ? ddz : nullptr, 1);

@@ -21,6 +21,9 @@ bool resident_supported(const tdw_ctx *c);
 // dropped oldest entry).
 int resident_step(tdw_ctx *c, tdw_state *s, int it, int grad_last, tdw_tape_step *tape = nullptr,
                   tdw_complex *y_out = nullptr, double2 *cbuf = nullptr, tdw_complex *f_next = nullptr);
+// 2D planes of 32 or 64 points a side: ddx, ddy and the Laplacian of m arrays
+// in one pass (no result may be another's array); *done = 0 elsewhere
+int plane_derivatives(tdw_ctx *c, int m, const double2 *in, double2 *ddx, double2 *ddy, double2 *lap, int *done);
 // out = H in - e in with <H> of in into qpe, or with use_e the given e (qpe
 // is then not written)
 int resident_h(tdw_ctx *c, int n, const double2 *in, double2 *out, const double *pots, double *qpe,
