@@ -9,7 +9,8 @@
 // Every K_d needs only spectral derivatives along axis d of psi and of
 // alpha psi, so the x terms are formed in an x-pencil pass (blocks of
 // pencils, in-place two-factor FFT in LDS) and stored in T, and the y, z
-// terms with the pointwise terms in a yz-plane pass (the same FFT) that
+// terms with the pointwise terms in a yz-plane pass (the same FFT, or
+// matrix-core products for FP64 planes of 24 and 32 points a side) that
 // reads psi and T and writes H psi with the <psi|H psi> partials.  This
 // replaces alpha*psi, the batched lap(alpha psi) through a scratch array,
 // and the H kernel that reads psi, its three gradients, its Laplacian and
@@ -241,7 +242,7 @@ ah_yz(const ac_t<SP> *__restrict__ y, const ac_t<SP> *__restrict__ T, ac_t<SP> *
 // twice, as the operands of tdw_planemm.hpp: one wave per component holds a
 // quarter of its plane and the three images (rows and columns past L / 2 of the
 // 16 x 16 tile are padding at 24: 44 % of the products, still the shorter
-// form).  1656 states of 24^3: 986 -> 870 us, 300 of 32^3 a whole step 1.18x
+// form).  1656 states of 24^3: 986 -> 840 us, 300 of 32^3 a whole step 1.18x
 // faster.  Two waves per SIMD (244 registers), the FP64 pipe (products and
 // sums) busy three quarters of the time; without the factors and tables loaded
 // ahead of the products that hide them it took 1227 us.

@@ -34,38 +34,29 @@ __device__ __forceinline__ void mm_clear(MmAcc &a)
         for (int q = 0; q < 2; q++) a.P[g][q] = a.Q[g][q] = dbl4{0.0, 0.0, 0.0, 0.0};
 }
 
-// one step of four columns of the matrix (mp, mm: its P and M elements)
-template <bool OUTER>
-__device__ __forceinline__ void mm_step(double mp, double mm, const double2 (&u)[2], const double2 (&v)[2], MmAcc &a)
-{
-#pragma unroll
-    for (int g = 0; g < 2; g++) {
-        const double pr = u[g].x + v[g].x, pi = u[g].y + v[g].y, qr = u[g].x - v[g].x, qi = u[g].y - v[g].y;
-        if constexpr (OUTER) {
-            a.P[g][0] = __builtin_amdgcn_mfma_f64_16x16x4f64(mp, pr, a.P[g][0], 0, 0, 0);
-            a.P[g][1] = __builtin_amdgcn_mfma_f64_16x16x4f64(mp, pi, a.P[g][1], 0, 0, 0);
-            a.Q[g][0] = __builtin_amdgcn_mfma_f64_16x16x4f64(mm, qr, a.Q[g][0], 0, 0, 0);
-            a.Q[g][1] = __builtin_amdgcn_mfma_f64_16x16x4f64(mm, qi, a.Q[g][1], 0, 0, 0);
-        } else {
-            a.P[g][0] = __builtin_amdgcn_mfma_f64_16x16x4f64(pr, mp, a.P[g][0], 0, 0, 0);
-            a.P[g][1] = __builtin_amdgcn_mfma_f64_16x16x4f64(pi, mp, a.P[g][1], 0, 0, 0);
-            a.Q[g][0] = __builtin_amdgcn_mfma_f64_16x16x4f64(qr, mm, a.Q[g][0], 0, 0, 0);
-            a.Q[g][1] = __builtin_amdgcn_mfma_f64_16x16x4f64(qi, mm, a.Q[g][1], 0, 0, 0);
-        }
-    }
-}
-
 // Products along the outer axis (rows, H = half its length, RS apart): x at
 // row lane / 16 and the lane's column of the tile, whose image is G columns
 // on; along the inner axis: x at row lane % 16 of the tile and column
-// lane / 16, the tile's image G rows on.
+// lane / 16, the tile's image G rows on.  One step of four columns of the
+// matrix (mp, mm: its P and M elements).
 template <bool OUTER, int H, int RS, int G>
-__device__ __forceinline__ void mm_operands(const double2 *x, int ks, double2 (&u)[2], double2 (&v)[2])
+__device__ __forceinline__ void mm_step(const double2 *x, int ks, double mp, double mm, MmAcc &a)
 {
 #pragma unroll
     for (int g = 0; g < 2; g++) {
-        u[g] = OUTER ? x[4 * ks * RS + g * G] : x[g * G * RS + 4 * ks];
-        v[g] = OUTER ? x[(4 * ks + H) * RS + g * G] : x[g * G * RS + 4 * ks + H];
+        const double2 u = OUTER ? x[4 * ks * RS + g * G] : x[g * G * RS + 4 * ks];
+        const double2 v = OUTER ? x[(4 * ks + H) * RS + g * G] : x[g * G * RS + 4 * ks + H];
+        if constexpr (OUTER) {
+            a.P[g][0] = __builtin_amdgcn_mfma_f64_16x16x4f64(mp, u.x + v.x, a.P[g][0], 0, 0, 0);
+            a.P[g][1] = __builtin_amdgcn_mfma_f64_16x16x4f64(mp, u.y + v.y, a.P[g][1], 0, 0, 0);
+            a.Q[g][0] = __builtin_amdgcn_mfma_f64_16x16x4f64(mm, u.x - v.x, a.Q[g][0], 0, 0, 0);
+            a.Q[g][1] = __builtin_amdgcn_mfma_f64_16x16x4f64(mm, u.y - v.y, a.Q[g][1], 0, 0, 0);
+        } else {
+            a.P[g][0] = __builtin_amdgcn_mfma_f64_16x16x4f64(u.x + v.x, mp, a.P[g][0], 0, 0, 0);
+            a.P[g][1] = __builtin_amdgcn_mfma_f64_16x16x4f64(u.y + v.y, mp, a.P[g][1], 0, 0, 0);
+            a.Q[g][0] = __builtin_amdgcn_mfma_f64_16x16x4f64(u.x - v.x, mm, a.Q[g][0], 0, 0, 0);
+            a.Q[g][1] = __builtin_amdgcn_mfma_f64_16x16x4f64(u.y - v.y, mm, a.Q[g][1], 0, 0, 0);
+        }
     }
 }
 
@@ -75,12 +66,7 @@ __device__ __forceinline__ void mm_product(const double2 *x, const double *M, Mm
 {
     mm_clear(a);
 #pragma unroll 2
-    for (int ks = 0; ks < H / 4; ks++) {
-        const double mp = M[ks * 128], mm = M[ks * 128 + 64];
-        double2 u[2], v[2];
-        mm_operands<OUTER, H, RS, G>(x, ks, u, v);
-        mm_step<OUTER>(mp, mm, u, v, a);
-    }
+    for (int ks = 0; ks < H / 4; ks++) mm_step<OUTER, H, RS, G>(x, ks, M[ks * 128], M[ks * 128 + 64], a);
 }
 
 // the same with the tables in registers (mm_load)
@@ -101,11 +87,7 @@ __device__ __forceinline__ void mm_product(const double2 *x, const MmTab<H> &t, 
 {
     mm_clear(a);
 #pragma unroll
-    for (int ks = 0; ks < H / 4; ks++) {
-        double2 u[2], v[2];
-        mm_operands<OUTER, H, RS, G>(x, ks, u, v);
-        mm_step<OUTER>(t.p[ks], t.m[ks], u, v, a);
-    }
+    for (int ks = 0; ks < H / 4; ks++) mm_step<OUTER, H, RS, G>(x, ks, t.p[ks], t.m[ks], a);
 }
 
 // results at row image h, column image g: re (q 0) or im (q 1), four rows
