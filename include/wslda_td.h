@@ -215,7 +215,10 @@ int tdw_vext_eval(tdw_ctx *c, int it, double *va, double *vb);
  * without FAST_CONST_EFFECTIVE_MASS_MODE), so ddx..ddz of the evolved axes
  * must be set; grad_last changes nothing there.  On 3D lattices with the
  * two-pass kernels the ASLDA step forms the gradients inside its density
- * and H passes and leaves ddx..ddz untouched. */
+ * and H passes and leaves ddx..ddz untouched.  1D and 2D lattices whose state
+ * (both components) fits in a CU's LDS run the step with the state resident
+ * there (constant effective mass); lap is then written only by a step with
+ * grad_last. */
 typedef struct {
     int n;
     tdw_complex *wf, *lap, *ddx, *ddy, *ddz;
@@ -235,9 +238,13 @@ int tdw_step(tdw_ctx *c, tdw_state *s, int it, int grad_last);
  * the normalisations and the <H> subtraction carried as per-state scalars,
  * so between steps wf is unnormalised and f[0] lacks only the subtraction
  * (same completion rules); it has a split form too (below; its
- * measurement steps also use ddy and ddz as FP64 scratch).  Other lattices
- * run the modular step (tdw_fused_supported() says whether the
- * constant-mass fused passes run).
+ * measurement steps also use ddy and ddz as FP64 scratch).  FP64 lattices of
+ * constant effective mass whose state fits in LDS (1D, 2D, and 3D lattices
+ * with fused passes up to 16^3) run the resident step, which leaves nothing to
+ * complete; those with axes of 18, 36 and 48 points run the six passes,
+ * completed at each step's end.  Other lattices run the modular step.
+ * tdw_fused_supported() says whether the lattice is one of those with fused
+ * passes in both precisions.
  *
  * Split precision (params.precision == TDW_SPLIT): the x / yz FFTs and the
  * kinetic term run in FP32 complex, and f[0..4] hold FP32 complex values
