@@ -1,8 +1,11 @@
 """The pointwise functional over the whole range of its inputs, through the C
 ABI against the CPU oracle: densities from far below the regularisation
-threshold to several times the uniform gas, mean fields on both sides of the
-band bottom (real and imaginary p0) and energies below the cutoff's reach
-(imaginary k_c), each functional, both regularisation schemes."""
+threshold to several times the uniform gas, each functional, both
+regularisation schemes.  The first test starts the mixing loop from mean fields
+on both sides of the band bottom; without an external potential the loop has
+left those behind at its end.  The second holds points outside the real range
+of the regularisation by an external potential: below the cutoff's reach
+(imaginary k_c) and, with the cubic cutoff, above it (p0 > pi / dx)."""
 import ctypes as C
 
 import numpy as np
@@ -88,3 +91,80 @@ def test_potentials_over_the_input_range(torch, functional, a1, reg, ec):
     lim = 10.0 * lim + 1e-12 * np.maximum(np.abs(ref), 1.0)
     d = np.abs(got - ref)
     assert (d[ok] <= lim[ok]).all(), (d[ok] / lim[ok]).max()
+
+
+@pytest.mark.parametrize("functional,a1", [(po.SLDA, 0), (po.BDG, 0), (po.ASLDA, 0), (po.SLDAE, 0), (po.SLDAE, 1)])
+@pytest.mark.parametrize("reg", [88, 89])
+def test_potentials_outside_the_real_range(torch, functional, a1, reg):
+    """A barrier of 8 ec beside a deep well: V_+ - mu_+ at the end of the loop
+    runs from beyond -(pi / dx)^2 / 2 over the band bottom to several ec, so the
+    last iterations see every branch of the regularisation."""
+    from wslda_amd import td
+    say("case: potentials in V_ext functional=%d a1=%d regularization=%d" % (functional, a1, reg))
+    ec, dx = 0.3, 1.1
+    vext = po.gauss_vext([(8.0 * ec, (-7.0, 0.0, 0.0), (-0.03, -0.02, 0.0)),
+                          (-7.0, (7.0, 0.0, 0.0), (-0.03, -0.02, 0.0))])
+    cfg = po.make_cfg(2, 24, 16, 4, dx=dx, functional=functional, force_a1=a1, vext=vext,
+                      sclgth=-0.9 if functional in (po.BDG, po.SLDAE) else 0.0)
+    # (the mean-field correction is the logarithm of a negative number above the
+    # cubic cutoff)
+    cfg.regularization, cfg.mf_correction = reg, int(reg == 88)
+    cfg.mu_a, cfg.mu_b, cfg.ec = 0.25, 0.2, ec
+    N = po.npts(cfg)
+    dens, pots = inputs(N, 31 + functional + reg)
+    va, vb = np.zeros(N), np.zeros(N)
+    po.lib().tdwo_vext_eval(C.byref(cfg), 1, po.ptr(va), po.ptr(vb))
+    # BdG is one evaluation from the V given
+    pots[:N] += va
+    pots[N:2 * N] += vb
+
+    def oracle(d, p):
+        p = p.copy()
+        po.lib().tdwo_potentials(C.byref(cfg), 1, po.ptr(np.ascontiguousarray(d)), po.ptr(p))
+        return p
+
+    ref = oracle(dens, pots)
+    ok = ~np.isnan(ref[:4 * N]).reshape(4, N).any(0)
+    # mu_+ - V_+ of the last evaluation, and which branch that is
+    last = pots if functional == po.BDG else ref
+    al = np.ones(N) if functional == po.BDG else 0.5 * (ref[4 * N:5 * N] + ref[5 * N:6 * N])
+    if functional == po.SLDA or a1:
+        al = np.ones(N)
+    t7 = 0.5 * (cfg.mu_a + cfg.mu_b - last[:N] - last[N:2 * N])
+    below = t7 < -ec
+    above = 2.0 * t7 / al > (np.pi / dx) ** 2
+    inside = (t7 > 0.0) & ~above
+    parts = [below, inside, (t7 < 0.0) & ~below] + ([above] if reg == 89 else [])
+    for part in parts:
+        assert (part & ok).sum() >= 10
+    # as in the first test: ten times what a relative change of the inputs by
+    # 1e-13 does to the point, plus round-off (of V_ext and mu, of order one,
+    # in V; of Delta itself in Delta)
+    r = np.random.default_rng(1)
+    amp = np.zeros(4 * N)
+    for _ in range(6):
+        d = oracle(dens * (1 + 1e-13 * r.choice([-1, 1], dens.size)), pots * (1 + 1e-13 * r.choice([-1, 1], pots.size)))
+        amp = np.maximum(amp, np.nan_to_num(np.abs(d - ref)[:4 * N]))
+
+    def points(a):   # per point: V_a, V_b, |Delta|
+        return np.stack([a[:N], a[N:2 * N], np.hypot(a[2 * N:4 * N:2], a[2 * N + 1:4 * N:2])])
+
+    scale = np.abs(points(np.abs(ref)))
+    scale[:2] = np.maximum(scale[:2], 1.0)
+    A = points(amp)
+    lim = 10.0 * np.maximum(A, scale * (A / scale).max(0)) + 1e-12 * scale
+    # the limit is a real one at most points of every branch
+    sharp = (lim <= 1e-10 * scale).all(0) & ok
+    for part in parts:
+        assert sharp[part].mean() > 0.6, (sharp[part].mean(), part.sum())
+    prm = tdgauss.to_params(cfg, td.FP64)
+    ctx = td.TDContext(prm, 4, 0)
+    dd, dp = cuda(torch, dens), cuda(torch, pots)
+    ctx.compute_potentials(1, dd, dp)
+    ctx.sync()
+    got = dp.cpu().numpy()
+    ctx.close()
+    assert np.array_equal(np.isnan(got), np.isnan(ref))
+    err = points(np.abs(got - ref)[:4 * N])
+    bad = (err > lim) & ok
+    assert not bad.any(), (functional, reg, bad.any(0).sum(), (err / lim)[:, ok].max())

@@ -178,9 +178,13 @@ __device__ __forceinline__ bool reg_real(const FParams &f, const MfConst &m, dou
     return p2 >= 1.0e-30 && p2 < 1.0e30 && d > 1.0e-10 * kc2 && kc2 < 1.0e30 && lx < 0.999;
 }
 
-// The 15 mixing iterations of V_a, V_b and Delta = -nu Re(alpha_+ / (C - wz))
+// The 15 mixing iterations of V_a, V_b and Delta = -nu g
 // (tdwslda_functionals.h:236-300) from the previous V_a, V_b: each new V_s is
 // V_s,const - e_s Re(Delta* nu) - c_s |Delta|^2 + the mean-field correction.
+// g = Re(alpha_+ / (C - wz)), or with REAL_WZ (SLDAE) alpha_+ / (C -
+// Re wz).  The two part where wz is complex: below the cutoff's reach (mu_+ -
+// V_+ < -ec) and, with the cubic cutoff, above it (p0 > pi / dx).
+template <bool REAL_WZ = false>
 __device__ __forceinline__ void mix_loop(const FParams &f, double n, double2 nu, double alph_plus, double C,
                                          double Va_const, double Vb_const, double ea, double eb, double ca, double cb,
                                          double &Va, double &Vb, double2 &delta)
@@ -204,7 +208,7 @@ __device__ __forceinline__ void mix_loop(const FParams &f, double n, double2 nu,
         } else {
             double2 wz, p0;
             reg_wz(f, t7, kscale2, wz, p0);
-            g = re_inv(alph_plus, C, wz);
+            g = REAL_WZ ? alph_plus / (C - wz.x) : re_inv(alph_plus, C, wz);
             if (f.mf) dl = mf_corr(m, p0.x, g);
         }
         const double dn = -g * nu2, d2 = g * g * nu2;   // Re(Delta* nu), |Delta|^2
@@ -327,8 +331,8 @@ __device__ __forceinline__ void sldae_point(const FParams &f, double na, double 
         Vb_const += ((af - 1.0) / nb - af_p) * t7;
         Vb_const -= cc * der_p_reg(f, nb) * (af - 1.0) * j2b / (2.0 * nb);
     }
-    mix_loop(f, n, nu, af, L.ctilde, Va_const, Vb_const, af_p / af, af_p / af, L.ctilde_p / af, L.ctilde_p / af, Va, Vb,
-             delta);
+    mix_loop<true>(f, n, nu, af, L.ctilde, Va_const, Vb_const, af_p / af, af_p / af, L.ctilde_p / af, L.ctilde_p / af,
+                   Va, Vb, delta);
 }
 
 // BdG potentials at one point (tdwslda_functionals.h:373-452).
