@@ -210,7 +210,9 @@ int tdw_vext_eval(tdw_ctx *c, int it, double *va, double *vb);
 
 /* One PECE step of pca.c:1401-1570 on the arrays of a run.  f[0..4] are
  * fkm1..fkm5 and are rotated in place (pointer swaps) as pca.c:1543-1562
- * does.  grad_last: full derivatives (tau, j) on this step's corrector.
+ * does.  grad_last: full derivatives (tau, j) on this step's corrector, which
+ * need lap and the evolved axes' ddx..ddz (the resident and the fused steps
+ * return TDW_EINVAL without them, before anything is written).
  * ASLDA computes the derivatives on both half-steps (the reference's path
  * without FAST_CONST_EFFECTIVE_MASS_MODE), so ddx..ddz of the evolved axes
  * must be set; grad_last changes nothing there.  On 3D lattices with the

@@ -83,3 +83,25 @@ def test_resident_step_vs_oracle(torch, dim, shape, n, scheme, functional):
             assert rel(R.wf.cpu().numpy(), P.wf) < TOL, it
             assert rel(R.qpe.cpu().numpy(), P.qpe) < TOL, it
     ctx.close()
+
+
+@pytest.mark.parametrize("dim,shape", [(1, (64, 4, 4)), (2, (16, 16, 4)), (2, (12, 18, 4)), (3, (8, 8, 8)),
+                                       (3, (12, 12, 12))])
+def test_gradient_step_without_its_arrays_is_refused(torch, dim, shape):
+    """The return code, and that nothing was written: no kernel is launched."""
+    from wslda_amd import td
+    n = 3
+    cfg, wf, fb, kt, cnt, pots = problem(dim, shape, n, po.AB4AM5, po.SLDA)
+    ctx = td.TDContext(tdgauss.to_params(cfg, td.FP64), n, 0)
+    ctx.set_states(fb, kt, cnt)
+    R = td.TDRun(ctx, wf, pots, fused=dim == 3)
+    fn = td.lib().tdw_step_fused if dim == 3 else td.lib().tdw_step
+    before, hist = R.wf.clone(), [R.st.f[k] for k in range(5)]
+    for name in ("lap", "ddx", "ddy", "ddz")[:dim + 1]:
+        keep = getattr(R.st, name)
+        setattr(R.st, name, None)
+        assert fn(ctx.h, C.byref(R.st), 0, 1) == td.TDW_EINVAL, name
+        setattr(R.st, name, keep)
+    ctx.sync()
+    assert torch.equal(R.wf, before) and hist == [R.st.f[k] for k in range(5)]
+    ctx.close()

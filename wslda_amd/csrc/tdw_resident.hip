@@ -562,6 +562,8 @@ int resident_h_only(tdw_ctx *c, int n, const double2 *in, double2 *out, const do
 int resident_step(tdw_ctx *c, tdw_state *s, int it, int grad_last, tdw_tape_step *tape, tdw_complex *y_out,
                   double2 *cbuf, tdw_complex *f_next)
 {
+    // a gradient step's derivative arrays: refused before anything is written
+    if (grad_last && (!s->lap || !s->ddx || (c->dim >= 2 && !s->ddy) || (c->dim >= 3 && !s->ddz))) return TDW_EINVAL;
     const int n = s->n, N = (int)c->N;
     const int h = c->p.scheme == TDW_AB3AM4 ? 3 : c->p.scheme == TDW_AB4AM5 ? 4 : 5;
     TDW_TRY(fused_state_vecs(c));
