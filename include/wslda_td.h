@@ -219,8 +219,9 @@ int tdw_vext_eval(tdw_ctx *c, int it, double *va, double *vb);
  * two-pass kernels the ASLDA step forms the gradients inside its density
  * and H passes and leaves ddx..ddz untouched.  1D and 2D lattices whose state
  * (both components) fits in a CU's LDS run the step with the state resident
- * there (constant effective mass); lap is then written only by a step with
- * grad_last. */
+ * there (constant effective mass).  lap holds the Laplacian of wf after a
+ * constant-mass tdw_step, except after one without grad_last on lattices of
+ * 32 x 32 and 64 x 64 points, where it is scratch. */
 typedef struct {
     int n;
     tdw_complex *wf, *lap, *ddx, *ddy, *ddz;

@@ -105,3 +105,24 @@ def test_gradient_step_without_its_arrays_is_refused(torch, dim, shape):
     ctx.sync()
     assert torch.equal(R.wf, before) and hist == [R.st.f[k] for k in range(5)]
     ctx.close()
+
+
+@pytest.mark.parametrize("dim,shape,n", [c for c in CASES if c[0] < 3 and c[1] not in ((64, 64, 4), (32, 32, 4))])
+def test_step_leaves_the_laplacian(torch, dim, shape, n):
+    """lap after a step without gradients (not on 32 x 32 and 64 x 64)."""
+    from wslda_amd import td
+    say("case: lap after a step dim=%d shape=%s n=%d" % (dim, shape, n))
+    cfg, wf, fb, kt, cnt, pots = problem(dim, shape, n, po.AB4AM5, po.SLDA)
+    ctx = td.TDContext(tdgauss.to_params(cfg, td.FP64), n, 0)
+    ctx.set_states(fb, kt, cnt)
+    R = td.TDRun(ctx, wf, pots)
+    R.initial_measure()
+    for it in range(2):
+        R.step(it)
+    ctx.sync()
+    got, y = R.lap.cpu().numpy(), R.wf.cpu().numpy()
+    ctx.close()
+    ref = np.zeros_like(y)
+    po.lib().tdwo_laplace(C.byref(cfg), 2 * n, po.ptr(y), po.ptr(ref))
+    # (relative to the largest: the highest modes carry the rounding)
+    assert np.abs(got - ref).max() <= TOL * np.abs(ref).max()

@@ -511,10 +511,9 @@ extern "C" int tdw_step(tdw_ctx *c, tdw_state *s, int it, int grad_last)
         if (!s->ddx || (c->dim >= 2 && !s->ddy) || (c->dim >= 3 && !s->ddz)) return TDW_EINVAL;
         return step_aslda(c, s, it, k, qpe);
     }
-    // 1D and 2D lattices whose state fits in LDS run the resident step; lap is
-    // then written only by a gradient step.  In 3D this entry stays the kernel
-    // sequence that a caller of the separate entry points gets, to the bit;
-    // tdw_step_fused runs the resident step there.
+    // 1D and 2D lattices whose state fits in LDS run the resident step.  In 3D
+    // this entry stays the kernel sequence that a caller of the separate entry
+    // points gets, to the bit; tdw_step_fused runs the resident step there.
     if (c->dim < 3 && resident_supported(c)) return resident_step(c, s, it, grad_last);
     // predictor
     TDW_TRY(abm1(c, n, D2(s->wf), D2(s->f[0]), D2(s->f[1]), D2(s->f[2]), D2(s->f[3]), D2(s->f[4])));

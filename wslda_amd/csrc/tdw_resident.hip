@@ -101,7 +101,7 @@ struct RsH {
     int bdg;
 };
 
-// CORR 0: out = H psi - <H> psi, psi = in.
+// CORR 0: out = H psi - <H> psi, psi = in; with lap, lap = its Laplacian.
 // CORR 1: psi = s_a in (the normalised prediction), out = the normalised
 // corrected state of -i dt a0 (H psi - <H> psi) + c (out may be in: a state
 // is read whole before it is written).
@@ -115,7 +115,7 @@ rs_h(const double2 *in, double2 *out, const double2 *__restrict__ c, const doubl
      const double *__restrict__ sc, const double *__restrict__ kt, const double *__restrict__ kt2, int n, int N,
      RsPlan pl, RsH hp, const double2 *__restrict__ twg, int ntw, const double *__restrict__ kx,
      const double *__restrict__ kin, const double *use_e, double *e_out, double *e_out2,
-     double *__restrict__ nrm_out)
+     double *__restrict__ nrm_out, double2 *lap)
 {
     extern __shared__ double2 rs_sm[];
     __shared__ double red[RS_NT / 64];
@@ -144,6 +144,10 @@ rs_h(const double2 *in, double2 *out, const double2 *__restrict__ c, const doubl
         const double Va = pots[i] - hp.mu_a - aa * k2t, Vb = pots[N + i] - hp.mu_b - ab * k2t;
         const double2 D = make_double2(pots[2 * N + 2 * i], pots[2 * N + 2 * i + 1]);
         const double2 tu = in[gu + i] * s, tv = in[gv + i] * s;
+        if (CORR == 0 && lap) {
+            lap[gu + i] = A[pe];
+            lap[gv + i] = A[pl.npc + pe];
+        }
         const double2 u = tu * Va + cmul(tv, D) + A[pe] * aa;
         const double2 v = tv * (-Vb) + cmulc(D, tu) - A[pl.npc + pe] * ab;
         if constexpr (CORR == 2) {
@@ -499,7 +503,8 @@ static int rs_threads(size_t lds, int n, int N)
 
 template <int CORR>
 static int launch_h(tdw_ctx *c, int n, const double2 *in, double2 *out, const double2 *cc, const double *pots,
-                    const double *sc, const double *use_e, double *e_out, double *e_out2, double *nrm_out)
+                    const double *sc, const double *use_e, double *e_out, double *e_out2, double *nrm_out,
+                    double2 *lap = nullptr)
 {
     const RsPlan &pl = *c->rplan;
     const int N = (int)c->N, ntw = pl.ax[0].L + (pl.dim > 1 ? pl.ax[1].L : 0) + (pl.dim > 2 ? pl.ax[2].L : 0);
@@ -529,7 +534,7 @@ static int launch_h(tdw_ctx *c, int n, const double2 *in, double2 *out, const do
         return (int)hipGetLastError();
     }
     hipLaunchKernelGGL(rs_h<CORR>, dim3(n), dim3(rs_threads(lds, n, N)), lds, c->stream, in, out, cc, pots, sc, kt, kt2,
-                       n, N, pl, hp, tw, ntw, kx, kx + pl.ax[0].L, use_e, e_out, e_out2, nrm_out);
+                       n, N, pl, hp, tw, ntw, kx, kx + pl.ax[0].L, use_e, e_out, e_out2, nrm_out, lap);
     return (int)hipGetLastError();
 }
 
@@ -615,8 +620,18 @@ int resident_step(tdw_ctx *c, tdw_state *s, int it, int grad_last, tdw_tape_step
     tdw_complex *tmp = f_next ? f_next : s->f[h - 1];
     for (int j = h - 1; j > 0; j--) s->f[j] = s->f[j - 1];
     s->f[0] = tmp;
+    // 1D and 2D steps leave the Laplacian of y in lap (a gradient step's
+    // derivatives have): rs_h stores it on its way (1 S, 1-2 % of a step).
+    // rs_mm does not (64 x 64 x 1024: 552 -> 640 us a step with the store, and
+    // the plane-wise step before it left H y_p there), so lap is scratch on
+    // 32 x 32 and 64 x 64; planes of 32 x 64 points take a pass of their own.
+    double2 *lap = c->dim < 3 && !grad_last ? (double2 *)s->lap : nullptr;
+    if (lap && mm_plane(c)) {
+        if (c->nx != c->ny) TDW_TRY(laplace(c, 2 * n, y, lap));
+        lap = nullptr;
+    }
     return launch_h<0>(c, n, y, (double2 *)s->f[0], nullptr, hp, nullptr, nullptr, qpe,
-                       tape ? tape->scal + 3 * n : nullptr, nullptr);
+                       tape ? tape->scal + 3 * n : nullptr, nullptr, lap);
 }
 
 }  // namespace tdw

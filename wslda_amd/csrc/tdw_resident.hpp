@@ -15,7 +15,7 @@ void resident_release(tdw_ctx *c);
 // constant-mass H in FP64 on a lattice with a plan
 bool resident_supported(const tdw_ctx *c);
 // The step of tdw_step (same arrays, complete at its end; lap is not
-// written by a step without gradients).  The adjoint's taped step is the
+// written in 3D without gradients).  The adjoint's taped step is the
 // same with tape: y to y_out (NULL: in place), the partial corrector to cbuf
 // (NULL: the oldest history entry), the new entry to f_next (NULL: the
 // dropped oldest entry).
