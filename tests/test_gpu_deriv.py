@@ -95,3 +95,23 @@ def test_derivatives_2d_planes(torch, shape, m):
     assert rel(D[2].cpu().numpy(), back(-(kx ** 2 + ky ** 2) * f)) < TOL
     assert rel(t.cpu().numpy(), a) == 0.0
     ctx.close()
+
+
+@pytest.mark.parametrize("shape", [(16, 16, 16), (16, 16, 18)])
+def test_one_timer_record_per_launch(torch, shape):
+    """A compiled plane and one without: each launch is recorded once."""
+    from wslda_amd import td
+    cfg = po.make_cfg(3, *shape, dx=0.9)
+    N = int(np.prod(shape))
+    ctx = td.TDContext(tdgauss.to_params(cfg, td.FP64), 2, 0)
+    t = cuda(torch, np.ones((2, N), dtype=complex))
+    D = [torch.zeros_like(t) for _ in range(4)]
+    ctx.timing(1)
+    ctx.compute_laplace(t, D[3])
+    ctx.compute_derivatives(t, *D)
+    ctx.sync()
+    rep = ctx.timing_report()
+    ctx.timing(0)
+    ctx.close()
+    assert {k: v[1] for k, v in rep.items()} == {"fft_outer": 1, "fft_inner": 1, "fft_outer_deriv": 1,
+                                                 "fft_inner_deriv": 1}

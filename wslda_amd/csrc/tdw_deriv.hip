@@ -222,6 +222,7 @@ static int run_yz(tdw_ctx *c, int m, const double2 *in, const double2 *T, double
 {
     const long np = (long)m * c->nx;
     const dim3 g((unsigned)((np + NP - 1) / NP));
+    TDW_TIMED(c, mode ? "fft_inner_deriv" : "fft_inner");
     if (mode == 0)
         hipLaunchKernelGGL((lap_yz<LY, LZ, NP, NT>), g, dim3(NT), 0, c->stream, in, T, out, np, c->d_tw[1], c->d_tw[2],
                            k2f(c, 1, LY), k2f(c, 2, LZ));

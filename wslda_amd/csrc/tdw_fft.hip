@@ -231,10 +231,7 @@ int launch_inner(tdw_ctx *c, int m, const double2 *in, const double2 *T, double2
     long nblk = (long)m * c->nx;   // inner blocks of S points
     if (c->dim == 3) {
         int done;
-        {
-            TDW_TIMED(c, mode ? "fft_inner_deriv" : "fft_inner");
-            TDW_TRY(deriv3d_inner(c, m, in, T, out, ddy, ddz, mode, &done));
-        }
+        TDW_TRY(deriv3d_inner(c, m, in, T, out, ddy, ddz, mode, &done));
         if (done) return 0;
         if (mode == 0) return launch_inner_k<0, 2>(c, nblk, 1, in, T, out, ddy, ddz);
         return launch_inner_k<1, 2>(c, nblk, 1, in, T, out, ddy, ddz);
