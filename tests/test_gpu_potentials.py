@@ -168,3 +168,42 @@ def test_potentials_outside_the_real_range(torch, functional, a1, reg):
     err = points(np.abs(got - ref)[:4 * N])
     bad = (err > lim) & ok
     assert not bad.any(), (functional, reg, bad.any(0).sum(), (err / lim)[:, ok].max())
+
+
+def test_mean_field_rounding(torch):
+    """V_s = dD/dn_s (no pairing, no external potential, 15 mixing steps of 3/4
+    from zero) against extended precision: its powers of 2/3 and 5/3 have to be as good as pow's.  Each
+    term of dD/dn is then good to about three units in the last place; the
+    limit is four for nine points in ten (dD/dn_b passes through zero)."""
+    from wslda_amd import td
+    cfg = po.make_cfg(2, 128, 128, 4, dx=1.1)
+    cfg.mu_a, cfg.mu_b, cfg.ec, cfg.mf_correction = 0.25, 0.2, 4.9, 1
+    N = po.npts(cfg)
+    dens, pots = inputs(N, 3)
+    dens[:2 * N], pots[:4 * N] = 0.0, 0.0
+    ld = np.longdouble
+    na, nb = dens[2 * N:3 * N].astype(ld), dens[7 * N:8 * N].astype(ld)
+    n, pi = na + nb, ld("3.14159265358979323846264338327950288")
+    lo, hi = ld(cfg.p_nmin), ld(cfg.p_nmax)
+    far = np.asarray((n > hi) | (n < lo))    # (between them p_reg amplifies rounding)
+    on = n > hi
+    p = np.where(on, (na - nb) / n, ld(0))
+    hp, hm, g0, g1 = (1 + p) / 2, (1 - p) / 2, ld(0.357), ld(0.642)
+    t23, t53 = ld(2) / 3, ld(5) / 3
+    base = g0 + g1 * p * p - hp ** t53 - hm ** t53
+    s = 2 * g1 * p - ld(5) / 6 * (hp ** t23 - hm ** t23)
+    x = 6 * pi * pi * n
+    prm = tdgauss.to_params(cfg, td.FP64)
+    ctx = td.TDContext(prm, 4, 0)
+    dd, dp = cuda(torch, dens), cuda(torch, pots)
+    ctx.compute_potentials(1, dd, dp)
+    ctx.sync()
+    got = dp.cpu().numpy()
+    ctx.close()
+    err = []
+    for k, dpol in ((0, 2 * nb / n ** 2), (1, -2 * na / n ** 2)):
+        ref = x ** t23 / 2 * base + x ** t53 / (20 * pi * pi) * s * np.where(on, dpol, ld(0))
+        ref *= 1 - ld(0.25) ** 15
+        err.append(np.asarray(np.abs(got[k * N:(k + 1) * N] - ref) / np.abs(ref), dtype=float)[far])
+    q = np.median(np.concatenate(err))
+    assert q < np.finfo(float).eps, q
