@@ -97,6 +97,46 @@ def test_derivatives_2d_planes(torch, shape, m):
     ctx.close()
 
 
+@pytest.mark.parametrize("shape", [(32, 32), (32, 64), (64, 32), (64, 64)])
+def test_plane_laplacian_has_no_bias(torch, shape):
+    """<psi|lap psi> of smooth states: the rounding of the operator's tables is
+    the same at every point and in every state, so it does not average out as
+    that of the products does.  Against extended precision, the mean over 40
+    states: entries rounded as they come are off by 1.4e-16 to 3.8e-16, the
+    limit is half of the spacing of doubles at one."""
+    from wslda_amd import td
+    say("case: bias of the plane Laplacian shape=%s" % (shape,))
+    m, ld = 40, np.longdouble
+    nx, ny = shape
+    cfg = po.make_cfg(2, nx, ny, 4, dx=1.0)
+    r = np.random.default_rng(nx + 2 * ny)
+    f = np.zeros((m, nx, ny), dtype=complex)
+    for i in range(-4, 5):
+        for j in range(-4, 5):
+            f[:, i, j] = (r.normal(size=m) + 1j * r.normal(size=m)) * np.exp(-(i * i + j * j) / 4)
+    a = np.fft.ifft2(f).reshape(m, nx * ny)
+    a /= np.linalg.norm(a, axis=1)[:, None]
+    ctx = td.TDContext(tdgauss.to_params(cfg, td.FP64), m, 0)
+    t = cuda(torch, a)
+    out = [torch.zeros_like(t) for _ in range(3)]
+    ctx.compute_derivatives(t, out[0], out[1], None, out[2])
+    ctx.sync()
+    got = out[2].cpu().numpy()
+    ctx.close()
+    pi = ld("3.14159265358979323846264338327950288")
+
+    def second(L):   # the operator along an axis, in extended precision
+        q = np.where(np.arange(L) < L // 2, np.arange(L), np.arange(L) - L).astype(ld)
+        c = -((2 * pi * q / L) ** 2 * np.cos(2 * pi * ((np.outer(np.arange(L), np.arange(L)) % L).astype(ld)) / L)).sum(1) / L
+        return c[(np.arange(L)[:, None] - np.arange(L)[None, :]) % L]
+
+    A = a.astype(np.clongdouble).reshape(m, nx, ny)
+    ref = np.tensordot(second(nx), A, (1, 1)).transpose(1, 0, 2) + np.tensordot(A, second(ny), (2, 1))
+    off = (A.conj() * (got.reshape(m, nx, ny) - ref)).sum((1, 2)).real
+    say("mean %.2e" % float(off.mean()))
+    assert abs(float(off.mean())) < 0.5 * np.finfo(float).eps
+
+
 @pytest.mark.parametrize("shape", [(16, 16, 16), (16, 16, 18)])
 def test_one_timer_record_per_launch(torch, shape):
     """A compiled plane and one without: each launch is recorded once."""

@@ -246,7 +246,8 @@ ah_yz(const ac_t<SP> *__restrict__ y, const ac_t<SP> *__restrict__ T, ac_t<SP> *
 // faster.  Two waves per SIMD (244 registers), the FP64 pipe (products and
 // sums) busy three quarters of the time; without the factors and tables loaded
 // ahead of the products that hide them it took 1227 us.
-// mt: second- and first-derivative tables of y, then of z (d_mmt).
+// mt: second- and first-derivative tables of y, then of z (d_mmt); uy, uz: the
+// units of the former.
 // The tiles of a wave's points: row image h, column image g, offset i in the
 // plane and j in its LDS copy; rows are 4 apart, R of them inside the tile.
 #define MM_TILES(h, g, i, j)                                                                     \
@@ -258,7 +259,7 @@ template <int L>
 __global__ void __launch_bounds__(128, 2)
 ah_yz_mm(const double2 *__restrict__ y, const double2 *__restrict__ T, double2 *__restrict__ out,
          const double *__restrict__ pots, const double *__restrict__ hx, int n, long N, int NX,
-         const double *__restrict__ mt, double mu_a, double mu_b, double *__restrict__ part,
+         const double *__restrict__ mt, double uy, double uz, double mu_a, double mu_b, double *__restrict__ part,
          const double *__restrict__ sc)
 {
     constexpr int H = L / 2, RS = L + 1, E = L * L, EP = L * RS, R = (H + 3) / 4, NT = 128, MT = (L / 8) * 128;
@@ -336,6 +337,7 @@ ah_yz_mm(const double2 *__restrict__ y, const double2 *__restrict__ T, double2 *
 #pragma unroll
     for (int ax = 0; ax < 2; ax++) {
         const int xo = ax ? cl * RS + lr : lr * RS + cl;
+        const double q2 = q * (ax ? uz : uy);
         // psi: second derivative
         if (ax) mm_product<false, H, RS, H>(X + xo, t2, acc);
         else mm_product<true, H, RS, H>(X + xo, t2, acc);
@@ -347,7 +349,7 @@ ah_yz_mm(const double2 *__restrict__ y, const double2 *__restrict__ T, double2 *
                 const dbl4 im = ax ? mm_inner_at(acc, h, g, 1) : mm_outer_at(acc, h, g, 1);
 #pragma unroll
                 for (int r = 0; r < R; r++) {
-                    const double f = q * fa[h][g][r];
+                    const double f = q2 * fa[h][g][r];
                     ore[h][g][r] += f * re[r];
                     oim[h][g][r] += f * im[r];
                 }
@@ -389,8 +391,8 @@ ah_yz_mm(const double2 *__restrict__ y, const double2 *__restrict__ T, double2 *
         for (int h = 0; h < 2; h++)
 #pragma unroll
             for (int g = 0; g < 2; g++) {
-                ore[h][g] += (ax ? mm_inner_at(acc, h, g, 0) : mm_outer_at(acc, h, g, 0)) * q;
-                oim[h][g] += (ax ? mm_inner_at(acc, h, g, 1) : mm_outer_at(acc, h, g, 1)) * q;
+                ore[h][g] += (ax ? mm_inner_at(acc, h, g, 0) : mm_outer_at(acc, h, g, 0)) * q2;
+                oim[h][g] += (ax ? mm_inner_at(acc, h, g, 1) : mm_outer_at(acc, h, g, 1)) * q2;
                 mm_keep(ore[h][g]);
                 mm_keep(oim[h][g]);
             }
@@ -630,7 +632,7 @@ dg_yz(const ac_t<SP> *__restrict__ y, const double *__restrict__ fbeta, const do
 template <int L>
 __global__ void __launch_bounds__(64, 2)
 dg_yz_mm(const double2 *__restrict__ y, const double *__restrict__ fbeta, const double *__restrict__ wgt, int n, long N,
-         int NX, int G, const double *__restrict__ mt, double *__restrict__ part)
+         int NX, int G, const double *__restrict__ mt, double uy, double uz, double *__restrict__ part)
 {
     constexpr int H = L / 2, RS = L + 1, E = L * L, EP = L * RS, R = (H + 3) / 4, KM = E / 64, MT = (L / 8) * 128;
     static_assert(H % 4 == 0 && H <= 16 && E % 64 == 0, "one 16 x 16 tile per quarter plane");
@@ -674,6 +676,7 @@ dg_yz_mm(const double2 *__restrict__ y, const double *__restrict__ fbeta, const 
 #pragma unroll
         for (int ax = 0; ax < 2; ax++) {
             const double *m2 = mt + 2 * ax * MT + lane, *m1 = m2 + MT;
+            const double w2 = w * (ax ? uz : uy);
             const int xo = ax ? cl * RS + lr : lr * RS + cl;
             __builtin_amdgcn_sched_barrier(0);
             if (ax) mm_product<false, H, RS, H>(X + xo, m2, acc);
@@ -683,7 +686,7 @@ dg_yz_mm(const double2 *__restrict__ y, const double *__restrict__ fbeta, const 
                 const dbl4 im = ax ? mm_inner_at(acc, h, g, 1) : mm_outer_at(acc, h, g, 1);
 #pragma unroll
                 for (int r = 0; r < R; r++) {
-                    ta[h][g][r] += cmulc(X[j + 4 * r * RS], make_double2(re[r], im[r])).x * w;
+                    ta[h][g][r] += cmulc(X[j + 4 * r * RS], make_double2(re[r], im[r])).x * w2;
                     mm_keep(ta[h][g][r]);
                 }
             }
@@ -725,7 +728,12 @@ int aslda_setup(tdw_ctx *c)
     if (!amm_plane(c)) return 0;
     std::vector<double> t;
     for (int d = 1; d < 3; d++)
-        for (int order = 2; order > 0; order--) mm_tables(c->ny, c->Lphys[d], order, t);
+        for (int order = 2; order > 0; order--) {
+            // (the first derivatives unscaled: a multiplication per point, 0.9 %
+            // of an ASLDA step, that no result was more exact for)
+            const double u = mm_tables(c->ny, c->Lphys[d], order, t, order == 2);
+            if (order == 2) c->mmt_unit[d - 1] = u;
+        }
     TDW_HIP(hipMalloc(&c->d_mmt, sizeof(double) * t.size()));
     return (int)hipMemcpy(c->d_mmt, t.data(), sizeof(double) * t.size(), hipMemcpyHostToDevice);
 }
@@ -858,7 +866,7 @@ static int dens_grad_t(tdw_ctx *c, int n, const ac_t<SP> *wf, const double *fbet
             mm = true;
             const auto fm = c->ny == 24 ? dg_yz_mm<24> : dg_yz_mm<32>;
             hipLaunchKernelGGL(fm, dim3((unsigned)(2L * nchunk * c->nx)), dim3(64), 0, c->stream, wf, fbeta, wgt, n, N,
-                               c->nx, G, c->d_mmt, pyz_part);
+                               c->nx, G, c->d_mmt, c->mmt_unit[0], c->mmt_unit[1], pyz_part);
         }
     if (!mm)
         hipLaunchKernelGGL(fy, dim3((unsigned)((long)nchunk * c->nx)), dim3(nt), lds, c->stream, wf, fbeta, wgt, n, N,
@@ -914,7 +922,8 @@ static int aslda_h_t(tdw_ctx *c, int n, const ac_t<SP> *in, ac_t<SP> *out, ac_t<
             if (c->d_mmt) {
                 const auto fm = c->ny == 24 ? ah_yz_mm<24> : ah_yz_mm<32>;
                 hipLaunchKernelGGL(fm, dim3((unsigned)((long)n * c->nx)), dim3(128), lds, c->stream, in, T, out, pots,
-                                   hx, n, N, c->nx, c->d_mmt, c->p.mu_a, c->p.mu_b, part, sc);
+                                   hx, n, N, c->nx, c->d_mmt, c->mmt_unit[0], c->mmt_unit[1], c->p.mu_a, c->p.mu_b, part,
+                                   sc);
                 return row_sums(c, part, n, c->nx, dvol_norm(c), d_qpe);
             }
         hipLaunchKernelGGL(fy, dim3((unsigned)((long)n * c->nx)), dim3(nt), lds, c->stream, in, T, out, pots, hx, n, N,

@@ -69,6 +69,7 @@ struct tdw_ctx {
     double *d_adjv;                      // 4n per-state scalars of the backward step
     // derivative tables of FP64 yz planes on the matrix cores (tdw_aslda.hip), or null
     double *d_mmt;
+    double mmt_unit[2];                  // units of the second-derivative tables of y, z
     // ASLDA (allocated on first use)
     double *d_hx;                        // 4N: lap alpha_a, lap alpha_b, div A_a, div A_b
     double2 *d_ascr;                     // 34N complex: the real fields of H and their derivatives

@@ -40,6 +40,7 @@ struct RsPlan {
     int dim, inner, npc, ll;      // points per x plane (padded), padded points per component, last axis length
     unsigned mll;                 // division by the last axis length
     RsAxis ax[3];
+    MmScale mm;                   // of the matrix-core planes
 };
 
 // Laplacian of both components in LDS, in place: the factor
@@ -221,7 +222,7 @@ template <int LX, int LY, int CORR>
 __global__ void __launch_bounds__(64 * 2 * (LX / 32) * (LY / 32), 2)
 rs_mm(const double2 *in, double2 *out, const double2 *__restrict__ c, const double *__restrict__ pots,
       const double *__restrict__ sc, const double *__restrict__ kt, int n, RsH hp, const double *__restrict__ mx,
-      const double *__restrict__ my, const double *use_e, double *e_out, double *e_out2, double *__restrict__ nrm_out)
+      const double *__restrict__ my, double rx, double ry, const double *use_e, double *e_out, double *e_out2, double *__restrict__ nrm_out)
 {
     constexpr int HX = LX / 2, HY = LY / 2, TX = HX / 16, TY = HY / 16, W = 2 * TX * TY, NT = 64 * W;
     constexpr int N = LX * LY, RS = LY + 1, NPC = LX * RS;
@@ -248,8 +249,8 @@ rs_mm(const double2 *in, double2 *out, const double2 *__restrict__ c, const doub
     for (int h = 0; h < 2; h++)
 #pragma unroll
         for (int g = 0; g < 2; g++) {
-            lre[h][g] = mm_outer_at(acc, h, g, 0);
-            lim[h][g] = mm_outer_at(acc, h, g, 1);
+            lre[h][g] = mm_outer_at(acc, h, g, 0) * rx;
+            lim[h][g] = mm_outer_at(acc, h, g, 1) * rx;
         }
     __builtin_amdgcn_sched_barrier(0);
     mm_product<false, HY, RS, HX>(X + (16 * tx + lc) * RS + lr, my + (long)ty * (HY / 4) * 128 + lane, acc);
@@ -257,8 +258,8 @@ rs_mm(const double2 *in, double2 *out, const double2 *__restrict__ c, const doub
     for (int h = 0; h < 2; h++)
 #pragma unroll
         for (int g = 0; g < 2; g++) {
-            lre[h][g] += mm_inner_at(acc, h, g, 0);
-            lim[h][g] += mm_inner_at(acc, h, g, 1);
+            lre[h][g] += mm_inner_at(acc, h, g, 0) * ry;
+            lim[h][g] += mm_inner_at(acc, h, g, 1) * ry;
         }
     const double k2t = kt ? kt[a] * kt[a] : 0.0;
     const long own = cmp ? gv : gu;
@@ -350,7 +351,7 @@ rs_mm(const double2 *in, double2 *out, const double2 *__restrict__ c, const doub
 // ---------------------------------------------------------------------------
 template <int LX, int LY>
 __global__ void __launch_bounds__(64 * (LX / 32) * (LY / 32), 2)
-rs_deriv(const double2 *in, double2 *ddx, double2 *ddy, double2 *lap, const double *__restrict__ tab)
+rs_deriv(const double2 *in, double2 *ddx, double2 *ddy, double2 *lap, const double *__restrict__ tab, MmScale sc)
 {
     constexpr int HX = LX / 2, HY = LY / 2, TX = HX / 16, TY = HY / 16, NT = 64 * TX * TY;
     constexpr int N = LX * LY, RS = LY + 1, MX = TX * (LX / 8) * 128, MY = TY * (LY / 8) * 128;
@@ -371,7 +372,7 @@ rs_deriv(const double2 *in, double2 *ddx, double2 *ddy, double2 *lap, const doub
     for (int h = 0; h < 2; h++)
 #pragma unroll
         for (int g = 0; g < 2; g++) {
-            const dbl4 re = mm_outer_at(acc, h, g, 0), im = mm_outer_at(acc, h, g, 1);
+            const dbl4 re = mm_outer_at(acc, h, g, 0) * sc.s[0][1], im = mm_outer_at(acc, h, g, 1) * sc.s[0][1];
 #pragma unroll
             for (int r = 0; r < 4; r++) ddx[o + (h * HX + 4 * r) * LY + g * HY] = make_double2(re[r], im[r]);
         }
@@ -381,7 +382,7 @@ rs_deriv(const double2 *in, double2 *ddx, double2 *ddy, double2 *lap, const doub
     for (int h = 0; h < 2; h++)
 #pragma unroll
         for (int g = 0; g < 2; g++) {
-            const dbl4 re = mm_inner_at(acc, h, g, 0), im = mm_inner_at(acc, h, g, 1);
+            const dbl4 re = mm_inner_at(acc, h, g, 0) * sc.s[1][1], im = mm_inner_at(acc, h, g, 1) * sc.s[1][1];
 #pragma unroll
             for (int r = 0; r < 4; r++) ddy[o + (h * HX + 4 * r) * LY + g * HY] = make_double2(re[r], im[r]);
         }
@@ -391,8 +392,8 @@ rs_deriv(const double2 *in, double2 *ddx, double2 *ddy, double2 *lap, const doub
     for (int h = 0; h < 2; h++)
 #pragma unroll
         for (int g = 0; g < 2; g++) {
-            lre[h][g] = mm_outer_at(acc, h, g, 0);
-            lim[h][g] = mm_outer_at(acc, h, g, 1);
+            lre[h][g] = mm_outer_at(acc, h, g, 0) * sc.s[0][0];
+            lim[h][g] = mm_outer_at(acc, h, g, 1) * sc.s[0][0];
         }
     __builtin_amdgcn_sched_barrier(0);
     mm_product<false, HY, RS, HX>(xi, my, acc);
@@ -400,7 +401,8 @@ rs_deriv(const double2 *in, double2 *ddx, double2 *ddy, double2 *lap, const doub
     for (int h = 0; h < 2; h++)
 #pragma unroll
         for (int g = 0; g < 2; g++) {
-            const dbl4 re = lre[h][g] + mm_inner_at(acc, h, g, 0), im = lim[h][g] + mm_inner_at(acc, h, g, 1);
+            const dbl4 re = lre[h][g] + mm_inner_at(acc, h, g, 0) * sc.s[1][0],
+                       im = lim[h][g] + mm_inner_at(acc, h, g, 1) * sc.s[1][0];
 #pragma unroll
             for (int r = 0; r < 4; r++) lap[o + (h * HX + 4 * r) * LY + g * HY] = make_double2(re[r], im[r]);
         }
@@ -466,7 +468,7 @@ int resident_setup(tdw_ctx *c)
     // the halves of the second-derivative circulants in rs_mm's operand order
     if (mm_plane(c))
         for (int d = 0; d < 2; d++)
-            for (int order = 2; order > 0; order--) mm_tables(len[d], c->Lphys[d], order, kt);
+            for (int order = 2; order > 0; order--) pl.mm.s[d][2 - order] = mm_tables(len[d], c->Lphys[d], order, kt);
     const size_t btw = sizeof(double2) * tw.size(), bk = sizeof(double) * kt.size();
     TDW_HIP(hipMalloc(&c->d_rtab, btw + bk));
     TDW_HIP(hipMemcpy(c->d_rtab, tw.data(), btw, hipMemcpyHostToDevice));
@@ -521,8 +523,8 @@ static int launch_h(tdw_ctx *c, int n, const double2 *in, double2 *out, const do
         const dim3 g(n), b(128 * (c->nx / 32) * (c->ny / 32));
         const size_t sm = sizeof(double2) * 2 * (size_t)pl.npc;
 #define RS_MM(LX, LY)                                                                                               \
-    hipLaunchKernelGGL((rs_mm<LX, LY, CORR>), g, b, sm, c->stream, in, out, cc, pots, sc, kt, n, hp, mx, my, use_e, \
-                       e_out, e_out2, nrm_out)
+    hipLaunchKernelGGL((rs_mm<LX, LY, CORR>), g, b, sm, c->stream, in, out, cc, pots, sc, kt, n, hp, mx, my, \
+                       pl.mm.s[0][0], pl.mm.s[1][0], use_e, e_out, e_out2, nrm_out)
         if (c->nx == 32) {
             if (c->ny == 32) RS_MM(32, 32);
             else RS_MM(32, 64);
@@ -548,7 +550,7 @@ int plane_derivatives(tdw_ctx *c, int m, const double2 *in, double2 *ddx, double
                                 : (c->ny == 32 ? rs_deriv<64, 32> : rs_deriv<64, 64>);
     TDW_TIMED(c, "rs_deriv");
     hipLaunchKernelGGL(fn, dim3((unsigned)m), dim3(64 * (c->nx / 32) * (c->ny / 32)), sizeof(double2) * (size_t)pl.npc,
-                       c->stream, in, ddx, ddy, lap, tab);
+                       c->stream, in, ddx, ddy, lap, tab, pl.mm);
     return (int)hipGetLastError();
 }
 
