@@ -126,3 +126,39 @@ def test_step_leaves_the_laplacian(torch, dim, shape, n):
     po.lib().tdwo_laplace(C.byref(cfg), 2 * n, po.ptr(y), po.ptr(ref))
     # (relative to the largest: the highest modes carry the rounding)
     assert np.abs(got - ref).max() <= TOL * np.abs(ref).max()
+
+
+@pytest.mark.parametrize("shape", [(36, 18, 4), (18, 36, 4), (24, 36, 4), (48, 54, 4), (16, 16, 4)])
+def test_transforms_are_as_exact_as_their_twiddles(torch, shape):
+    """The Laplacian that a step leaves, of states with all modes, against
+    extended precision: with correctly rounded twiddles its relative error (of
+    the 2-norm) is below two units of rounding on axes with factors of 3 as on
+    powers of two; radices 6 and 9 whose twiddles are off by three units give
+    2.4 to 2.5."""
+    from wslda_amd import td
+    say("case: transform accuracy shape=%s" % (shape,))
+    n, ld = 60, np.longdouble
+    nx, ny = shape[:2]
+    cfg, wf, fb, kt, cnt, pots = problem(2, shape, n, po.AB4AM5, po.SLDA)
+    ctx = td.TDContext(tdgauss.to_params(cfg, td.FP64), n, 0)
+    ctx.set_states(fb, kt, cnt)
+    R = td.TDRun(ctx, wf, pots)
+    R.initial_measure()
+    R.step(0)
+    ctx.sync()
+    got, y = R.lap.cpu().numpy(), R.wf.cpu().numpy()
+    ctx.close()
+    pi = ld("3.14159265358979323846264338327950288")
+
+    def second(L, dx):   # the operator along an axis, in extended precision
+        i = np.arange(L)
+        k = 2 * pi * np.where(i < L // 2, i, i - L).astype(ld) / (L * ld(dx))
+        c = -(k ** 2 * np.cos(2 * pi * (np.outer(i, i) % L).astype(ld) / L)).sum(1) / L
+        return c[(i[:, None] - i[None, :]) % L]
+
+    A = y.astype(np.clongdouble).reshape(2 * n, nx, ny)
+    ref = np.tensordot(second(nx, 1.1), A, (1, 1)).transpose(1, 0, 2) + np.tensordot(A, second(ny, 0.9), (2, 1))
+    ref = ref.reshape(2 * n, -1)
+    err = float(np.sqrt((np.abs(got - ref) ** 2).sum() / (np.abs(ref) ** 2).sum()))
+    say("%.2e" % err)
+    assert err < 2 * np.finfo(float).eps

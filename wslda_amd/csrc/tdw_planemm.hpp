@@ -130,7 +130,7 @@ static inline size_t mm_doubles(int L) { return (size_t)mm_tiles(L) * (L / 8) * 
 // the FFT's was 1.1e-14.  Two or three of the entries are nearly all of it, so
 // a scale is chosen with which those are nearly exact: of 4e9 values in [1, 2)
 // (6e9 for 64 points) the one with the least rms rounding over all entries,
-// 14 to 140 times below that of scale 1.
+// 7 to 140 times below that of scale 1.
 static inline double mm_unit(int L, int order)
 {
     switch (L) {
