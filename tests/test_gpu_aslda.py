@@ -359,6 +359,55 @@ def test_aslda_h_two_pass_equals_modular(torch, shape):
     ctx.close()
 
 
+def test_aslda_fields_of_large_lattices(torch):
+    """The grid fields of H and tau where they are transformed one at a time
+    (above 2^20 points) equal those of a quarter of the lattice, repeated four
+    times along x, where they go together; and their scratch stays that of one
+    field."""
+    from wslda_amd import td
+    say("case: ASLDA fields of 512 x 48 x 48 points")
+    outs = []
+    for rep in (1, 4):
+        nx, ny, nz = 128 * rep, 48, 48
+        cfg = po.make_cfg(3, nx, ny, nz, dx=1.1, functional=po.ASLDA)
+        cfg.mu_a, cfg.mu_b = 0.3, 0.25
+        N = nx * ny * nz
+        x = torch.arange(nx, device="cuda:0", dtype=torch.float64)[:, None, None] * (2 * np.pi / 128)
+        y = torch.arange(ny, device="cuda:0", dtype=torch.float64)[None, :, None] * (2 * np.pi / ny)
+        z = torch.arange(nz, device="cuda:0", dtype=torch.float64)[None, None, :] * (2 * np.pi / nz)
+        smooth = lambda p: (torch.sin(3 * x + p) * torch.cos(2 * y - p) + 0.5 * torch.cos(z + 2 * p)).reshape(-1)
+        W = torch.stack([torch.complex(smooth(0.1 + k), smooth(0.6 + k)) for k in range(2)])
+        pots = torch.stack([0.1 * smooth(0.3 + k) for k in range(12)])
+        pots[4:6] += 1.0
+        pots[2:4] = torch.stack([pots[2], pots[3]], 1).reshape(2, N)   # Delta, complex
+        dens = torch.stack([0.02 + 0.001 * smooth(0.2 + k) for k in range(12)])
+        dens[[3, 8]] *= -1.0   # tau = lap rho / 2 - these, positive
+        pots, dens = pots.reshape(-1).contiguous(), dens.reshape(-1).contiguous()
+        ctx = td.TDContext(tdgauss.to_params(cfg), 1, 0)
+        ctx.set_states(np.ones(1))
+        D = [torch.zeros_like(W) for _ in range(5)]
+        ctx.compute_derivatives(W, *D[:4])
+        ctx.multiply_wf_by_alpha(W, D[4], pots)
+        ctx.compute_laplace(D[4], D[4])
+        out, q = torch.zeros_like(W), torch.zeros(1, dtype=torch.float64, device="cuda:0")
+        ctx.sync()
+        free = torch.cuda.mem_get_info(0)[0]
+        ctx.apply_hamiltonian_full(0, W, out, *D[:4], D[4], pots, qpe=q)
+        td.check(ctx.L.tdw_density_tau(ctx.h, dens.data_ptr()), "tau")
+        ctx.sync()
+        grown = free - torch.cuda.mem_get_info(0)[0]
+        ctx.close()
+        out = out + W * q[0]   # H psi without the subtraction, which sums over the lattice
+        o = torch.cat([torch.view_as_real(out).permute(0, 2, 1).reshape(4, N), dens.reshape(12, N)])
+        outs.append(o.reshape(16, rep, -1, ny * nz))
+    assert grown < 16 * N * 16
+    small, large = outs
+    assert float(small[[7, 12]].min()) > 0.0   # tau of both spins
+    for r in range(4):
+        err = (large[:, r] - small[:, 0]).abs().amax((1, 2)) / small[:, 0].abs().amax((1, 2))
+        assert float(err.max()) < TOL, (r, err)
+
+
 @pytest.mark.parametrize("shape,n", [((12, 12, 12), 40), ((16, 16, 16), 24), ((24, 24, 24), 70), ((32, 32, 32), 8)])
 def test_densities_gradients_in_passes(torch, shape, n):
     """Densities with gradients formed inside the x / yz density passes

@@ -198,7 +198,7 @@ extern "C" int tdw_create(const tdw_params *p, int nwf, int device, tdw_ctx **ou
     if (!e) e = (int)hipMalloc(&c->d_qpe, sizeof(double) * nwf);
     if (!e) e = (int)hipMalloc(&c->d_scale, sizeof(double) * nwf);
     if (!e) e = (int)hipMalloc(&c->d_esum, sizeof(double) * 64);
-    if (!e) e = (int)hipMalloc(&c->d_rtmp, sizeof(double2) * 2 * c->N);
+    if (!e) e = (int)hipMalloc(&c->d_rtmp, sizeof(double2) * (c->N > FIELDS_AT_ONCE ? 1 : 2) * c->N);
     if (!e) e = (int)hipMalloc(&c->d_vext, sizeof(double) * 2 * c->N);
     if (!e) e = (int)hipMemset(c->d_kt, 0, sizeof(double) * 2 * nwf);
     if (!e) e = noalloc_setup(device);

@@ -53,7 +53,7 @@ struct tdw_ctx {
     double *d_qpe;                       // n <H>
     double *d_esum;                      // energies (TDW_NITEMS)
     double2 *d_T;    size_t T_cap;       // laplacian scratch (complex elements)
-    double2 *d_rtmp;                     // 2N complex (real-field transforms)
+    double2 *d_rtmp;                     // 2N complex, N beyond FIELDS_AT_ONCE (real-field transforms)
     double *d_vext;                      // 2N
     void *ref_workarea;                  // set_workspace_for_cufftPlan()
     // fused-path state
@@ -72,7 +72,8 @@ struct tdw_ctx {
     double mmt_unit[2];                  // units of the second-derivative tables of y, z
     // ASLDA (allocated on first use)
     double *d_hx;                        // 4N: lap alpha_a, lap alpha_b, div A_a, div A_b
-    double2 *d_ascr;                     // 34N complex: the real fields of H and their derivatives
+    double2 *d_ascr;                     // the real fields of H and their derivatives: 34N complex, 4N beyond
+                                         // FIELDS_AT_ONCE
     double2 *d_aw;   size_t aw_cap;      // lap(alpha psi) (complex elements)
     // grid-field helpers (tdw_grid.hip, allocated on first use)
     double2 *d_gscr;                     // 6N complex
@@ -101,6 +102,12 @@ namespace tdw {
 // The functionals whose effective mass varies in space: the step takes
 // derivatives on every half-step and H carries the alpha, A terms
 // (ASLDA; SLDAE unless built with SLDA_FORCE_A1).
+// Up to this many points the real fields of a step (two densities, eight
+// fields of H) go through the transforms together, from scratch arrays for
+// all; beyond it one at a time, in the scratch of one.  Launches count on small
+// lattices (48^3: aslda_fields 65 us, 543 one by one) and less on large ones
+// (256 x 48 x 48: 420 and 652), where the scratch grows: 570 MB at the line.
+constexpr size_t FIELDS_AT_ONCE = (size_t)1 << 20;
 inline bool varying_mass(const tdw_ctx *c)
 {
     return c->p.functional == TDW_ASLDA || (c->p.functional == TDW_SLDAE && !c->p.force_a1);

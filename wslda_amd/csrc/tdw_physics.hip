@@ -634,15 +634,19 @@ int density_tau(tdw_ctx *c, double *dens)
     TimingOff quiet(c);
     long N = (long)c->N;
     // b component first, then a (pca_dens.cu:317-333), both through the
-    // transforms at once; in spin-symmetric mode tau_a is a copy of tau_b
-    // (pca_dens.cu:329-331)
-    const int m = c->p.spinsymmetry ? 1 : 2;
-    const long tot = m * N;
+    // transforms at once up to FIELDS_AT_ONCE; in spin-symmetric mode tau_a is
+    // a copy of tau_b (pca_dens.cu:329-331)
+    const int m = c->p.spinsymmetry ? 1 : 2, at = c->N > FIELDS_AT_ONCE ? 1 : m;
+    const long tot = at * N;
     TDW_TRY(ensure_T(c, (size_t)tot));
     const dim3 g((tot + NT - 1) / NT);
-    hipLaunchKernelGGL(k_rho2cplx, g, dim3(NT), 0, c->stream, dens + 7 * N, dens + 2 * N, c->d_rtmp, N, tot);
-    TDW_TRY(laplace(c, m, c->d_rtmp, c->d_T));
-    hipLaunchKernelGGL(k_tau, g, dim3(NT), 0, c->stream, c->d_T, dens + 8 * N, dens + 3 * N, N, tot);
+    for (int k = 0; k < m; k += at) {
+        const double *rho = dens + (k ? 2 : 7) * N;
+        double *tau = dens + (k ? 3 : 8) * N;
+        hipLaunchKernelGGL(k_rho2cplx, g, dim3(NT), 0, c->stream, rho, dens + 2 * N, c->d_rtmp, N, tot);
+        TDW_TRY(laplace(c, at, c->d_rtmp, c->d_T));
+        hipLaunchKernelGGL(k_tau, g, dim3(NT), 0, c->stream, c->d_T, tau, dens + 3 * N, N, tot);
+    }
     if (c->p.spinsymmetry) return copy_f64(c, dens + 8 * N, dens + 3 * N, N);
     return (int)hipGetLastError();
 }
@@ -915,12 +919,21 @@ k_hx(const double2 *__restrict__ lap, const double2 *__restrict__ gx, const doub
     }
 }
 
+// acc = Re(dd) (first) or acc += Re(dd)
+__global__ void __launch_bounds__(NT)
+k_re_acc(const double2 *__restrict__ dd, double *__restrict__ acc, long N, int first)
+{
+    const long i = (long)blockIdx.x * NT + threadIdx.x;
+    if (i >= N) return;
+    acc[i] = first ? dd[i].x : acc[i] + dd[i].x;
+}
+
 static int ensure_aslda(tdw_ctx *c)
 {
     const size_t N = c->N;
     if (!c->d_hx) TDW_HIP(hipMalloc(&c->d_hx, sizeof(double) * 4 * N));
-    // 8 fields, 2 Laplacians, 4 x 6 derivative arrays
-    if (!c->d_ascr) TDW_HIP(hipMalloc(&c->d_ascr, sizeof(double2) * 34 * N));
+    // 8 fields, 2 Laplacians, 4 x 6 derivative arrays, or the latter of one field
+    if (!c->d_ascr) TDW_HIP(hipMalloc(&c->d_ascr, sizeof(double2) * (N > FIELDS_AT_ONCE ? 4 : 34) * N));
     return 0;
 }
 
@@ -929,13 +942,28 @@ static int ensure_aslda(tdw_ctx *c)
 // Nyquist derivative set to zero, pca_kernels.cu:700-760).  The eight fields
 // follow one another in the potential block and go through the transforms
 // together: six launches instead of thirty-two of a few microseconds each
-// (24^3 x 2048 ASLDA step 7.62 -> 7.31 ms, with the same for tau).
+// (24^3 x 2048 ASLDA step 7.62 -> 7.31 ms, with the same for tau); one by one
+// beyond FIELDS_AT_ONCE.
 int aslda_fields(tdw_ctx *c, const double *pots)
 {
     TDW_TRY(ensure_aslda(c));
     TDW_TIMED(c, "aslda_fields");
     TimingOff quiet(c);
     const long N = (long)c->N;
+    if (c->N > FIELDS_AT_ONCE) {
+        TDW_TRY(laplace_real(c, pots + 4 * N, c->d_hx));
+        TDW_TRY(laplace_real(c, pots + 5 * N, c->d_hx + N));
+        const dim3 grid((N + NT - 1) / NT);
+        double2 *g = c->d_ascr;
+        for (int k = 0; k < 6; k++) {
+            const int d = k % 3;
+            if (d >= c->dim) continue;
+            hipLaunchKernelGGL(k_real2cplx, grid, dim3(NT), 0, c->stream, pots + (6 + k) * N, c->d_rtmp, N);
+            TDW_TRY(derivatives(c, 1, c->d_rtmp, g, g + N, g + 2 * N, g + 3 * N));
+            hipLaunchKernelGGL(k_re_acc, grid, dim3(NT), 0, c->stream, g + d * N, c->d_hx + (2 + k / 3) * N, N, d == 0);
+        }
+        return (int)hipGetLastError();
+    }
     double2 *z = c->d_ascr, *lap = z + 8 * N, *g = lap + 2 * N;
     hipLaunchKernelGGL(k_real2cplx, dim3((8 * N + NT - 1) / NT), dim3(NT), 0, c->stream, pots + 4 * N, z, 8 * N);
     TDW_TRY(laplace(c, 2, z, lap));
