@@ -377,6 +377,7 @@ def test_aslda_fields_of_large_lattices(torch):
         z = torch.arange(nz, device="cuda:0", dtype=torch.float64)[None, None, :] * (2 * np.pi / nz)
         smooth = lambda p: (torch.sin(3 * x + p) * torch.cos(2 * y - p) + 0.5 * torch.cos(z + 2 * p)).reshape(-1)
         W = torch.stack([torch.complex(smooth(0.1 + k), smooth(0.6 + k)) for k in range(2)])
+        W /= (128 * ny * nz * 1.1 ** 3) ** 0.5   # <H>, subtracted below, of order one
         pots = torch.stack([0.1 * smooth(0.3 + k) for k in range(12)])
         pots[4:6] += 1.0
         pots[2:4] = torch.stack([pots[2], pots[3]], 1).reshape(2, N)   # Delta, complex
