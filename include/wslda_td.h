@@ -245,9 +245,12 @@ int tdw_step(tdw_ctx *c, tdw_state *s, int it, int grad_last);
  * constant effective mass whose state fits in LDS (1D, 2D, and 3D lattices
  * with fused passes up to 16^3) run the resident step, which leaves nothing to
  * complete; those with axes of 18, 36 and 48 points run the six passes,
- * completed at each step's end.  Other lattices run the modular step.
+ * completed at each step's end.  Other lattices, and those three lengths in a
+ * project build with modify_potentials, run the modular step.
  * tdw_fused_supported() says whether the lattice is one of those with fused
- * passes in both precisions.
+ * passes in both precisions; these take the effective masses as 1 along x
+ * (SLDA's are), the other forms as the potential block has them.  On 3D
+ * lattices lap is scratch.
  *
  * Split precision (params.precision == TDW_SPLIT): the x / yz FFTs and the
  * kinetic term run in FP32 complex, and f[0..4] hold FP32 complex values

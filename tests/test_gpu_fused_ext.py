@@ -55,3 +55,33 @@ def test_extended_fused_step_vs_oracle(torch, shape, n, scheme, functional):
     with pytest.raises(td.TDWError):
         R.step(0)
     ctx.close()
+
+
+@pytest.mark.parametrize("shape,n", [((18, 18, 18), 7), ((36, 36, 36), 2), ((48, 24, 24), 3), ((24, 36, 36), 2),
+                                     ((48, 8, 12), 6)])
+def test_extended_fused_step_takes_the_masses_given(torch, shape, n):
+    """alpha_a, alpha_b of the potential block enter H as the caller gives
+    them, along x too: different for the components, varying in space."""
+    from wslda_amd import td
+    say("case: extended fused step with masses, shape=%s n=%d" % (shape, n))
+    cfg, wf, fb, kt, cnt, pots = problem(3, shape, n, po.AB4AM5, po.SLDA)
+    N = po.npts(cfg)
+    X = np.meshgrid(*[2 * np.pi * np.arange(L) / L for L in shape], indexing="ij")
+    w = (np.sin(X[0]) * np.cos(X[1]) + 0.5 * np.cos(X[2])).ravel()
+    pots[4 * N:5 * N], pots[5 * N:6 * N] = 1.1 + 0.1 * w, 0.9 - 0.1 * w
+    P = po.Problem(cfg, wf.copy(), fb, kt=kt, cnt=cnt, pots=pots.copy())
+    ctx = td.TDContext(tdgauss.to_params(cfg, td.FP64), n, 0)
+    ctx.set_states(fb, kt, cnt)
+    R = td.TDRun(ctx, wf, pots, fused=True)
+    P.initial_measure()
+    R.initial_measure()
+    emax = 3 * 0.5 * (np.pi / 0.9) ** 2 * np.abs(P.wf).max()
+    for it in range(4):
+        P.step(it, grad_last=it == 2)
+        R.step(it, grad_last=it == 2)
+        ctx.sync()
+        assert rel(R.wf.cpu().numpy(), P.wf) < TOL, it
+        assert rel(R.dens.cpu().numpy(), P.dens) < TOL, it
+        assert rel(R.qpe.cpu().numpy(), P.qpe) < TOL, it
+        assert np.abs(R.history()[0].cpu().numpy() - P.history()[0]).max() < TOL * emax, it
+    ctx.close()

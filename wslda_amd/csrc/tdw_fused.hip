@@ -81,6 +81,36 @@ __device__ __forceinline__ void xkin_inplace(C (&r)[LX], double sig_kscale_half,
     rf::fft<LX, +1, C>(r);
 }
 
+// The effective masses of an SLDA run are the caller's (alpha = 1 in earnest)
+// and enter H as they are.  The x passes of the lattices of fused_ext take
+// them into account: a pass over alpha_a, alpha_b at the step's start says
+// whether they are 1 (one flag per workgroup), and of two forms of each x pass,
+// AL_ONE and AL_ANY, the one that does not apply ends at once (5 us of a step
+// of 3.9 ms).  AL_ANY forms the x part of H psi and of <H> point by point
+// instead of by Parseval; in one kernel with the other it took its registers
+// (48 points: 1.9 KB of scratch per lane).
+static constexpr int ONE_BLOCKS = 64;
+struct XAlpha {
+    const double *al;   // alpha_a, alpha_b (2N), null: 1
+    const int *one;     // ONE_BLOCKS flags
+};
+
+__global__ void __launch_bounds__(FT) f_alpha_one(const double *__restrict__ al, long n2, int *__restrict__ one)
+{
+    int ok = 1;
+    for (long i = (long)blockIdx.x * FT + threadIdx.x; i < n2; i += (long)ONE_BLOCKS * FT) ok &= al[i] == 1.0;
+    ok = __syncthreads_and(ok);
+    if (threadIdx.x == 0) one[blockIdx.x] = ok;
+}
+
+// whether the form AL of an x pass runs (for whole waves)
+enum { AL_NONE, AL_ONE, AL_ANY };
+template <int AL> __device__ __forceinline__ bool alpha_form(const XAlpha &xa)
+{
+    if constexpr (AL == AL_NONE) return true;
+    return (!xa.al || __all(xa.one[threadIdx.x & (ONE_BLOCKS - 1)])) == (AL == AL_ONE);
+}
+
 // sum_x conj(y) sigma (-1/2 D_x) y of a pencil by Parseval, sigma kscale / 2
 // sum_m m^2 |Y_m|^2 (r is transformed in place)
 template <int LX, typename C>
@@ -94,6 +124,21 @@ __device__ __forceinline__ double xkin_energy(C (&r)[LX], double sig_kscale_half
         x += (double)(mm * mm) * cnorm(to64(r[m]));
     }
     return x * sig_kscale_half;
+}
+
+// the same with alpha: r is transformed back, y the pencil in memory
+template <int LX>
+__device__ __forceinline__ double xkin_energy_alpha(double2 (&r)[LX], double sig_kscale_half, const double2 *y,
+                                                    const double *al, int S)
+{
+    xkin_inplace<LX>(r, sig_kscale_half, 0.0);
+    double x = 0.0;
+#pragma unroll
+    for (int i = 0; i < LX; i++) {
+        x += al[(long)i * S] * cmulc(y[(long)i * S], r[i]).x;
+        if (i % 4 == 3) __builtin_amdgcn_sched_barrier(0);
+    }
+    return x;
 }
 
 // ---------------------------------------------------------------------------
@@ -124,13 +169,15 @@ constexpr int x_waves(int LX) { return LX >= 36 ? 2 : 1; }
 
 template <int LX> constexpr bool pred_hold() { return LX <= 24; }
 
-template <int LX, int SCH, bool SP>
+template <int LX, int SCH, bool SP, int AL = AL_NONE>
 __global__ void __launch_bounds__(FT, x_waves(LX))
 f_pred(double2 *__restrict__ y, hc_t<SP> *f1, const hc_t<SP> *f2, const hc_t<SP> *f3, const hc_t<SP> *f4,
        const hc_t<SP> *f5, hc_t<SP> *fold, double *__restrict__ xpart,
        const double *__restrict__ sk, const double *__restrict__ ek, int pending, int n, long N, int S, double dt,
-       double kscale, int wave, double *__restrict__ part)
+       double kscale, int wave, double *__restrict__ part, XAlpha xa)
 {
+    if (!alpha_form<AL>(xa)) return;
+    if constexpr (AL != AL_NONE) pending = 0;   // these lattices' steps are completed
     typedef hc_t<SP> HC;
     const long P = (long)blockIdx.x * FT + threadIdx.x;
     const long Ptot = 2L * n * S;
@@ -186,7 +233,8 @@ f_pred(double2 *__restrict__ y, hc_t<SP> *f1, const hc_t<SP> *f2, const hc_t<SP>
             nrm += cnorm(yp);
             if (i % 4 == 3) __builtin_amdgcn_sched_barrier(0);
         }
-        xk = xkin_energy<LX>(r, skh);
+        if constexpr (AL == AL_ANY) xk = xkin_energy_alpha<LX>(r, skh, y + base, xa.al + (a2 < n ? 0 : N) + j, S);
+        else xk = xkin_energy<LX>(r, skh);
     }
     put_norm_part(nrm, wave != 0, P, Ptot, part);
     put_norm_part(xk, wave != 0, P, Ptot, xpart);
@@ -206,12 +254,13 @@ f_pred(double2 *__restrict__ y, hc_t<SP> *f1, const hc_t<SP> *f2, const hc_t<SP>
 // refresh's yz pass reads no D_x either; the next predictor completes the
 // entry).
 // ---------------------------------------------------------------------------
-template <int LX, bool SP>
+template <int LX, bool SP, int AL = AL_NONE>
 __global__ void __launch_bounds__(FT, x_waves(LX))
 f_corr(double2 *__restrict__ y, const hc_t<SP> *hin, const hc_t<SP> *__restrict__ cin,
        double *__restrict__ xpart, const double *__restrict__ sp_, const double *__restrict__ ep_, int n, long N,
-       int S, double dta0, double kscale, int wave, double *__restrict__ part, float2 *y32)
+       int S, double dta0, double kscale, int wave, double *__restrict__ part, float2 *y32, XAlpha xa)
 {
+    if (!alpha_form<AL>(xa)) return;
     typedef hc_t<SP> HC;
     const long P = (long)blockIdx.x * FT + threadIdx.x;
     const long Ptot = 2L * n * S;
@@ -229,7 +278,15 @@ f_corr(double2 *__restrict__ y, const hc_t<SP> *hin, const hc_t<SP> *__restrict_
             if constexpr (SP) r[i] = cin[base + (long)i * S];   // the FP32 copy of y_p
             else r[i] = y[base + (long)i * S];                  // y_p
         }
-        xkin_inplace<LX>(r, skh, -e / LX);
+        xkin_inplace<LX>(r, skh, AL == AL_ANY ? 0.0 : -e / LX);
+        if constexpr (AL == AL_ANY) {
+            const double *al = xa.al + (a2 < n ? 0 : N) + j;
+#pragma unroll
+            for (int i = 0; i < LX; i++) {
+                r[i] = r[i] * al[(long)i * S] - y[base + (long)i * S] * e;
+                if (i % 4 == 3) __builtin_amdgcn_sched_barrier(0);
+            }
+        }
         // keep the loop's loads out of the transforms, and form the loop's
         // addresses anew rather than holding the preload's across them
         // (registers)
@@ -251,7 +308,8 @@ f_corr(double2 *__restrict__ y, const hc_t<SP> *hin, const hc_t<SP> *__restrict_
             // (registers: r[] is live across the loop)
             if (i % 4 == 3) __builtin_amdgcn_sched_barrier(0);
         }
-        xk = xkin_energy<LX>(r, skh);
+        if constexpr (AL == AL_ANY) xk = xkin_energy_alpha<LX>(r, skh, y + base, xa.al + (a2 < n ? 0 : N) + j, S);
+        else xk = xkin_energy<LX>(r, skh);
     }
     put_norm_part(nrm, wave != 0, P, Ptot, part);
     put_norm_part(xk, wave != 0, P, Ptot, xpart);
@@ -540,11 +598,12 @@ f_fixup(double2 *__restrict__ y, hc_t<SP> *__restrict__ f0, const double *__rest
 // The pending state of a fused step made explicit (tdw_finalize): y *= s,
 // and the newest history entry completed, f0 += s sigma (-1/2 D_x) y - e y_k
 // (x-pencils, as the predictor does it)
-template <int LX, bool SP>
+template <int LX, bool SP, int AL = AL_NONE>
 __global__ void __launch_bounds__(FT, x_waves(LX))
 f_fixup_x(double2 *__restrict__ y, hc_t<SP> *__restrict__ f0, const double *__restrict__ sk,
-          const double *__restrict__ ek, int n, long N, int S, double kscale)
+          const double *__restrict__ ek, int n, long N, int S, double kscale, XAlpha xa)
 {
+    if (!alpha_form<AL>(xa)) return;
     typedef hc_t<SP> HC;
     const long P = (long)blockIdx.x * FT + threadIdx.x;
     if (P >= 2L * n * S) return;
@@ -556,6 +615,11 @@ f_fixup_x(double2 *__restrict__ y, hc_t<SP> *__restrict__ f0, const double *__re
 #pragma unroll
     for (int i = 0; i < LX; i++) r[i] = cvt<HC>(y[base + (long)i * S]);
     xkin_inplace<LX>(r, (a2 < n ? 0.5 : -0.5) * kscale, 0.0);
+    if constexpr (AL == AL_ANY) {
+        const double *al = xa.al + (a2 < n ? 0 : N) + j;
+#pragma unroll
+        for (int i = 0; i < LX; i++) r[i] = r[i] * al[(long)i * S];
+    }
     // as in the corrector: loads kept out of the transforms, addresses formed
     // here (registers)
     __builtin_amdgcn_sched_barrier(0);
@@ -600,6 +664,7 @@ int fused_state_vecs(tdw_ctx *c)
     TDW_HIP(hipMalloc(&c->d_sp, sizeof(double) * c->nwf));
     TDW_HIP(hipMalloc(&c->d_s2, sizeof(double) * c->nwf));
     TDW_HIP(hipMalloc(&c->d_ep, sizeof(double) * c->nwf));
+    TDW_HIP(hipMalloc(&c->d_one, sizeof(int) * ONE_BLOCKS));
     return 0;
 }
 
@@ -609,6 +674,7 @@ void fused_release(tdw_ctx *c)
     if (c->d_sp) hipFree(c->d_sp);
     if (c->d_s2) hipFree(c->d_s2);
     if (c->d_ep) hipFree(c->d_ep);
+    if (c->d_one) hipFree(c->d_one);
     c->d_fpart = nullptr;
     c->d_sp = c->d_s2 = c->d_ep = nullptr;
 }
@@ -629,56 +695,44 @@ constexpr int ext_nt(int ny) { return ny == 18 ? 192 : ny == 36 ? 448 : 384; }
 template <bool SP> struct FusedFns {
     typedef hc_t<SP> HC;
     typedef void (*pred_fn)(double2 *, HC *, const HC *, const HC *, const HC *, const HC *, HC *, double *,
-                            const double *, const double *, int, int, long, int, double, double, int, double *);
+                            const double *, const double *, int, int, long, int, double, double, int, double *, XAlpha);
     typedef void (*corr_fn)(double2 *, const HC *, const HC *, double *, const double *, const double *, int, long,
-                            int, double, double, int, double *, float2 *);
-    typedef void (*fix_fn)(double2 *, HC *, const double *, const double *, int, long, int, double);
+                            int, double, double, int, double *, float2 *, XAlpha);
+    typedef void (*fix_fn)(double2 *, HC *, const double *, const double *, int, long, int, double, XAlpha);
     typedef void (*hyz_fn)(const HC *, const HC *, HC *, const double *, const double *, int, long, int,
                            const HC *, const HC *, double, double, HParams, double *);
 
-    template <int LX> static pred_fn pick_pred(int sch)
+    template <int LX, int AL> static pred_fn pick_pred(int sch)
     {
-        if (sch == TDW_AB3AM4) return f_pred<LX, 34, SP>;
-        if (sch == TDW_AB4AM5) return f_pred<LX, 45, SP>;
-        return f_pred<LX, 55, SP>;
+        if (sch == TDW_AB3AM4) return f_pred<LX, 34, SP, AL>;
+        if (sch == TDW_AB4AM5) return f_pred<LX, 45, SP, AL>;
+        return f_pred<LX, 55, SP, AL>;
     }
 
-    static bool xpass(int nx, int sch, pred_fn *p, corr_fn *cf)
+    // AL: the forms of the lattices of fused_ext
+    template <int LX, int AL> static bool xset(int sch, pred_fn *p, corr_fn *cf, fix_fn *f)
     {
-        switch (nx) {
-        case 8: *p = pick_pred<8>(sch); *cf = f_corr<8, SP>; return true;
-        case 12: *p = pick_pred<12>(sch); *cf = f_corr<12, SP>; return true;
-        case 16: *p = pick_pred<16>(sch); *cf = f_corr<16, SP>; return true;
-        case 24: *p = pick_pred<24>(sch); *cf = f_corr<24, SP>; return true;
-        case 32: *p = pick_pred<32>(sch); *cf = f_corr<32, SP>; return true;
-        default: break;
-        }
-        if constexpr (!SP) {
-            switch (nx) {
-            case 18: *p = pick_pred<18>(sch); *cf = f_corr<18, SP>; return true;
-            case 36: *p = pick_pred<36>(sch); *cf = f_corr<36, SP>; return true;
-            case 48: *p = pick_pred<48>(sch); *cf = f_corr<48, SP>; return true;
-            default: break;
-            }
-        }
-        return false;
+        if (p) *p = pick_pred<LX, AL>(sch);
+        if (cf) *cf = f_corr<LX, SP, AL>;
+        if (f) *f = f_fixup_x<LX, SP, AL>;
+        return true;
     }
 
-    static bool fix(int nx, fix_fn *f)
+    template <int AL = AL_NONE> static bool xpass(int nx, int sch, pred_fn *p, corr_fn *cf, fix_fn *f = nullptr)
     {
         switch (nx) {
-        case 8: *f = f_fixup_x<8, SP>; return true;
-        case 12: *f = f_fixup_x<12, SP>; return true;
-        case 16: *f = f_fixup_x<16, SP>; return true;
-        case 24: *f = f_fixup_x<24, SP>; return true;
-        case 32: *f = f_fixup_x<32, SP>; return true;
+        case 8: return xset<8, AL>(sch, p, cf, f);
+        case 12: return xset<12, AL>(sch, p, cf, f);
+        case 16: return xset<16, AL>(sch, p, cf, f);
+        case 24: return xset<24, AL>(sch, p, cf, f);
+        case 32: return xset<32, AL>(sch, p, cf, f);
         default: break;
         }
-        if constexpr (!SP) {
+        if constexpr (AL != AL_NONE) {
             switch (nx) {
-            case 18: *f = f_fixup_x<18, SP>; return true;
-            case 36: *f = f_fixup_x<36, SP>; return true;
-            case 48: *f = f_fixup_x<48, SP>; return true;
+            case 18: return xset<18, AL>(sch, p, cf, f);
+            case 36: return xset<36, AL>(sch, p, cf, f);
+            case 48: return xset<48, AL>(sch, p, cf, f);
             default: break;
             }
         }
@@ -767,11 +821,21 @@ bool fused_supported(const tdw_ctx *c)
 static bool fused_ext(const tdw_ctx *c)
 {
     if (c->dim != 3 || varying_mass(c) || c->p.precision != TDW_FP64 || fused_supported(c)) return false;
+    // (a callback may change alpha between the x passes of a step)
+    if (project_changes_potentials(c)) return false;
     FusedFns<false>::pred_fn p;
     FusedFns<false>::corr_fn cf;
     FusedFns<false>::hyz_fn h;
-    return FusedFns<false>::xpass(c->nx, c->p.scheme, &p, &cf) && FusedFns<false>::hyz(c->ny, c->nz, false, &h) &&
+    return FusedFns<false>::xpass<AL_ONE>(c->nx, c->p.scheme, &p, &cf) && FusedFns<false>::hyz(c->ny, c->nz, false, &h) &&
            hyz_lds<false>(c) <= (size_t)c->max_lds;
+}
+
+// the effective masses of an ext step (BdG's H has none); its flags are filled
+// at the step's start
+static XAlpha ext_alpha(const tdw_ctx *c, const tdw_state *s)
+{
+    if (c->p.functional == TDW_BDG) return {nullptr, nullptr};
+    return {s->pots + 4 * c->N, c->d_one};
 }
 
 static int nhist(const tdw_ctx *c) { return c->p.scheme == TDW_AB3AM4 ? 3 : c->p.scheme == TDW_AB4AM5 ? 4 : 5; }
@@ -787,13 +851,26 @@ template <bool SP> static int fixup(tdw_ctx *c, double2 *y, void *f0, int n, int
 
 template <bool SP> static int fixup_x(tdw_ctx *c, tdw_state *s)
 {
-    typename FusedFns<SP>::fix_fn f;
-    if (!FusedFns<SP>::fix(c->nx, &f)) return TDW_EINVAL;
+    typename FusedFns<SP>::fix_fn f = nullptr, f2 = nullptr;
+    XAlpha xa{nullptr, nullptr};
+    bool ext = false;
+    if constexpr (!SP) ext = fused_ext(c);
+    if (ext) {
+        if constexpr (!SP) {
+            FusedFns<false>::xpass<AL_ONE>(c->nx, c->p.scheme, nullptr, nullptr, &f);
+            FusedFns<false>::xpass<AL_ANY>(c->nx, c->p.scheme, nullptr, nullptr, &f2);
+        }
+        xa = ext_alpha(c, s);
+    } else if (!FusedFns<SP>::template xpass<>(c->nx, c->p.scheme, nullptr, nullptr, &f)) {
+        return TDW_EINVAL;
+    }
     const int n = s->n, S = c->S;
     const double kxs = pow(2.0 * M_PI / c->Lphys[0], 2) / c->nx;
     TDW_TIMED(c, "f_fixup");
-    hipLaunchKernelGGL(f, dim3((2L * n * S + FT - 1) / FT), dim3(FT), 0, c->stream, (double2 *)s->wf,
-                       (hc_t<SP> *)s->f[0], c->d_scale, c->d_qpe, n, (long)c->N, S, kxs);
+    for (auto k : {f, xa.al ? f2 : nullptr})
+        if (k)
+            hipLaunchKernelGGL(k, dim3((2L * n * S + FT - 1) / FT), dim3(FT), 0, c->stream, (double2 *)s->wf,
+                               (hc_t<SP> *)s->f[0], c->d_scale, c->d_qpe, n, (long)c->N, S, kxs, xa);
     return (int)hipGetLastError();
 }
 
@@ -878,7 +955,25 @@ static int fused_step_t(tdw_ctx *c, tdw_state *s, int it, int grad_last, tdw_tap
     double *xpart = c->d_fpart + xoff;
     typename FusedFns<SP>::pred_fn fp;
     typename FusedFns<SP>::corr_fn fc;
-    FusedFns<SP>::xpass(c->nx, c->p.scheme, &fp, &fc);
+    // fp2, fc2: the second forms of the ext lattices
+    typename FusedFns<SP>::pred_fn fp2 = nullptr;
+    typename FusedFns<SP>::corr_fn fc2 = nullptr;
+    XAlpha xa{nullptr, nullptr};
+    bool ext = false;
+    if constexpr (!SP) ext = fused_ext(c);
+    if (ext) {
+        if constexpr (!SP) {
+            FusedFns<false>::xpass<AL_ONE>(c->nx, c->p.scheme, &fp, &fc);
+            FusedFns<false>::xpass<AL_ANY>(c->nx, c->p.scheme, &fp2, &fc2);
+        }
+        xa = ext_alpha(c, s);
+        if (xa.al) {
+            hipLaunchKernelGGL(f_alpha_one, dim3(ONE_BLOCKS), dim3(FT), 0, c->stream, xa.al, 2 * N, c->d_one);
+            TDW_HIP(hipGetLastError());
+        }
+    } else {
+        FusedFns<SP>::template xpass<>(c->nx, c->p.scheme, &fp, &fc);
+    }
     const double kxs = pow(2.0 * M_PI / c->Lphys[0], 2) / c->nx;
     const long nblk = (2L * n * S + FT - 1) / FT;
     // H of the prediction lives in lap (in the split form FP32 values, and
@@ -893,8 +988,11 @@ static int fused_step_t(tdw_ctx *c, tdw_state *s, int it, int grad_last, tdw_tap
     // ---- predictor ----
     {
         TDW_TIMED(c, "f_pred");
-        hipLaunchKernelGGL(fp, dim3(nblk), dim3(FT), 0, c->stream, y, f[0], f[1], f[2], f[3], f[4], fold,
-                           xpart, c->d_scale, c->d_qpe, c->pending, n, N, S, c->p.dt, kxs, wave, c->d_fpart);
+        for (auto k : {fp, xa.al ? fp2 : nullptr})
+            if (k)
+                hipLaunchKernelGGL(k, dim3(nblk), dim3(FT), 0, c->stream, y, f[0], f[1], f[2], f[3], f[4], fold,
+                                   xpart, c->d_scale, c->d_qpe, c->pending, n, N, S, c->p.dt, kxs, wave, c->d_fpart,
+                                   xa);
         TDW_HIP(hipGetLastError());
     }
     c->pending = 0;
@@ -918,8 +1016,10 @@ static int fused_step_t(tdw_ctx *c, tdw_state *s, int it, int grad_last, tdw_tap
     const double a0 = (c->p.scheme == TDW_AB3AM4) ? 9. / 24. : 251. / 720.;
     {
         TDW_TIMED(c, "f_corr");
-        hipLaunchKernelGGL(fc, dim3(nblk), dim3(FT), 0, c->stream, y, H, fold, xpart, c->d_sp, c->d_ep, n, N,
-                           S, c->p.dt * a0, kxs, wave, c->d_fpart, SP ? (float2 *)H : nullptr);
+        for (auto k : {fc, xa.al ? fc2 : nullptr})
+            if (k)
+                hipLaunchKernelGGL(k, dim3(nblk), dim3(FT), 0, c->stream, y, H, fold, xpart, c->d_sp, c->d_ep, n, N,
+                                   S, c->p.dt * a0, kxs, wave, c->d_fpart, SP ? (float2 *)H : nullptr, xa);
         TDW_HIP(hipGetLastError());
     }
     TDW_TRY(xpass_norm(c, n, c->d_scale, c->d_s2, wave, tape ? tape->scal + 2 * n : nullptr));

@@ -148,6 +148,8 @@ const double *h_view(tdw_ctx *c, int it, const double *pots)
     return c->d_potsH;
 }
 
+bool project_changes_potentials(const tdw_ctx *c) { return c->proj && c->proj->modify_potentials; }
+
 int project_modify_potentials(tdw_ctx *c, int it, const double *dens, double *pots)
 {
     if (!c->proj || !c->proj->modify_potentials) return 0;

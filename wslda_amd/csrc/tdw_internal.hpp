@@ -60,6 +60,7 @@ struct tdw_ctx {
     double *d_scale;                     // n: 1/sqrt(norm) of the stored (unnormalised) y
     double *d_sp, *d_s2, *d_ep;          // n: predictor scale, scale^2, predictor <H>
     double *d_fpart;  size_t fpart_cap;  // partial sums of the fused kernels
+    int *d_one;                          // ONE_BLOCKS flags: alpha is 1 (lattices of fused_ext)
     int pending;                         // y and f[0] carry a pending scale / <H> fix-up
     // resident-state step (tdw_resident.hip): plan and tables, null where a
     // state does not fit in LDS

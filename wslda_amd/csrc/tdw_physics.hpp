@@ -68,6 +68,7 @@ const double *vel_field(tdw_ctx *c, int it);
 // A_s - v_s when the problem has those callbacks (null on a launch error)
 const double *h_view(tdw_ctx *c, int it, const double *pots);
 int project_modify_potentials(tdw_ctx *c, int it, const double *dens, double *pots);
+bool project_changes_potentials(const tdw_ctx *c);
 // modify_densities (host) before the potentials of a whole step
 int step_potentials(tdw_ctx *c, int it, double *dens, double *pots);
 // functional parameters of the context
