@@ -40,20 +40,17 @@ inline unsigned rs_magic(int d) { return d > 1 ? (unsigned)((1ull << 32) / (unsi
 
 // KIND 0: a forward stage; 1: an inverse stage; 2: the last forward stage,
 // op(position, pencil, value) on the spectrum and the first inverse stage in
-// registers; 3: the last forward stage and op on the spectrum, nothing stored
-// (sums).  pencil is q % qd (q for qd = 0).  TP > 0: TP pencils side by side
-// (P = is = TP, a power of two), the geometry of a tile of x pencils, whose
-// plan has no radix above 8 (rs_axis: top; registers).
-template <int R, int KIND, int TP, typename C, typename OP>
+// registers.  pencil is q % qd (q for qd = 0).
+template <int R, int KIND, typename C, typename OP>
 __device__ __forceinline__ void rs_stage(C *A, const C *tw, const RsAxis &ax, const RsStage &st, OP &&op)
 {
-    const unsigned tot = (TP ? TP : ax.P) * (ax.L / R);
-    const unsigned is = TP ? TP : ax.is;
+    const unsigned tot = ax.P * (ax.L / R);
+    const unsigned is = ax.is;
     for (unsigned b = threadIdx.x; b < tot; b += blockDim.x) {
-        const unsigned jj = TP ? b / TP : rs_div(b, ax.P, ax.mP), q = TP ? b % TP : b - jj * ax.P;
+        const unsigned jj = rs_div(b, ax.P, ax.mP), q = b - jj * ax.P;
         const unsigned blk = rs_div(jj, st.sub, st.msub), j = jj - blk * st.sub;
-        unsigned qi = q, base = TP ? q : q * ax.qh;
-        if (!TP && ax.qd) {
+        unsigned qi = q, base = q * ax.qh;
+        if (ax.qd) {
             const unsigned hi = rs_div(q, ax.qd, ax.mqd);
             qi = q - hi * ax.qd;
             base = hi * ax.qh + qi;
@@ -82,7 +79,6 @@ __device__ __forceinline__ void rs_stage(C *A, const C *tw, const RsAxis &ax, co
             } else {
 #pragma unroll
                 for (int t = 0; t < R; t++) op(i0 + t, qi, v[t]);
-                if constexpr (KIND == 3) continue;
                 rf::dft_inplace<R, +1, C>(v);
             }
         }
@@ -92,50 +88,39 @@ __device__ __forceinline__ void rs_stage(C *A, const C *tw, const RsAxis &ax, co
     __syncthreads();
 }
 
-template <int KIND, int TP, typename C, typename OP>
+template <int KIND, typename C, typename OP>
 __device__ __forceinline__ void rs_run(C *A, const C *tw, const RsAxis &ax, int s, OP &&op)
 {
     const RsStage st = ax.st[s];
     switch (st.R) {
-    case 2: rs_stage<2, KIND, TP>(A, tw + ax.tw, ax, st, op); break;
-    case 3: rs_stage<3, KIND, TP>(A, tw + ax.tw, ax, st, op); break;
-    case 4: rs_stage<4, KIND, TP>(A, tw + ax.tw, ax, st, op); break;
-    case 6: rs_stage<6, KIND, TP>(A, tw + ax.tw, ax, st, op); break;
-    case 8: rs_stage<8, KIND, TP>(A, tw + ax.tw, ax, st, op); break;
-    case 9:
-        if constexpr (TP == 0) rs_stage<9, KIND, TP>(A, tw + ax.tw, ax, st, op);
-        break;
-    default:
-        if constexpr (TP == 0) rs_stage<12, KIND, TP>(A, tw + ax.tw, ax, st, op);
-        break;
+    case 2: rs_stage<2, KIND>(A, tw + ax.tw, ax, st, op); break;
+    case 3: rs_stage<3, KIND>(A, tw + ax.tw, ax, st, op); break;
+    case 4: rs_stage<4, KIND>(A, tw + ax.tw, ax, st, op); break;
+    case 6: rs_stage<6, KIND>(A, tw + ax.tw, ax, st, op); break;
+    case 8: rs_stage<8, KIND>(A, tw + ax.tw, ax, st, op); break;
+    case 9: rs_stage<9, KIND>(A, tw + ax.tw, ax, st, op); break;
+    default: rs_stage<12, KIND>(A, tw + ax.tw, ax, st, op); break;
     }
 }
 struct RsNop {
     template <typename C> __device__ void operator()(unsigned, unsigned, C &) const {}
 };
 // all forward / all inverse stages of an axis
-template <int TP = 0, typename C> __device__ __forceinline__ void rs_forward(C *A, const C *tw, const RsAxis &ax)
+template <typename C> __device__ __forceinline__ void rs_forward(C *A, const C *tw, const RsAxis &ax)
 {
-    for (int s = 0; s < ax.nst; s++) rs_run<0, TP>(A, tw, ax, s, RsNop());
+    for (int s = 0; s < ax.nst; s++) rs_run<0>(A, tw, ax, s, RsNop());
 }
-template <int TP = 0, typename C> __device__ __forceinline__ void rs_inverse(C *A, const C *tw, const RsAxis &ax)
+template <typename C> __device__ __forceinline__ void rs_inverse(C *A, const C *tw, const RsAxis &ax)
 {
-    for (int s = ax.nst - 1; s >= 0; s--) rs_run<1, TP>(A, tw, ax, s, RsNop());
+    for (int s = ax.nst - 1; s >= 0; s--) rs_run<1>(A, tw, ax, s, RsNop());
 }
 // F^-1 op F along the axis (nst >= 1)
-template <int TP = 0, typename C, typename OP>
+template <typename C, typename OP>
 __device__ __forceinline__ void rs_filter(C *A, const C *tw, const RsAxis &ax, OP &&op)
 {
-    for (int s = 0; s < ax.nst - 1; s++) rs_run<0, TP>(A, tw, ax, s, RsNop());
-    rs_run<2, TP>(A, tw, ax, ax.nst - 1, op);
-    for (int s = ax.nst - 2; s >= 0; s--) rs_run<1, TP>(A, tw, ax, s, RsNop());
-}
-// op on the spectrum, which is not stored
-template <int TP = 0, typename C, typename OP>
-__device__ __forceinline__ void rs_spectrum(C *A, const C *tw, const RsAxis &ax, OP &&op)
-{
-    for (int s = 0; s < ax.nst - 1; s++) rs_run<0, TP>(A, tw, ax, s, RsNop());
-    rs_run<3, TP>(A, tw, ax, ax.nst - 1, op);
+    for (int s = 0; s < ax.nst - 1; s++) rs_run<0>(A, tw, ax, s, RsNop());
+    rs_run<2>(A, tw, ax, ax.nst - 1, op);
+    for (int s = ax.nst - 2; s >= 0; s--) rs_run<1>(A, tw, ax, s, RsNop());
 }
 
 // ---------------------------------------------------------------------------
@@ -154,17 +139,16 @@ inline bool rs_split(int rem, int m, int top, int *R)
         }
     return false;
 }
-inline int rs_radices(int L, int *R, int most)
+inline int rs_radices(int L, int *R)
 {
     for (int m = 0; m <= RS_MAXST; m++)
         for (int top : {2, 3, 4, 6, 8, 9, 12})
-            if (top <= most && rs_split(L, m, top, R)) return m;
+            if (rs_split(L, m, top, R)) return m;
     return -1;
 }
 
-// fills ax (geometry as given, radices up to most); false where the length
-// has no plan
-inline bool rs_axis(RsAxis &ax, int L, int is, int P, int qd, int qh, int tw, int most = 12)
+// fills ax (geometry as given); false where the length has no plan
+inline bool rs_axis(RsAxis &ax, int L, int is, int P, int qd, int qh, int tw)
 {
     int R[RS_MAXST];
     ax.L = L;
@@ -175,7 +159,7 @@ inline bool rs_axis(RsAxis &ax, int L, int is, int P, int qd, int qh, int tw, in
     ax.tw = tw;
     ax.mP = rs_magic(P);
     ax.mqd = rs_magic(qd);
-    ax.nst = rs_radices(L, R, most);
+    ax.nst = rs_radices(L, R);
     if (ax.nst < 0) return false;
     int sub = L, mul = 1;
     for (int s = 0; s < ax.nst; s++) {
