@@ -56,6 +56,7 @@ CASES = [
     (2, (8, 12, 6), 270), (2, (36, 18, 4), 20), (2, (6, 128, 4), 9), (2, (48, 54, 4), 7), (2, (64, 64, 4), 5),
     (2, (32, 32, 4), 300), (2, (32, 64, 4), 6), (2, (64, 32, 4), 6),
     (2, (72, 72, 4), 4),       # the state (166 KB) does not fit: the plane-wise step
+    (1, (27, 4, 4), 9), (1, (243, 4, 4), 20), (2, (9, 27, 4), 12), (2, (27, 16, 4), 30), (2, (12, 9, 4), 260),
     (3, (12, 12, 12), 30), (3, (8, 6, 4), 600), (3, (16, 16, 16), 6), (3, (4, 18, 24), 12),
 ]
 
