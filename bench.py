@@ -61,24 +61,26 @@ def algorithmic_units(name, scheme, split=False):
     }.get(name, 0)
 
 
-def design_units(name, scheme, split=False):
+def design_units(name, scheme, split=False, nx=32):
     """Bytes (units of S per state and launch) this implementation's kernels
     must move: reads and writes of state-sized arrays (FP64 S; the split
     form's history, T / H scratch and the FP32 copies of the prediction and
-    of the corrected state are S/2)."""
+    of the corrected state are S/2).  nx: the predictor holds its pencil of y
+    in registers up to 24 points and reads it twice beyond (for the x kinetic
+    part of f_1, then for the points)."""
     h = nhist(scheme)
+    y = 1 if nx <= 24 else 2
     if split:
         return {
-            # y (twice: its pencil for the x kinetic part of f_1, then the
-            # points), f_1..f_h; c, y_p (FP32), f_1 completed
-            "f_pred": 2 + 0.5 * h + 1 + 0.5 + 0.5,
+            # y, f_1..f_h; c, y_p (FP32), f_1 completed
+            "f_pred": y + 0.5 * h + 1 + 0.5 + 0.5,
             "f_corr": 1 + 0.5 + 0.5 + 1 + 0.5,             # c, H y_p, y_p (FP32); y, y (FP32)
             "f_hyz": 1.0,                                   # y (FP32); H
             "densities": 0.5,                               # y (FP32)
             "f_fixup": 2,
         }.get(name, 0)
     return {
-        "f_pred": (h + 2) + 3,   # read y (twice, as above), f_1..f_h; write y_p, c, f_1 (completed)
+        "f_pred": (h + y) + 3,   # read y, f_1..f_h; write y_p, c, f_1 (completed)
         "f_corr": 4,             # read y_p, H y_p, c; write y
         "f_hyz": 2,              # read y; write H y
         "densities": 1,          # read y
@@ -216,7 +218,7 @@ def run_gpu(args, prec):
         moved = dbytes
     else:
         dbytes = algorithmic_units(dname, p.scheme, prec == td.SPLIT) * S * n
-        moved = design_units(dname, p.scheme, prec == td.SPLIT) * S * n
+        moved = design_units(dname, p.scheme, prec == td.SPLIT, p.nx) * S * n
     achieved = dbytes / davg / 1e9 if dbytes else None
     step_bytes = step_units(p.scheme, prec == td.SPLIT) * S * n
     out = dict(qps=qps, ms=ms, wall=wall, n=n, N=N, rep=rep, dname=dname, davg=davg, dbytes=dbytes,
@@ -284,12 +286,14 @@ def cpu_baseline(g, args):
 
 # HBM bytes per launch of the dominant kernel, keyed by (kernel, lattice,
 # states, scheme, precision): FETCH_SIZE x 2 + WRITE_SIZE (KiB x 1024) of one
-# launch, from the counter runs of `bench.py --steps 4 --warmup 1 --no-cpu
-# --meas-every 1000 --copy-calib-mib 4096 --trap-states 0` (the 4096 MiB copy
-# reads FETCH_SIZE = half its bytes and WRITE_SIZE = all of them)
+# launch that completes the pending entry, from the counter runs of `bench.py
+# --steps 4 --warmup 1 --no-cpu --meas-every 1000 --copy-calib-mib 4096
+# --trap-states 0 --line-tube-steps 0 --line-adjoint 0` (the 4096 MiB copy
+# reads FETCH_SIZE = half its bytes and WRITE_SIZE = all of them).  9.0 S and
+# 5.5 S, as design_units has it.
 MEASURED_TRAFFIC = {
-    ("f_pred", (24, 24, 24), 16308, 55, "fp64"): (24629179 * 2 + 21140835) * 1024,
-    ("f_pred", (24, 24, 24), 16308, 55, "split"): (15591706 * 2 + 14094742) * 1024,
+    ("f_pred", (24, 24, 24), 16308, 55, "fp64"): (21136833 * 2 + 21139887) * 1024,
+    ("f_pred", (24, 24, 24), 16308, 55, "split"): (12330270 * 2 + 14094732) * 1024,
 }
 
 

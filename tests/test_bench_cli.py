@@ -31,6 +31,13 @@ def test_design_units_add_up_to_the_measured_step():
     assert step_sum(bench.design_units, 55, True) == 13
 
 
+def test_design_units_of_axes_held_in_registers():
+    # up to 24 points the predictor reads y once
+    u = lambda *a: bench.design_units(*a, nx=24)
+    assert step_sum(u, 55, False) == 19
+    assert step_sum(u, 55, True) == 12
+
+
 def test_algorithmic_units_add_up_to_the_compulsory_step():
     assert step_sum(bench.algorithmic_units, 55, False) == bench.step_units(55, False) == 13
     assert step_sum(bench.algorithmic_units, 55, True) == bench.step_units(55, True) == 9
