@@ -191,3 +191,17 @@ def test_fused_taped_step_matches_modular_step(torch):
     say("  max rel diff over %d steps (y, f_new, dens, pots, <H>): %.2e" % (steps, worst))
     assert worst <= 1e-12
     prob.close()
+
+
+@pytest.mark.parametrize("ngauss", [0, -1])
+def test_gradient_without_gaussians(torch, ngauss):
+    """No Gaussian in use (a negative count means none, as in V_ext): the
+    backward run leaves their gradient at zero."""
+    prob, theta = setup_problem(*CASES[0])
+    v = gauss_slots(theta, 2)
+    v.ngauss = ngauss
+    prob.set_vext(v)
+    prob.forward()
+    g = np.asarray(prob.backward())
+    prob.close()
+    assert np.all(g == 0.0)

@@ -554,8 +554,8 @@ static int pot_vjp(tdw_ctx *c, int it, const double *dens, const double *pots_pr
     TDW_TRY(ensure_part(c, (size_t)nblk * NTHETA));
     hipLaunchKernelGGL(k_pot_vjp, dim3(nblk), dim3(PT), 0, c->stream, fparams(c), make_vext(c, it), N, dens,
                        pots_prev, lU, dens_add, lD, lUprev, c->d_part);
-    const int np = 7 * std::min(make_vext(c, it).v.ngauss, TDW_MAX_GAUSS);
-    if (np) hipLaunchKernelGGL(k_gsum, dim3(np), dim3(AT), 0, c->stream, c->d_part, nblk, theta_grad);
+    const int np = 7 * std::min(make_vext(c, it).v.ngauss, TDW_MAX_GAUSS);   // (less than one: none in use)
+    if (np > 0) hipLaunchKernelGGL(k_gsum, dim3(np), dim3(AT), 0, c->stream, c->d_part, nblk, theta_grad);
     return (int)hipGetLastError();
 }
 
