@@ -77,11 +77,15 @@ struct Thirds {
 };
 __device__ __forceinline__ Thirds thirds(double x)
 {
+    // the parts' roundings are what is computed here: no contraction but the
+    // fma written
+#pragma clang fp contract(off)
     const double c = x < 0.0 ? nan("") : cbrt(x);
-    const double p = c * c, pl = fma(c, c, -p), q = p * c, ql = fma(p, c, -q);
-    const double r = (x - q) - fma(pl, c, ql);
-    // (zero and infinity are their own powers)
-    const double t = p > 0.0 && p < 1.0e300 ? fma(2.0 / 3.0, r / c, pl) : 0.0;
+    const double p = c * c, pl = fma(c, c, -p);
+    const double r = fma(-pl, c, fma(-p, c, x));   // x - c^3
+    // (zero and infinity are their own powers; an estimate of 1 / c is enough
+    // for a correction in the last place)
+    const double t = p > 0.0 && p < 1.0e300 ? fma((2.0 / 3.0) * r, __builtin_amdgcn_rcp(c), pl) : 0.0;
     const double h = p + t;
     return {c, h, fma(x, t - (h - p), x * h)};
 }
