@@ -242,9 +242,10 @@ int tdw_step(tdw_ctx *c, tdw_state *s, int it, int grad_last);
  * so between steps wf is unnormalised and f[0] lacks only the subtraction
  * (same completion rules); it has a split form too (below; its
  * measurement steps also use ddy and ddz as FP64 scratch).  FP64 lattices of
- * constant effective mass whose state fits in LDS (1D, 2D, and 3D lattices
- * with fused passes up to 16^3) run the resident step, which leaves nothing to
- * complete; those with axes of 18, 36 and 48 points run the six passes,
+ * constant effective mass whose state fits in LDS (1D, 2D) run the resident
+ * step, which leaves nothing to complete, as do 3D lattices with fused passes
+ * of which two states fit (12^3), or one of a plane whose points are no multiple
+ * of 64; those with axes of 18, 36 and 48 points run the six passes,
  * completed at each step's end.  Other lattices, and those three lengths in a
  * project build with modify_potentials, run the modular step.
  * tdw_fused_supported() says whether the lattice is one of those with fused

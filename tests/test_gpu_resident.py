@@ -57,7 +57,8 @@ CASES = [
     (2, (32, 32, 4), 300), (2, (32, 64, 4), 6), (2, (64, 32, 4), 6),
     (2, (72, 72, 4), 4),       # the state (166 KB) does not fit: the plane-wise step
     (1, (27, 4, 4), 9), (1, (243, 4, 4), 20), (2, (9, 27, 4), 12), (2, (27, 16, 4), 30), (2, (12, 9, 4), 260),
-    (3, (12, 12, 12), 30), (3, (8, 6, 4), 600), (3, (16, 16, 16), 6), (3, (4, 18, 24), 12),
+    (3, (12, 12, 12), 30), (3, (8, 16, 16), 9), (3, (12, 16, 16), 9), (3, (32, 12, 12), 7), (3, (8, 24, 24), 7),
+     (3, (8, 6, 4), 600), (3, (16, 16, 16), 6), (3, (4, 18, 24), 12),
 ]
 
 

@@ -1135,9 +1135,8 @@ int fused_adj_step(tdw_ctx *c, tdw_state *s, int it, tdw_complex *y_out, double2
 int fused_step(tdw_ctx *c, tdw_state *s, int it, int grad_last)
 {
     if (aslda_step_supported(c)) return aslda_fused_step(c, s, it, grad_last);
-    // FP64 states that fit in LDS: the resident step (15 S against 20 S, and
-    // half the launches), which leaves nothing pending
-    if (fused_supported(c) && resident_supported(c)) {
+    // small FP64 lattices: the resident step, which leaves nothing pending
+    if (fused_supported(c) && resident_pays3d(c)) {
         TDW_TRY(fused_finalize(c, s));
         return resident_step(c, s, it, grad_last);
     }

@@ -490,6 +490,21 @@ bool resident_supported(const tdw_ctx *c)
     return c->rplan && !varying_mass(c) && c->p.precision == TDW_FP64;
 }
 
+// The six passes move 19-20 S for the resident step's 15 S, in twice the
+// launches, but stream them from a full chip.  A state that shares its CU's LDS
+// with a second one is faster resident, as is one of a plane whose points are
+// not whole waves (the passes' norm partials are then one per pencil instead of
+// one per wave).  us per step of 4, 600, 4000 states, six passes and resident:
+// 12^3 80, 182, 1009 and 75, 181, 884; 32 x 12 x 12 100, 439, 2601 and 111, 435,
+// 2474; but 12 x 16 x 16 76, 270, 1654 and 97, 314, 1824; 8 x 24 x 24 80, 366, 2340
+// and 116, 444, 2556; 16^3 82, 341, 2188 and 117, 426, 2484.
+bool resident_pays3d(const tdw_ctx *c)
+{
+    if (!resident_supported(c)) return false;
+    const size_t lds = rs_lds(*c->rplan, c->nx + c->ny + c->nz) + 1024;
+    return 2 * lds <= (size_t)c->max_lds || c->S % 64 != 0;
+}
+
 // Threads of a workgroup: 16 waves per CU (four per SIMD, what 103 VGPRs of
 // rs_h leave) over the workgroups that share it, as many as the LDS holds or
 // as the states give; a whole number of waves, no more than one point per

@@ -14,6 +14,9 @@ int resident_setup(tdw_ctx *c);
 void resident_release(tdw_ctx *c);
 // constant-mass H in FP64 on a lattice with a plan
 bool resident_supported(const tdw_ctx *c);
+// 3D lattices with a plan whose step the six passes of tdw_fused.hip do not do
+// faster
+bool resident_pays3d(const tdw_ctx *c);
 // The step of tdw_step (same arrays, complete at its end; lap is not
 // written in 3D without gradients).  The adjoint's taped step is the
 // same with tape: y to y_out (NULL: in place), the partial corrector to cbuf
