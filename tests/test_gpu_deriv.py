@@ -155,3 +155,30 @@ def test_one_timer_record_per_launch(torch, shape):
     ctx.close()
     assert {k: v[1] for k, v in rep.items()} == {"fft_outer": 1, "fft_inner": 1, "fft_outer_deriv": 1,
                                                  "fft_inner_deriv": 1}
+
+
+@pytest.mark.parametrize("n", [3, 56, 57, 248, 249])
+@pytest.mark.parametrize("shape", [(9, 3, 9), (4, 8, 8)])
+def test_densities_chunk_counts(torch, shape, n):
+    """Densities with gradients over 1, 7, 8, 31 and 32 chunks of states, the
+    limits of the forms of the sum over the chunks; points that do and do not
+    fill its workgroups."""
+    import ctypes as C
+    from wslda_amd import td
+    say("case: densities over chunks shape=%s n=%d" % (shape, n))
+    cfg = po.make_cfg(3, *shape, dx=0.9)
+    N = int(np.prod(shape))
+    r = np.random.default_rng(n)
+    W = [r.normal(size=(2 * n, N)) + 1j * r.normal(size=(2 * n, N)) for _ in range(5)]
+    fb = r.random(n)
+    ref = np.zeros(12 * N)
+    po.lib().tdwo_densities(C.byref(cfg), n, *[po.ptr(w) for w in W], po.ptr(fb), None, None, po.ptr(ref), 1)
+    ctx = td.TDContext(tdgauss.to_params(cfg, td.FP64), n, 0)
+    ctx.set_states(fb)
+    dens = torch.zeros(12 * N, dtype=torch.float64, device="cuda:0")
+    ctx.calculate_densities(*[cuda(torch, w) for w in W], dens, 1)
+    ctx.sync()
+    got = dens.cpu().numpy()
+    ctx.close()
+    # (a sum of n terms of either sign, each of order one)
+    assert np.abs(got - ref).max() < 1e-14 * n

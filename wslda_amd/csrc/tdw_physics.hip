@@ -311,17 +311,19 @@ k_dens_part(const W *__restrict__ wf, const double2 *__restrict__ ddx, const dou
 // dens (the 12*N block) from the chunk partials.  Output f: 0 Re nu, 1 Im nu,
 // 2 rho_a, 3 tau_a, 4-6 j_a, 7 rho_b, 8 tau_b, 9-11 j_b; field f of a chunk
 // is field A.f[f] of the partials A plus field B.f[f] of B (-1: none).
-// A workgroup takes FP points of one field with FL lanes over the chunks, so
-// that the sum over the chunks (up to some hundreds on small lattices) is
-// spread over lanes instead of one chain per point: at 12^3 and 223 chunks a
-// thread per point took 76 us, this takes 7.7 us.  The order of the sum is
-// fixed by the launch shape.
-static constexpr int FP = 16, FL = 16;
-
-__global__ void __launch_bounds__(FP *FL)
+// A workgroup takes points of one field with FL threads over the chunks of
+// each.  Small lattices have up to hundreds of chunks, and a chain of them per
+// point would be the kernel's time (12^3 and 223 chunks: a thread per point 76
+// us, sixteen 7.7); large ones have a handful, and threads without a chunk
+// cost: 48^3 with 5 chunks, the density pass with this sum 31.8 us with one
+// thread, 36.2 with four, 53.9 with sixteen, and 24^3 with 64 chunks 57.2, 47.7
+// and 46.8.  The order of the sum is fixed by the launch shape.
+template <int FL>
+__global__ void __launch_bounds__(NT)
 k_chunk_final(ChunkSrc A, ChunkSrc B, int nchunk, long N, double tr, double *__restrict__ dens)
 {
-    __shared__ double red[FL][FP + 1];
+    constexpr int FP = NT / FL;
+    __shared__ double red[FL > 1 ? FL : 1][FL > 1 ? FP + 1 : 1];
     const int f = blockIdx.y, p = threadIdx.x % FP, l = threadIdx.x / FP;
     const long i = (long)blockIdx.x * FP + p;
     const int fa = A.f[f], fb = B.f[f];
@@ -332,12 +334,15 @@ k_chunk_final(ChunkSrc A, ChunkSrc B, int nchunk, long N, double tr, double *__r
         if (fb >= 0)
             for (int k = l; k < nchunk; k += FL) s += B.part[((long)k * B.nf + fb) * N + i];
     }
-    red[l][p] = s;
-    __syncthreads();
-    if (l || i >= N) return;
-    s = 0.0;
+    if constexpr (FL > 1) {
+        red[l][p] = s;
+        __syncthreads();
+        if (l) return;
+        s = 0.0;
 #pragma unroll
-    for (int k = 0; k < FL; k++) s += red[k][p];
+        for (int k = 0; k < FL; k++) s += red[k][p];
+    }
+    if (i >= N) return;
     const double v = s / 10000. / tr;
     if (f < 2) dens[2 * i + f] = v;
     else dens[(long)f * N + i] = v;
@@ -346,8 +351,10 @@ k_chunk_final(ChunkSrc A, ChunkSrc B, int nchunk, long N, double tr, double *__r
 int chunk_final(tdw_ctx *c, const ChunkSrc &A, const ChunkSrc &B, int nchunk, double *dens)
 {
     const long N = (long)c->N;
-    hipLaunchKernelGGL(k_chunk_final, dim3((unsigned)((N + FP - 1) / FP), 12), dim3(FP * FL), 0, c->stream, A, B,
-                       nchunk, N, dens_transverse(c), dens);
+    const int fl = nchunk < 8 ? 1 : nchunk < 32 ? 4 : 16;
+    const auto k = fl == 16 ? k_chunk_final<16> : fl == 4 ? k_chunk_final<4> : k_chunk_final<1>;
+    hipLaunchKernelGGL(k, dim3((unsigned)((N * fl + NT - 1) / NT), 12), dim3(NT), 0, c->stream, A, B, nchunk, N,
+                       dens_transverse(c), dens);
     TDW_TRY((int)hipGetLastError());
     return spin_fold(c, dens);
 }
